@@ -18,7 +18,8 @@
 // format's dot layout (written once by the gate/up blocks); the down rows are
 // dotted in K parts of 2048 with the h slices in LDS, and a last launch adds the
 // weighted parts per (token, row) in slot order.  Larger calls stage f32 h per
-// block, 4 tokens per pass.
+// block, 4 tokens per pass.  Calls of 4 rows or more whose formats and shapes fit
+// go to the matrix cores instead, whatever their pair count (decode_mfma.hip).
 #include "decode.h"
 #include "decode_mfma.h"
 #include "rowdot.h"
@@ -722,11 +723,12 @@ int tok_cap(int dtype, int k) {
     return cap < 1 ? 0 : (cap > kTokMax ? kTokMax : cap);
 }
 
-// Scratch of one decode call (n = rows * width pairs):
+// Scratch of one decode call (n = rows * width pairs), and the size the no-alloc entry
+// point's capacity is stated in:
 //   seg_count, bad | seg_key[n] | seg_begin[n+1] | perm[n] | h | dpart.
-// Staged-h path: h = n vectors in the down format's dot layout (or, on the matrix
-// cores, f16 x [rows, H] and h [n, I]), dpart = K parts x n x H f32.  Otherwise
-// h = n x I f32 and no dpart.
+// Staged-h path: h = n vectors in the down format's dot layout, dpart = K parts x n x H
+// f32.  Otherwise h = n x I f32 and no dpart.  Calls on the matrix cores lay out their
+// own (NaiwaMfmaLayout) and take as many passes over the rows as it needs to fit.
 struct DecodeScratch {
     size_t off_key, off_begin, off_perm, off_h, off_dpart, total;
     DecodeScratch(int rows, int width, int H, int I, int down_dtype) {
@@ -736,9 +738,9 @@ struct DecodeScratch {
         off_perm = off_begin + (((size_t)(n + 1) * 4 + 255) & ~size_t(255));
         off_h = off_perm + (((size_t)n * 4 + 255) & ~size_t(255));
         if (split_path(n, width)) {
-            // h in the down format's dot layout, or the matrix-core path's f16 x and h
-            const size_t hb =
-                std::max((size_t)n * naiwa_stage_bytes(down_dtype, I), naiwa_decode_mfma_bytes(rows, n, H, I));
+            // h in the down format's dot layout, or x and h in 16 bits
+            const size_t x16 = ((size_t)rows * H * 2 + 255) & ~size_t(255);
+            const size_t hb = std::max((size_t)n * naiwa_stage_bytes(down_dtype, I), x16 + (size_t)n * I * 2);
             off_dpart = off_h + ((hb + 255) & ~size_t(255));
             total = off_dpart + (size_t)split_parts(I) * n * H * 4;
         } else {
@@ -751,6 +753,28 @@ struct DecodeScratch {
 __global__ void zero_f32_kernel(float* p, int64_t n) {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
         p[i] = 0.0f;
+}
+
+// Calls of several rows whose formats fit run on the matrix cores, in passes over the rows
+// when one pass would need more than `cap` bytes of scratch.  Which path a call takes, and
+// its bits, depend on neither cap nor the weights.
+struct MfmaPlan {
+    bool on;
+    int rows; // per pass
+    size_t bytes;
+};
+constexpr size_t kMfmaScratchMax = size_t(256) << 20; // the K parts' dots of a large call stay in the caches
+MfmaPlan mfma_plan(const naiwa_bank* gate, const naiwa_bank* up, const naiwa_bank* down, const void* x, int rows,
+                   int width, size_t cap) {
+    const int mr = mfma_rows();
+    MfmaPlan p{mr > 0 && rows >= mr && width > 0 && width <= NAIWA_MFMA_MAX_WIDTH &&
+                   naiwa_decode_mfma_ok(gate, up, down, x),
+               0, 0};
+    if (!p.on) return p;
+    const int H = gate->k, I = gate->n;
+    p.rows = naiwa_decode_mfma_rows_per_pass(rows, width, H, I, split_parts(I), cap);
+    p.bytes = NaiwaMfmaLayout(p.rows, width, H, I, split_parts(I)).total;
+    return p;
 }
 
 // Argument checks shared by the entry points; 0 when the call is valid.
@@ -873,16 +897,35 @@ int staged_launch(BankArg g, BankArg u, BankArg d, int gdt, int ddt, const void*
     return NAIWA_E_UNSUPPORTED;
 }
 
-// The launches of one checked call over scratch ws (DecodeScratch(...).total bytes).
+// Scratch bytes of a call.
+size_t call_bytes(const MfmaPlan& mfma, const naiwa_bank* gate, const naiwa_bank* down, int rows, int width) {
+    return mfma.on ? mfma.bytes : DecodeScratch(rows, width, gate->k, gate->n, down->dtype).total;
+}
+
+// The launches of one checked call over scratch ws (call_bytes).
 // res (bf16 x, staged calls only): the ordered combine also adds the result to it in
 // place, x = bf16(x + y); out may then be null.
 int decode_launch(const naiwa_bank* gate, const naiwa_bank* up, const naiwa_bank* down, const void* x, int x_dtype,
                   const uint32_t* slot_ids, const float* w, int rows, int width, int act, float* out, int flags,
-                  uint8_t* ws, hipStream_t st, uint16_t* res = nullptr, const naiwa_decode_wait* wait = nullptr) {
+                  const MfmaPlan& mfma, uint8_t* ws, hipStream_t st, uint16_t* res = nullptr,
+                  const naiwa_decode_wait* wait = nullptr) {
     WaitArg wt{nullptr, 0u, 0ull, nullptr};
     if (wait) wt = WaitArg{wait->flag, wait->target, wait->limit_ticks, wait->fail};
     const int accumulate = (flags & NAIWA_DECODE_ACCUMULATE) ? 1 : 0;
     const int H = gate->k, I = gate->n;
+    if (mfma.on) {
+        // the wait is not folded into the expert blocks here: one wave waits first
+        if (wt.flag) decode_wait_kernel<<<1, 64, 0, st>>>(wt);
+        for (int r0 = 0; r0 < rows; r0 += mfma.rows) {
+            const int64_t o = (int64_t)r0 * H, p = (int64_t)r0 * width;
+            const void* xr = (const uint8_t*)x + o * (x_dtype == NAIWA_BF16 ? 2 : 4);
+            const int rc = naiwa_decode_mfma(gate, up, down, xr, x_dtype, slot_ids + p, w + p,
+                                             std::min(mfma.rows, rows - r0), width, act, out ? out + o : nullptr,
+                                             accumulate, res ? res + o : nullptr, split_ks(I), split_parts(I), ws, st);
+            if (rc) return rc;
+        }
+        return NAIWA_OK;
+    }
     if (width == 0) {
         if (accumulate) return NAIWA_OK;
         const int64_t n = (int64_t)rows * H;
@@ -904,13 +947,11 @@ int decode_launch(const naiwa_bank* gate, const naiwa_bank* up, const naiwa_bank
     BankArg g{(const uint8_t*)gate->base, gate->slot_stride, naiwa_row_bytes(gate->dtype, H)};
     BankArg u{(const uint8_t*)up->base, up->slot_stride, naiwa_row_bytes(up->dtype, H)};
     BankArg d{(const uint8_t*)down->base, down->slot_stride, naiwa_row_bytes(down->dtype, I)};
-    const int mr = mfma_rows();
     const bool staged = split_path(n, width);
-    const bool mfma = staged && mr > 0 && rows >= mr && naiwa_decode_mfma_ok(gate, up, down, x);
     // a staged call of few pairs is segmented by its gate/up blocks; every other call
     // by one segments launch first
     SegIn seg_in{nullptr, nullptr, 0, 0, nullptr};
-    if (staged && !mfma && n <= kSmallSeg) {
+    if (staged && n <= kSmallSeg) {
         seg_in = SegIn{slot_ids, w, n, gate->slots, bad};
     } else if (wt.flag) {
         // the wait is not folded into gate/up blocks here: one wave waits first
@@ -922,14 +963,6 @@ int decode_launch(const naiwa_bank* gate, const naiwa_bank* up, const naiwa_bank
                                                          seg_begin, bad);
     if (staged) {
         float* dpart = (float*)(ws + L.off_dpart);
-        if (mfma) {
-            const int ks = split_ks(I), segs = std::max(1, std::min(n, gate->slots));
-            int rc = naiwa_decode_mfma_experts(gate, up, down, x, x_dtype, rows, width, act, n, segs, ks, seg_count,
-                                               seg_key, seg_begin, perm, (uint8_t*)hbuf, dpart, st);
-            if (rc) return rc;
-            return combine_launch(dpart, split_parts(I), n, H, rows, width, seg_count, seg_begin, perm, w,
-                                  accumulate, out, st, res);
-        }
         return staged_launch(g, u, d, gate->dtype, down->dtype, x, x_dtype, H, I, rows, width, act, w, out,
                              accumulate, n, gate->slots, seg_count, seg_key, seg_begin, perm, (uint8_t*)hbuf, dpart,
                              seg_in, st, res, wt);
@@ -1006,12 +1039,12 @@ extern "C" int naiwa_moe_decode_ex(const naiwa_bank* gate, const naiwa_bank* up,
     int rc = check_args(gate, up, down, x, x_dtype, slot_ids, w, rows, width, act, out, flags);
     if (rc || rows == 0) return rc;
     uint8_t* ws = nullptr;
+    const MfmaPlan mfma = mfma_plan(gate, up, down, x, rows, width, kMfmaScratchMax);
     if (width > 0) {
-        const DecodeScratch L(rows, width, gate->k, gate->n, down->dtype);
-        ws = (uint8_t*)naiwa_scratch(NAIWA_SCRATCH_DECODE, L.total, &rc);
+        ws = (uint8_t*)naiwa_scratch(NAIWA_SCRATCH_DECODE, call_bytes(mfma, gate, down, rows, width), &rc);
         if (!ws) return rc;
     }
-    return decode_launch(gate, up, down, x, x_dtype, slot_ids, w, rows, width, act, out, flags, ws,
+    return decode_launch(gate, up, down, x, x_dtype, slot_ids, w, rows, width, act, out, flags, mfma, ws,
                          (hipStream_t)stream);
 }
 
@@ -1022,9 +1055,13 @@ extern "C" int naiwa_moe_decode_noalloc(const naiwa_bank* gate, const naiwa_bank
     if (rc || rows == 0) return rc;
     if (width > 0 && DecodeScratch(rows, width, gate->k, gate->n, down->dtype).total > kNoAllocScratchBytes)
         return NAIWA_E_TOO_LARGE;
+    // on the matrix cores in passes that fit: an accepted call has at least 4 rows there, so
+    // one row takes little more than a quarter of the array
+    const MfmaPlan mfma = mfma_plan(gate, up, down, x, rows, width, kNoAllocScratchBytes);
+    if (mfma.on && mfma.bytes > kNoAllocScratchBytes) return NAIWA_E_TOO_LARGE;
     uint8_t* ws = nullptr;
     if ((rc = noalloc_scratch(&ws))) return rc;
-    return decode_launch(gate, up, down, x, x_dtype, slot_ids, w, rows, width, act, out, flags, ws,
+    return decode_launch(gate, up, down, x, x_dtype, slot_ids, w, rows, width, act, out, flags, mfma, ws,
                          (hipStream_t)stream);
 }
 
@@ -1041,13 +1078,13 @@ int naiwa_moe_decode_residual(const naiwa_bank* gate, const naiwa_bank* up, cons
     int rc = check_args(gate, up, down, x, NAIWA_BF16, slot_ids, w, rows, width, act, y, 0);
     if (rc || rows == 0 || width == 0) return rc;
     if (wait && (!wait->flag || !wait->fail)) return NAIWA_E_INVALID;
-    const DecodeScratch L(rows, width, gate->k, gate->n, down->dtype);
-    uint8_t* ws = (uint8_t*)naiwa_scratch(NAIWA_SCRATCH_DECODE, L.total, &rc);
+    const MfmaPlan mfma = mfma_plan(gate, up, down, x, rows, width, kMfmaScratchMax);
+    uint8_t* ws = (uint8_t*)naiwa_scratch(NAIWA_SCRATCH_DECODE, call_bytes(mfma, gate, down, rows, width), &rc);
     if (!ws) return rc;
-    if (split_path(rows * width, width))
+    if (mfma.on || split_path(rows * width, width))
         return decode_launch(gate, up, down, x, NAIWA_BF16, slot_ids, w, rows, width, act, keep_y ? y : nullptr, 0,
-                             ws, (hipStream_t)stream, (uint16_t*)x, wait);
-    if ((rc = decode_launch(gate, up, down, x, NAIWA_BF16, slot_ids, w, rows, width, act, y, 0, ws,
+                             mfma, ws, (hipStream_t)stream, (uint16_t*)x, wait);
+    if ((rc = decode_launch(gate, up, down, x, NAIWA_BF16, slot_ids, w, rows, width, act, y, 0, mfma, ws,
                             (hipStream_t)stream, nullptr, wait)))
         return rc;
     return naiwa_residual_add_bf16(x, y, (int64_t)rows * gate->k, stream);
@@ -1060,9 +1097,9 @@ int naiwa_moe_decode_wait(const naiwa_bank* gate, const naiwa_bank* up, const na
     if (rc || rows == 0) return rc;
     if (wait && (!wait->flag || !wait->fail)) return NAIWA_E_INVALID;
     uint8_t* ws = nullptr;
+    const MfmaPlan mfma = mfma_plan(gate, up, down, x, rows, width, kMfmaScratchMax);
     if (width > 0) {
-        const DecodeScratch L(rows, width, gate->k, gate->n, down->dtype);
-        ws = (uint8_t*)naiwa_scratch(NAIWA_SCRATCH_DECODE, L.total, &rc);
+        ws = (uint8_t*)naiwa_scratch(NAIWA_SCRATCH_DECODE, call_bytes(mfma, gate, down, rows, width), &rc);
         if (!ws) return rc;
     } else if (wait) {
         // nothing to compute: the wait still orders the stream
@@ -1070,8 +1107,8 @@ int naiwa_moe_decode_wait(const naiwa_bank* gate, const naiwa_bank* up, const na
             WaitArg{wait->flag, wait->target, wait->limit_ticks, wait->fail});
         if ((rc = naiwa_hip_rc(hipGetLastError()))) return rc;
     }
-    return decode_launch(gate, up, down, x, x_dtype, slot_ids, w, rows, width, act, out, 0, ws, (hipStream_t)stream,
-                         nullptr, width > 0 ? wait : nullptr);
+    return decode_launch(gate, up, down, x, x_dtype, slot_ids, w, rows, width, act, out, 0, mfma, ws,
+                         (hipStream_t)stream, nullptr, width > 0 ? wait : nullptr);
 }
 
 extern "C" int naiwa_moe_decode(const naiwa_bank* gate, const naiwa_bank* up, const naiwa_bank* down,

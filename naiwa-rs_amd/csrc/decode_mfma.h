@@ -1,20 +1,31 @@
-// The expert GEMMs of naiwa_moe_decode calls with several tokens per expert, on
-// the matrix cores (prefill.hip): x -> bf16 in the 16x16x32 K order, gate/up per
-// (64 features, slot segment), down per (64 rows, K part, slot segment) into
-// unweighted partial dots that the decode's ordered combine adds up.
+// naiwa_moe_decode calls of several rows, with the expert GEMMs on the matrix cores
+// (decode_mfma.hip): segments and activations in one launch, gate/up per (64
+// features, slot segment), down per (rows, K part, slot segment) into unweighted
+// partial dots, and the ordered combine.
 #pragma once
 
 #include "common.h"
 
+// Most pairs per token the combine orders.
+#define NAIWA_MFMA_MAX_WIDTH 16
+
 // Whether the call's formats and shapes fit the matrix-core decode.
 bool naiwa_decode_mfma_ok(const naiwa_bank* gate, const naiwa_bank* up, const naiwa_bank* down, const void* x);
 
-// Scratch bytes of its bf16 x [rows, H] and h [n, I].
-size_t naiwa_decode_mfma_bytes(int rows, int n, int H, int I);
+// Scratch of one pass over `rows` rows.
+struct NaiwaMfmaLayout {
+    size_t off_key, off_begin, off_perm, off_inv, off_xa, off_xs, off_xr, off_ha, off_hs, off_he, off_dpart, total;
+    NaiwaMfmaLayout(int rows, int width, int H, int I, int kparts);
+};
 
-// The launches: ws holds naiwa_decode_mfma_bytes bytes; dpart receives K parts of
-// ks values of I: dpart[(part * n + sorted position) * H + row].
-int naiwa_decode_mfma_experts(const naiwa_bank* gate, const naiwa_bank* up, const naiwa_bank* down, const void* x,
-                              int x_dtype, int rows, int width, int act, int n, int seg_bound, int ks,
-                              const int* seg_count, const uint32_t* seg_key, const uint32_t* seg_begin,
-                              const uint32_t* perm, uint8_t* ws, float* dpart, hipStream_t st);
+// The most rows (of `rows`, halved until they fit) one pass may take with `bytes` of scratch.
+// A row's result does not depend on the rows beside it, so a call in several passes gives
+// the bits of one pass.
+int naiwa_decode_mfma_rows_per_pass(int rows, int width, int H, int I, int kparts, size_t bytes);
+
+// One pass over scratch ws (NaiwaMfmaLayout(rows, ...).total bytes): out = (accumulate ? out
+// : 0) + the weighted experts, and with res (bf16 [rows, H]) x = bf16(x + out) in place
+// (out may then be null).  K parts of ks values of I, kparts of them.
+int naiwa_decode_mfma(const naiwa_bank* gate, const naiwa_bank* up, const naiwa_bank* down, const void* x, int x_dtype,
+                      const uint32_t* slot_ids, const float* w, int rows, int width, int act, float* out,
+                      int accumulate, uint16_t* res, int ks, int kparts, uint8_t* ws, hipStream_t st);

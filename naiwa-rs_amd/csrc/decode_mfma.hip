@@ -1,0 +1,866 @@
+// Multi-token decode on the matrix cores: the expert GEMMs of naiwa_moe_decode
+// calls of several rows, exact in the weights.
+//
+// A block of 4 waves takes one slot segment (the sorted pairs of one slot) and a
+// strip of weight rows (64 gate and the same 64 up rows, or 128 down rows);
+// chunks of up to MR of the segment's tokens are the A operand of
+// v_mfma_f32_16x16x32_f16.  Lane l = 16 g + m holds A[m][8 g + 0..7] (token m),
+// B[8 g + 0..7][m] (weight row m of the wave's 16) and D[4 g + i][m].
+//
+// What bounds it: the weights are read once per chunk of tokens and nothing else
+// is large, so HBM.  A lane that loads its own rows' pieces into registers
+// touches 16 rows with each 16-byte load, and the cache's line lookups then cap
+// the stream (4.36 TB/s for a load-only kernel on a 528 MB gate/up bank of K
+// 4096, against 6.1 for a linear read).  Here each wave copies its rows' bytes
+// to LDS by DMA with consecutive lanes on consecutive pieces of a row (5.5 TB/s
+// for the copies alone) and the lanes unpack from LDS.  Measured, router included,
+// against register loads with weights rounded to bf16 (time; bytes of weights / time):
+// 8 rows of 128 experts top-8 at H 2048, I 768, Q4_K 69.7 -> 58.3 us (2.4 TB/s; five
+// launches' starts are 20 us of it), 96 rows 1,310 (the vector path then) -> 115 us
+// (3.0 TB/s); 8 experts top-2 at H 4096, I 14336 16 rows 213 -> 187-193 us (4.1-4.2),
+// 64 rows 258 -> 227-245 us (3.2-3.5).  The distance to a 64-bit reference fell from
+// 3.3e-3 (1.7e-3 on the vector path) to 2.1e-4.
+//
+// Exact operands.  A quantised weight is an integer times a scale, so the B
+// operand is that integer in f16 and the scales are applied in f32 afterwards:
+//   Q4_K: sc * q (6-bit scale times nibble, at most 945) is exact in f16; one
+//         packed fma makes two of them.  Over a 256-value block D = sum (sc q) x
+//         and M = sum m6_j X_j (X_j the activation sums of the 8 sub-blocks, as
+//         two f16 terms each, on one 16x16x16 MFMA): y += d D - dmin M;
+//   Q8_0: q (signed byte) is exact in f16; per 32-value block y += d sum q x.
+// Activations are f16 times a power of two per row chosen from the row's largest
+// magnitude (2^9 <= max < 2^10), so any finite f32 row fits: a bf16 value within
+// 2^-23 of the row's largest is kept exactly and smaller ones to 2^-34 of it.
+//   x: one scale per token (prep kernel);
+//   h: one scale per (pair, 64 features), the block's own strip, stored beside it;
+//      the down kernel brings a row's strips to one scale as it reads the A operand.
+//
+// K order: group G = 4 s + g of 8 f16 is lane group g's A operand at step s.
+//   Q4_K (256 values): lane group g takes 64-value chunk g; step s = 2 p + t its
+//        quant bytes 8 p + 0..7, low nibbles for t = 0 and high ones for t = 1:
+//        values 64 g + 32 t + 8 p + (0 2 1 3 4 6 5 7);
+//   Q8_0 (128 values): step s is block s, so that D has one scale: values
+//        32 s + 8 g + 0..7, the natural order.
+#include "decode_mfma.h"
+#include "common.h"
+#include "segments.h"
+
+#include <algorithm>
+
+namespace {
+
+typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+typedef _Float16 half4v __attribute__((ext_vector_type(4)));
+typedef _Float16 half8v __attribute__((ext_vector_type(8)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kThreads = 256; // 4 waves of 16 weight rows (per matrix)
+constexpr int kF = 64;        // weight rows per block and matrix
+constexpr int kChunk = 64;    // features of h that share one scale: a gate/up block's strip
+
+struct Bank {
+    const uint8_t* base;
+    int64_t stride;
+    int64_t row_bytes;
+};
+
+template <int DT> struct KB;
+template <> struct KB<NAIWA_Q4_K> {
+    static constexpr int kVals = 256, kSteps = 8, kGroups = 32, kBytes = NAIWA_Q4_K_BYTES;
+};
+template <> struct KB<NAIWA_Q8_0> {
+    static constexpr int kVals = 128, kSteps = 4, kGroups = 16, kBytes = 4 * NAIWA_Q8_0_BYTES;
+};
+
+// Element i of a laid-out Q4_K run of 8 values holds value q4_elem(i) of the run (an involution).
+__host__ __device__ constexpr int q4_elem(int i) { return (i == 1 || i == 2 || i == 5 || i == 6) ? (i ^ 3) : i; }
+
+// The group that holds run r (values 8 r .. 8 r + 7) of a K-block.
+template <int DT>
+__device__ __forceinline__ int group_of_run(int r) {
+    if (DT == NAIWA_Q4_K) {
+        const int g = r >> 3, t = (r >> 2) & 1, p = r & 3;
+        return 4 * (2 * p + t) + g;
+    }
+    return r;
+}
+
+// The power of two that brings magnitude mx to [2^9, 2^10), as its exponent (at most
+// 126, so that an all-zero or tiny row's scale and its inverse stay normal numbers).
+__device__ __forceinline__ int scale_exp(float mx) { return min(126, 136 - (int)((__float_as_uint(mx) >> 23) & 255u)); }
+__device__ __forceinline__ float pow2f(int e) { return __uint_as_float((uint32_t)(e + 127) << 23); }
+
+// A run of 8 f32 values (natural order), scaled and rounded to f16 in the K order of DT;
+// sum: the sum of the rounded values.
+template <int DT>
+__device__ __forceinline__ half8v pack_run(const float (&f)[8], float scale, float& sum) {
+    half8v o;
+    sum = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const _Float16 v = (_Float16)(f[DT == NAIWA_Q4_K ? q4_elem(i) : i] * scale);
+        o[i] = v;
+        sum += (float)v;
+    }
+    return o;
+}
+
+// Slot of sub-block sum j (0..7) of a K-block: f16 halves hi [0..7] and lo [8..15].
+__device__ __forceinline__ void put_sum(_Float16* s16, int j, float sum) {
+    const _Float16 hi = (_Float16)sum;
+    s16[j] = hi;
+    s16[8 + j] = (_Float16)(sum - (float)hi);
+}
+
+// ---------------------------------------------------------------------------
+// segments + activations, one launch
+// ---------------------------------------------------------------------------
+// Block 0 sorts the pairs into segments (tok: the token of each sorted position); block 1 + t lays out token t's row of x:
+// f16 groups xa [rows][H], sub-block sums xs [rows][H / 256][16] (Q4_K) and the
+// row's inverse scale xr [rows].  The two parts share nothing, and a launch of its
+// own costs each about 4.5 us of a 60 us call.
+template <int DT>
+__global__ void __launch_bounds__(kThreads)
+seg_prep_kernel(const uint32_t* slot_ids, const float* w, int n, int width, int nslots, uint32_t* tok, uint32_t* inv,
+                int* seg_count, uint32_t* seg_key, uint32_t* seg_begin, int* bad, const void* x, int x_bf16, int H,
+                _Float16* xa, _Float16* xs, float* xr) {
+    __shared__ NaiwaSegSmem sm;
+    const int tid = threadIdx.x;
+    if (blockIdx.x == 0) {
+        naiwa_segment(sm, slot_ids, w, n, nslots, tok, nullptr, seg_count, seg_key, seg_begin, bad, inv, width);
+        return;
+    }
+    const int t = blockIdx.x - 1, runs = H / 8;
+    auto run_of = [&](int run, float (&f)[8]) {
+        if (x_bf16) {
+            const u32x4 v = *reinterpret_cast<const u32x4*>((const uint16_t*)x + (size_t)t * H + 8 * run);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                f[2 * j] = __uint_as_float(v[j] << 16);
+                f[2 * j + 1] = __uint_as_float(v[j] & 0xffff0000u);
+            }
+        } else {
+            const floatx4* src = reinterpret_cast<const floatx4*>((const float*)x + (size_t)t * H + 8 * run);
+            const floatx4 a = src[0], b = src[1];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                f[j] = a[j];
+                f[4 + j] = b[j];
+            }
+        }
+    };
+    float mx = 0.0f;
+    for (int run = tid; run < runs; run += kThreads) {
+        float f[8];
+        run_of(run, f);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) mx = fmaxf(mx, fabsf(f[j]));
+    }
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) mx = fmaxf(mx, __shfl_xor(mx, m, 64));
+    float* red = reinterpret_cast<float*>(sm.part);
+    if ((tid & 63) == 0) red[tid >> 6] = mx;
+    __syncthreads();
+    mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    const int e = scale_exp(mx);
+    const float sc = pow2f(e);
+    if (tid == 0) xr[t] = pow2f(-e);
+    // whole rounds of the block, so that the lanes of a sub-block's 4 runs shuffle together
+    for (int r0 = 0; r0 < runs; r0 += kThreads) {
+        const int run = r0 + tid;
+        const bool in = run < runs;
+        float f[8] = {}, sum;
+        if (in) run_of(run, f);
+        const half8v o = pack_run<DT>(f, sc, sum);
+        constexpr int R = KB<DT>::kVals / 8;
+        const int kb = run / R, r = run % R;
+        if (in) *reinterpret_cast<half8v*>(xa + (size_t)t * H + kb * KB<DT>::kVals + 8 * group_of_run<DT>(r)) = o;
+        if (DT == NAIWA_Q4_K) {
+            sum += __shfl_xor(sum, 1, 64);
+            sum += __shfl_xor(sum, 2, 64);
+            if (in && (r & 3) == 0) put_sum(xs + ((size_t)t * (H / 256) + kb) * 16, r >> 2, sum);
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// LDS DMA
+// ---------------------------------------------------------------------------
+// lane i of the wave copies 16 (or 4) bytes from base + off to lds + 16 i (4 i).  Issued
+// as inline assembly so that the compiler does not make every later LDS read wait for
+// every copy in flight; each read of copied data follows an explicit vmcnt wait of the
+// issuing wave and, where another wave reads it, a barrier.  M0 is reserved and written
+// only here.
+__device__ __forceinline__ uint32_t lds_addr(const void* p) {
+    return __builtin_amdgcn_readfirstlane((uint32_t)(size_t)(__attribute__((address_space(3))) const void*)p);
+}
+__device__ __forceinline__ void dma16(const void* base, uint32_t off, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                 :: "v"(off), "s"(base), "s"(lds) : "memory", "m0");
+}
+__device__ __forceinline__ void dma4(const void* base, uint32_t off, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
+                 :: "v"(off), "s"(base), "s"(lds) : "memory", "m0");
+}
+__device__ __forceinline__ void wait_copies() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// A tile of MR token rows of one K-block.  One DMA instruction brings kRpd whole rows
+// (the lanes cover them piece by piece); row m's piece c holds group c ^ (m % kRpd) and
+// each instruction's rows start 16 kRpd bytes further on, so the 16 rows' pieces of one
+// group fall on distinct banks while a step's read keeps a fixed offset from the lane's
+// own base: (m / kRpd) kStride + (m % kRpd) 16 kGroups + 16 (g ^ m % kRpd) + 64 s.
+template <int DT, int MR> struct ATile {
+    static constexpr int G = KB<DT>::kGroups, kRpd = 64 / G, kDma = MR / kRpd, kStride = 1024 + 16 * kRpd;
+    static constexpr bool kSums = DT == NAIWA_Q4_K;
+    __align__(16) uint8_t v[kDma * kStride];
+    __align__(16) _Float16 sums[kSums ? MR * 16 : 8]; // [row][hi 0..7 | lo 0..7]
+};
+
+// Raw weight bytes of one K-block: a wave's 16 rows of NP matrices.
+template <int DT, int NP> struct WTile {
+    static constexpr int kMat = 16 * KB<DT>::kBytes;
+    static constexpr bool k16 = DT == NAIWA_Q4_K; // 16-byte pieces; Q8_0 rows are 8-byte aligned: dwords
+    static constexpr int kPieces = kMat / (k16 ? 16 : 4);
+    static constexpr int kDma = (kPieces + 63) / 64;
+    __align__(16) uint8_t v[NP * kMat];
+};
+
+// The lane's unpacking of its weight row's K-block, from LDS into B operands and scales.
+struct NibMask {
+    uint32_t lo, hi;
+};
+__device__ __forceinline__ NibMask nib_mask() {
+    NibMask n{0x000F000Fu, 0x00F000F0u};
+    asm("" : "+v"(n.lo)); // masks in VGPRs: (w & mask) | magic is then one v_and_or_b32
+    asm("" : "+v"(n.hi));
+    return n;
+}
+__device__ __forceinline__ half2v h2(uint32_t v) { return __builtin_bit_cast(half2v, v); }
+__device__ __forceinline__ half2v splat(_Float16 v) { return half2v{v, v}; }
+
+// Two bytes of w (at bits 0 and 16 after masking) as f16 integers.
+__device__ __forceinline__ half2v bytes_f16(uint32_t w, uint32_t sel) {
+    return h2(__builtin_amdgcn_perm(0x64646464u, w, sel)) - splat((_Float16)1024.0f);
+}
+
+// One lane's raw weight words of a K-block (NP rows), out of LDS: the stage is free for the
+// next copies as soon as every lane holds its own.
+template <int DT, int NP> struct WRegs;
+template <int NP> struct WRegs<NAIWA_Q4_K, NP> {
+    u32x4 hd[NP], q0[NP], q1[NP]; // header; quant bytes 0-15 and 16-31 of 64-value chunk g
+    __device__ __forceinline__ void load(const WTile<NAIWA_Q4_K, NP>& wt, int g, int m) {
+#pragma unroll
+        for (int q = 0; q < NP; ++q) {
+            const uint8_t* row = wt.v + q * WTile<NAIWA_Q4_K, NP>::kMat + m * NAIWA_Q4_K_BYTES;
+            hd[q] = *reinterpret_cast<const u32x4*>(row);
+            q0[q] = *reinterpret_cast<const u32x4*>(row + 16 + 32 * g);
+            q1[q] = *reinterpret_cast<const u32x4*>(row + 32 + 32 * g);
+        }
+    }
+};
+template <int NP> struct WRegs<NAIWA_Q8_0, NP> {
+    // block s: d at byte 34 s, this lane's 8 codes from 34 s + 2 + 8 g; even blocks start on
+    // a word (codes in 3 words from 34 s + 8 g), odd ones 2 bytes into one (codes in 2 words)
+    uint32_t ev[NP][2][3], od[NP][2][2], dw[NP][4];
+    __device__ __forceinline__ void load(const WTile<NAIWA_Q8_0, NP>& wt, int g, int m) {
+#pragma unroll
+        for (int q = 0; q < NP; ++q)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const uint8_t* blk = wt.v + q * WTile<NAIWA_Q8_0, NP>::kMat + m * KB<NAIWA_Q8_0>::kBytes + 2 * j * NAIWA_Q8_0_BYTES;
+                const uint32_t* p = reinterpret_cast<const uint32_t*>(blk + 8 * g);
+#pragma unroll
+                for (int i = 0; i < 3; ++i) ev[q][j][i] = p[i];
+#pragma unroll
+                for (int i = 0; i < 2; ++i) od[q][j][i] = p[9 + i];
+                dw[q][2 * j] = *reinterpret_cast<const uint32_t*>(blk);
+                dw[q][2 * j + 1] = *reinterpret_cast<const uint32_t*>(blk + 32);
+            }
+    }
+    __device__ __forceinline__ float d(int q, int s) const {
+        return naiwa_f16_to_f32((s & 1) ? dw[q][s] >> 16 : dw[q][s] & 0xffffu);
+    }
+    __device__ __forceinline__ uint32_t code(int q, int s, int i) const {
+        return (s & 1) ? od[q][s >> 1][i] : __builtin_amdgcn_alignbyte(ev[q][s >> 1][i + 1], ev[q][s >> 1][i], 2);
+    }
+};
+
+// One K-block of a wave: acc[q][mt] += rows q of the weights times the A tile's subtiles.
+// fac (h only): the row's per-chunk f16 factors from this K-block's chunk on.
+template <int DT, int NP, int MT, int MR, bool HF>
+__device__ __forceinline__ void kblock(const WRegs<DT, NP>& wr, const ATile<DT, MR>& at, const uint16_t* fac, int fst,
+                                       int g, int m, const NibMask& nm, floatx4 (&acc)[NP][MT]) {
+    using A = ATile<DT, MR>;
+    auto arow = [&](int mt) { return MR < 16 ? (m & (MR - 1)) : 16 * mt + m; };
+    const uint8_t* abase[MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+        const int r = arow(mt), c = r % A::kRpd;
+        abase[mt] = at.v + (r / A::kRpd) * A::kStride + c * (16 * A::G) + 16 * (g ^ c);
+    }
+    auto ld_a = [&](int mt, int s) {
+        return __builtin_bit_cast(half8v, *reinterpret_cast<const u32x4*>(abase[mt] + 64 * s));
+    };
+    if constexpr (DT == NAIWA_Q4_K) {
+        half2v sc[NP];
+        half4v m6[NP];
+        float d[NP], dmin[NP];
+#pragma unroll
+        for (int q = 0; q < NP; ++q) {
+            const u32x4 hd = wr.hd[q];
+            d[q] = naiwa_f16_to_f32(hd.x & 0xffffu);
+            dmin[q] = naiwa_f16_to_f32(hd.x >> 16);
+            // scales of sub-blocks 2 g and 2 g + 1; mins of sub-blocks 4 (g % 2) .. + 3
+            const uint32_t slo = hd.y & 0x3f3f3f3fu, shi = (hd.w & 0x0f0f0f0fu) | ((hd.y >> 2) & 0x30303030u);
+            const uint32_t mlo = hd.z & 0x3f3f3f3fu, mhi = ((hd.w >> 4) & 0x0f0f0f0fu) | ((hd.z >> 2) & 0x30303030u);
+            const uint32_t sw = (g & 2) ? shi : slo, mw = (g & 1) ? mhi : mlo;
+            sc[q] = bytes_f16(sw, (g & 1) ? 0x04030402u : 0x04010400u);
+            const half2v a = bytes_f16(mw, 0x04010400u), b = bytes_f16(mw, 0x04030402u);
+            m6[q] = half4v{a[0], a[1], b[0], b[1]};
+        }
+        half4v xs[MT];
+        half2v fg[MT];
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            xs[mt] = __builtin_bit_cast(half4v, *reinterpret_cast<const u32x2*>(at.sums + arow(mt) * 16 + 4 * g));
+            if constexpr (HF) {
+                const uint16_t* f = fac + arow(mt) * fst;
+                fg[mt] = splat(__builtin_bit_cast(_Float16, f[g]));
+                const half2v fj = h2(*reinterpret_cast<const uint32_t*>(f + 2 * (g & 1)));
+                xs[mt] *= half4v{fj[0], fj[0], fj[1], fj[1]};
+            }
+        }
+        floatx4 D[NP][MT], M[NP][MT];
+#pragma unroll
+        for (int q = 0; q < NP; ++q)
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                D[q][mt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+                M[q][mt] = __builtin_amdgcn_mfma_f32_16x16x16f16(xs[mt], m6[q], D[q][mt], 0, 0, 0);
+            }
+#pragma unroll
+        for (int s = 0; s < KB<DT>::kSteps; ++s) {
+            const int p = s >> 1, t = s & 1;
+            half8v a8[MT];
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                a8[mt] = ld_a(mt, s);
+                if constexpr (HF) {
+                    const half2v f = fg[mt];
+                    a8[mt] *= half8v{f[0], f[1], f[0], f[1], f[0], f[1], f[0], f[1]};
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < NP; ++q) {
+                const u32x4& qv = p < 2 ? wr.q0[q] : wr.q1[q];
+                const uint32_t w[2] = {(p & 1) ? qv.z : qv.x, (p & 1) ? qv.w : qv.y};
+                // (magic + nibble) * sc - magic * sc = sc * nibble, exact in one f16 fma
+                const uint32_t mk = t ? nm.hi : nm.lo, magic = t ? 0x54005400u : 0x64006400u;
+                const half2v s2 = splat(sc[q][t]), o2 = s2 * splat((_Float16)(t ? -64.0f : -1024.0f));
+                u32x4 b;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const uint32_t v = (((i & 1) ? w[i >> 1] >> 8 : w[i >> 1]) & mk) | magic;
+                    b[i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(h2(v), s2, o2));
+                }
+                const half8v b8 = __builtin_bit_cast(half8v, b);
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+                    D[q][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a8[mt], b8, D[q][mt], 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < NP; ++q)
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    acc[q][mt][i] = __builtin_fmaf(d[q], D[q][mt][i], __builtin_fmaf(-dmin[q], M[q][mt][i], acc[q][mt][i]));
+    } else {
+        half2v fc[MT];
+        if constexpr (HF) {
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) fc[mt] = h2(*reinterpret_cast<const uint32_t*>(fac + arow(mt) * fst));
+        }
+#pragma unroll
+        for (int s = 0; s < KB<DT>::kSteps; ++s) {
+            half8v a8[MT];
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                a8[mt] = ld_a(mt, s);
+                if constexpr (HF) {
+                    const _Float16 f = fc[mt][s >> 1];
+                    a8[mt] *= half8v{f, f, f, f, f, f, f, f};
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < NP; ++q) {
+                const float d = wr.d(q, s);
+                uint32_t c0 = wr.code(q, s, 0), c1 = wr.code(q, s, 1);
+                // byte ^ 0x80 = q + 128, as f16 1024 + 128 + q; minus 1152: q, exact
+                c0 ^= 0x80808080u;
+                c1 ^= 0x80808080u;
+                u32x4 b;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const uint32_t v = __builtin_amdgcn_perm(0x64646464u, i < 2 ? c0 : c1, (i & 1) ? 0x04030402u : 0x04010400u);
+                    b[i] = __builtin_bit_cast(uint32_t, h2(v) - splat((_Float16)1152.0f));
+                }
+                const half8v b8 = __builtin_bit_cast(half8v, b);
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) {
+                    const floatx4 D =
+                        __builtin_amdgcn_mfma_f32_16x16x32_f16(a8[mt], b8, floatx4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) acc[q][mt][i] = __builtin_fmaf(d, D[i], acc[q][mt][i]);
+                }
+            }
+        }
+    }
+}
+
+// LDS of one block: a weight stage per wave and two A tiles.  More weight stages cost
+// blocks: with 2 the 8- and 96-row calls at H 2048, I 768 took 63 and 131 us against 61
+// and 120, and 16 and 64 rows at H 4096, I 14336 the same 188 and 227.
+template <int DT, int NP, int MR> struct Smem {
+    WTile<DT, NP> w[kThreads / 64];
+    ATile<DT, MR> a[2];
+};
+
+// A value every lane of the wave reads, through the scalar cache (its own counter, so it
+// does not wait for copies in flight).
+__device__ __forceinline__ uint32_t scalar_ld(const uint32_t* p) {
+    return *(const __attribute__((address_space(4))) uint32_t*)(uintptr_t)p;
+}
+
+// The K loop of one chunk of MR tokens over NP matrices' 16 rows per wave.  start() sends
+// out the first copies (weights first: they need nothing but the segment), run() goes
+// through the K-blocks with one barrier each: the wave's copies for it have landed (its own
+// vmcnt), the barrier makes every wave's part of the A tile visible and frees the other A
+// buffer, the next A copies go out, the lanes take their weight words, the next K-block's
+// copies go out into the freed stage, and the K-block is computed.
+template <int DT, int NP, int MT, int MR> struct KLoop {
+    using A = ATile<DT, MR>;
+    using W = WTile<DT, NP>;
+    static constexpr int PB = W::k16 ? 16 : 4, kPer = KB<DT>::kBytes / PB; // pieces per row
+    static constexpr int kAd = (A::kDma + 3) / 4; // A copies of a wave: instructions wave, wave + 4, ...
+    Smem<DT, NP, MR>& sm;
+    const uint8_t *abase, *sums;
+    const uint8_t* wrow[NP];
+    int kb0, nkb, lane, wave;
+    uint32_t woff[W::kDma], aoff[kAd], soff[kAd];
+
+    __device__ __forceinline__ void issue_w(int kb) {
+#pragma unroll
+        for (int q = 0; q < NP; ++q) {
+            const uint8_t* wb = wrow[q] + (size_t)kb * KB<DT>::kBytes;
+#pragma unroll
+            for (int i = 0; i < W::kDma; ++i)
+                if (64 * (i + 1) <= W::kPieces || lane < W::kPieces - 64 * i) {
+                    const uint32_t l = lds_addr(sm.w[wave].v + q * W::kMat + 64 * PB * i);
+                    if (W::k16)
+                        dma16(wb, woff[i], l);
+                    else
+                        dma4(wb, woff[i], l);
+                }
+        }
+    }
+    __device__ __forceinline__ void issue_a(int kb, int buf) {
+        const uint8_t* ab = abase + (size_t)kb * (KB<DT>::kVals * 2);
+#pragma unroll
+        for (int i = 0; i < kAd; ++i) {
+            const int d = wave + 4 * i;
+            if (d >= A::kDma) break;
+            dma16(ab, aoff[i], lds_addr(sm.a[buf].v + d * A::kStride));
+            if (A::kSums && lane < 2 * A::kRpd)
+                dma16(sums + (size_t)kb * 32, soff[i], lds_addr(sm.a[buf].sums + d * A::kRpd * 16));
+        }
+    }
+    // row(i): the A row of tile row i (uniform); A rows of arow bytes, their sums of srow
+    template <class F>
+    __device__ __forceinline__ void start(int64_t row_bytes, uint32_t arow, uint32_t srow, const F& row) {
+#pragma unroll
+        for (int i = 0; i < W::kDma; ++i) {
+            const int p = min(lane + 64 * i, W::kPieces - 1);
+            woff[i] = (uint32_t)((p / kPer) * row_bytes) + (uint32_t)(p % kPer) * PB;
+        }
+        issue_w(kb0);
+#pragma unroll
+        for (int i = 0; i < kAd; ++i) {
+            const int d = min(wave + 4 * i, A::kDma - 1);
+            uint32_t ra = row(d * A::kRpd), rs = ra;
+#pragma unroll
+            for (int k = 1; k < A::kRpd; ++k) {
+                const uint32_t r = row(d * A::kRpd + k);
+                ra = lane / A::G == k ? r : ra;
+                rs = (lane >> 1) == k ? r : rs;
+            }
+            aoff[i] = ra * arow + 16u * (uint32_t)((lane % A::G) ^ (lane / A::G));
+            soff[i] = rs * srow + 16u * (uint32_t)(lane & 1);
+        }
+        issue_a(kb0, 0);
+    }
+    template <bool HF, int NFAC>
+    __device__ __forceinline__ void run(const uint16_t (*fac)[NFAC], floatx4 (&acc)[NP][MT]) {
+        const int g = lane >> 4, m = lane & 15;
+        const NibMask nm = nib_mask();
+        for (int j = 0; j < nkb; ++j) {
+            const int jn = min(j + 1, nkb - 1);
+            wait_copies();
+            lds_barrier();
+            issue_a(kb0 + jn, (j + 1) & 1);
+            WRegs<DT, NP> wr;
+            wr.load(sm.w[wave], g, m);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // held in registers: the stage is free
+            issue_w(kb0 + jn);
+            kblock<DT, NP, MT, MR, HF>(wr, sm.a[j & 1], HF ? &fac[0][j * (KB<DT>::kVals / kChunk)] : nullptr, NFAC, g, m,
+                                       nm, acc);
+        }
+        // the last K-block's copies went out once more: they land before the LDS is used for
+        // anything else
+        wait_copies();
+        lds_barrier();
+    }
+};
+
+// gate/up: block (64 features, slot segment); h = act(gate) * up of the pair at its sorted
+// position, f16 in the K order of DD with a scale per (pair, 64 features).
+template <int DG, int DD, int MT, int MR>
+__global__ void __launch_bounds__(kThreads, 2)
+gateup_mfma_kernel(Bank gate, Bank up, const _Float16* xa, const _Float16* xs, const float* xr, int H, int I,
+                   const int* seg_count, const uint32_t* seg_key, const uint32_t* seg_begin, const uint32_t* tok,
+                   int act, _Float16* ha, _Float16* hs, int8_t* he) {
+    constexpr int kHt = kF + 4; // floats per row of the h exchange
+    __shared__ Smem<DG, 2, MR> sm;
+    static_assert(sizeof(float) * MR * kHt <= sizeof(sm), "the h exchange reuses the tiles");
+    const int sg = blockIdx.y;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int tid = threadIdx.x, g = lane >> 4, m = lane & 15;
+    // the arrays have an entry for every possible segment
+    const uint32_t slot = scalar_ld(seg_key + sg);
+    const int b = (int)scalar_ld(seg_begin + sg), e = (int)scalar_ld(seg_begin + sg + 1);
+    const int segs = (int)scalar_ld((const uint32_t*)seg_count);
+    asm volatile("" ::"s"(slot), "s"(b), "s"(e), "s"(segs)); // one round trip
+    if (sg >= segs) return;
+    const int n0 = blockIdx.x * kF;
+    const int64_t r0 = n0 + 16 * wave;
+    KLoop<DG, 2, MT, MR> kl{sm, (const uint8_t*)xa, (const uint8_t*)xs,
+                                 {gate.base + (int64_t)slot * gate.stride + r0 * gate.row_bytes,
+                                  up.base + (int64_t)slot * up.stride + r0 * up.row_bytes},
+                                 0, H / KB<DG>::kVals, lane, wave};
+    for (int c0 = b; c0 < e; c0 += MR) {
+        const int cnt = min(MR, e - c0);
+        // rows past the segment repeat its last token; their results are dropped
+        kl.start(gate.row_bytes, (uint32_t)H * 2, (uint32_t)(H / 256) * 32,
+                 [&](int r) { return scalar_ld(tok + c0 + min(r, cnt - 1)); });
+        float rs[MT][4];
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) rs[mt][i] = xr[tok[c0 + min(16 * mt + 4 * g + i, cnt - 1)]];
+        floatx4 acc[2][MT] = {};
+        kl.template run<false, 2>(nullptr, acc);
+        float* ht = reinterpret_cast<float*>(&sm);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int mm = 16 * mt + 4 * g + i;
+                if (mm < MR)
+                    ht[mm * kHt + 16 * wave + m] =
+                        naiwa_act(act, acc[0][mt][i] * rs[mt][i]) * (acc[1][mt][i] * rs[mt][i]);
+            }
+        __syncthreads();
+        // thread: one run of 8 features of one token; 8 consecutive lanes hold the strip
+#pragma unroll
+        for (int u0 = 0; u0 < MR * 8; u0 += kThreads) {
+            const int u = u0 + tid, mm = u >> 3, run = u & 7;
+            if (MR * 8 < kThreads && u >= MR * 8) break;
+            float f[8], mx = 0.0f, sum;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                f[j] = ht[mm * kHt + 8 * run + j];
+                mx = fmaxf(mx, fabsf(f[j]));
+            }
+#pragma unroll
+            for (int k = 1; k < 8; k <<= 1) mx = fmaxf(mx, __shfl_xor(mx, k, 64));
+            const int ex = scale_exp(mx);
+            const half8v o = pack_run<DD>(f, pow2f(ex), sum);
+            constexpr int KV = KB<DD>::kVals;
+            const int kb = n0 / KV, r = (n0 % KV) / 8 + run;
+            const size_t pos = c0 + mm;
+            if (DD == NAIWA_Q4_K) {
+                sum += __shfl_xor(sum, 1, 64);
+                sum += __shfl_xor(sum, 2, 64);
+            }
+            if (mm < cnt) {
+                *reinterpret_cast<half8v*>(ha + pos * I + kb * KV + 8 * group_of_run<DD>(r)) = o;
+                if (DD == NAIWA_Q4_K && (run & 3) == 0) put_sum(hs + (pos * (I / 256) + kb) * 16, r >> 2, sum);
+                if (run == 0) he[pos * (I / kChunk) + n0 / kChunk] = (int8_t)ex;
+            }
+        }
+        __syncthreads(); // the exchange is free for the next chunk
+    }
+}
+
+// down: block (128 rows, K part, slot segment); the unweighted partial dot of (K part,
+// sorted position, row) into dpart.
+template <int DD, int MT, int MR>
+__global__ void __launch_bounds__(kThreads, 2)
+down_mfma_kernel(Bank down, const _Float16* ha, const _Float16* hs, const int8_t* he, int H, int I, int ks, int npairs,
+                 const int* seg_count, const uint32_t* seg_key, const uint32_t* seg_begin, float* dpart) {
+    constexpr int NP = 2;    // two strips of 64 rows: H is a multiple of 128 in every served format
+    constexpr int kFac = 34; // K parts of at most 2048: 32 chunks, rows an odd number of words apart
+    __shared__ Smem<DD, NP, MR> sm;
+    __shared__ uint16_t fac[MR][kFac];
+    __shared__ float rs[MR];
+    const int sg = blockIdx.z;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int g = lane >> 4, m = lane & 15;
+    const uint32_t slot = scalar_ld(seg_key + sg);
+    const int b = (int)scalar_ld(seg_begin + sg), e = (int)scalar_ld(seg_begin + sg + 1);
+    const int segs = (int)scalar_ld((const uint32_t*)seg_count);
+    asm volatile("" ::"s"(slot), "s"(b), "s"(e), "s"(segs)); // one round trip
+    if (sg >= segs) return;
+    const int kp = blockIdx.y, k0 = kp * ks, kn = min(ks, I - k0);
+    const int64_t r0 = (int64_t)blockIdx.x * (NP * kF) + 16 * wave; // matrix q: rows r0 + 64 q
+    KLoop<DD, NP, MT, MR> kl{sm, (const uint8_t*)ha, (const uint8_t*)hs, {}, k0 / KB<DD>::kVals,
+                                  kn / KB<DD>::kVals, lane, wave};
+#pragma unroll
+    for (int q = 0; q < NP; ++q)
+        kl.wrow[q] = down.base + (int64_t)slot * down.stride + (r0 + kF * q) * down.row_bytes;
+    for (int c0 = b; c0 < e; c0 += MR) {
+        const int cnt = min(MR, e - c0);
+        kl.start(down.row_bytes, (uint32_t)I * 2, (uint32_t)(I / 256) * 32,
+                 [&](int r) { return (uint32_t)(c0 + min(r, cnt - 1)); });
+        // each row's scales over the K part to the smallest one of them: 32 lanes a row
+#pragma unroll
+        for (int i = 0; i < MR; i += kThreads / 32) {
+            const int r = i + (tid >> 5), c = tid & 31;
+            int ex = 127;
+            if (c < kn / kChunk) ex = he[(size_t)(c0 + min(r, cnt - 1)) * (I / kChunk) + k0 / kChunk + c];
+            int lo = ex;
+#pragma unroll
+            for (int k = 1; k < 32; k <<= 1) lo = min(lo, __shfl_xor(lo, k, 64));
+            fac[r][c] = __builtin_bit_cast(uint16_t, (_Float16)pow2f(max(lo - ex, -40)));
+            if (c == 0) rs[r] = pow2f(-lo);
+        }
+        floatx4 acc[NP][MT] = {};
+        kl.template run<true, kFac>(fac, acc);
+#pragma unroll
+        for (int q = 0; q < NP; ++q)
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int mm = 16 * mt + 4 * g + i;
+                    if (mm < cnt) dpart[((size_t)kp * npairs + c0 + mm) * H + r0 + kF * q + m] = acc[q][mt][i] * rs[mm];
+                }
+        __syncthreads(); // the scales are free for the next chunk
+    }
+}
+
+// out (token, row) from the K parts' unweighted dots: the token's pairs in ascending sorted
+// position (= ascending slot), each w * (its parts in part order), from 0 or from out.  inv
+// gives a pair's position (all ones: dropped), so a token's list takes one round of loads.
+// With res (bf16 [rows, H]): x = bf16(x + y) in place.  4 rows a lane.
+__global__ void __launch_bounds__(64)
+combine_mfma_kernel(const float* dpart, int kparts, int npairs, int H, int width, const uint32_t* inv, const float* w,
+                    int accumulate, float* out, uint16_t* res) {
+    const int lane = threadIdx.x, t = blockIdx.y, r = blockIdx.x * 256 + 4 * lane;
+    const bool in = r < H;
+    const uint32_t pos = lane < width ? inv[(size_t)t * width + lane] : 0xffffffffu;
+    const float wv = lane < width ? w[(size_t)t * width + lane] : 0.0f;
+    const size_t o = (size_t)t * H + r;
+    floatx4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    uint16_t x0[4] = {0, 0, 0, 0};
+    if (in && accumulate)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i] = out[o + i]; // out is only 4-byte aligned
+    if (in && res)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x0[i] = res[o + i];
+    int rank = 0;
+    for (int j = 0; j < width; ++j) rank += (uint32_t)__builtin_amdgcn_readlane((int)pos, j) < pos ? 1 : 0;
+    const bool valid = pos != 0xffffffffu;
+    const int cnt = __popcll(__ballot(valid));
+    // pair k of the list: its position and weight, in every lane
+    auto pair = [&](int k, uint32_t& pk, float& wk) {
+        const int src = __ffsll((long long)__ballot(valid && rank == k)) - 1;
+        pk = (uint32_t)__builtin_amdgcn_readlane((int)pos, src);
+        wk = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wv), src));
+    };
+    auto dot = [&](int p, uint32_t pk) {
+        return *reinterpret_cast<const floatx4*>(dpart + ((size_t)p * npairs + pk) * H + (in ? r : 0));
+    };
+    auto add = [&](float wk, const floatx4& v) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i] = __builtin_fmaf(wk, v[i], acc[i]);
+    };
+    constexpr int kB = 8; // loads in flight
+    if (kparts == 1) {
+        for (int k0 = 0; k0 < cnt; k0 += kB) {
+            floatx4 v[kB];
+            float wk[kB];
+#pragma unroll
+            for (int q = 0; q < kB; ++q)
+                if (k0 + q < cnt) {
+                    uint32_t pk;
+                    pair(k0 + q, pk, wk[q]);
+                    v[q] = dot(0, pk);
+                }
+#pragma unroll
+            for (int q = 0; q < kB; ++q)
+                if (k0 + q < cnt) add(wk[q], v[q]);
+        }
+    } else {
+        for (int k = 0; k < cnt; ++k) {
+            uint32_t pk;
+            float wk;
+            pair(k, pk, wk);
+            floatx4 sum;
+            for (int p0 = 0; p0 < kparts; p0 += kB) {
+                floatx4 v[kB];
+#pragma unroll
+                for (int i = 0; i < kB; ++i)
+                    if (p0 + i < kparts) v[i] = dot(p0 + i, pk);
+#pragma unroll
+                for (int i = 0; i < kB; ++i)
+                    if (p0 + i < kparts) sum = p0 + i == 0 ? v[i] : sum + v[i];
+            }
+            add(wk, sum);
+        }
+    }
+    if (!in) return;
+    if (res)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) res[o + i] = (uint16_t)naiwa_f32_to_bf16(naiwa_bf16_to_f32(x0[i]) + acc[i]);
+    if (out)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) out[o + i] = acc[i];
+}
+
+struct Call {
+    Bank g, u, d;
+    int H, I, rows, n, segs, ks, kparts, act;
+    int* seg_count;
+    uint32_t *seg_key, *seg_begin, *tok;
+    _Float16 *xa, *xs, *ha, *hs;
+    float *xr, *dpart;
+    int8_t* he;
+    hipStream_t st;
+};
+
+template <int DG, int DD, int MT, int MR>
+void experts(const Call& c) {
+    gateup_mfma_kernel<DG, DD, MT, MR><<<dim3(c.I / kF, c.segs), kThreads, 0, c.st>>>(
+        c.g, c.u, c.xa, c.xs, c.xr, c.H, c.I, c.seg_count, c.seg_key, c.seg_begin, c.tok, c.act, c.ha, c.hs, c.he);
+    down_mfma_kernel<DD, MT, MR><<<dim3(c.H / (2 * kF), c.kparts, c.segs), kThreads, 0, c.st>>>(
+        c.d, c.ha, c.hs, c.he, c.H, c.I, c.ks, c.n, c.seg_count, c.seg_key, c.seg_begin, c.dpart);
+}
+
+// Token rows of the A tile.  8: a segment of a call of at most 8 rows holds no more (unless
+// a token repeats a slot), and the smaller tile lets a fifth block fit on a CU.  32 when
+// segments average more than 8 tokens: a weight is then unpacked once per 32 tokens.
+template <int DG, int DD>
+void experts_rows(const Call& c) {
+    if (c.rows <= 8)
+        experts<DG, DD, 1, 8>(c);
+    else if (c.n > 8 * c.segs)
+        experts<DG, DD, 2, 32>(c);
+    else
+        experts<DG, DD, 1, 16>(c);
+}
+
+bool fmt_ok(int dt, int k) {
+    return (dt == NAIWA_Q4_K && k % KB<NAIWA_Q4_K>::kVals == 0) || (dt == NAIWA_Q8_0 && k % KB<NAIWA_Q8_0>::kVals == 0);
+}
+
+size_t a256(size_t b) { return (b + 255) & ~size_t(255); }
+
+} // namespace
+
+bool naiwa_decode_mfma_ok(const naiwa_bank* gate, const naiwa_bank* up, const naiwa_bank* down, const void* x) {
+    const int H = gate->k, I = gate->n;
+    if (gate->dtype != up->dtype || !fmt_ok(gate->dtype, H) || !fmt_ok(down->dtype, I)) return false;
+    if (H % kF || I % kF) return false;
+    if ((uint64_t)naiwa_row_bytes(gate->dtype, H) * 16 > UINT32_MAX || (uint64_t)naiwa_row_bytes(down->dtype, I) * 16 > UINT32_MAX)
+        return false; // 32-bit offsets within a wave's rows
+    return ((uintptr_t)x & 15) == 0; // 16-byte loads of x
+}
+
+NaiwaMfmaLayout::NaiwaMfmaLayout(int rows, int width, int H, int I, int kparts) {
+    const size_t n = (size_t)rows * width;
+    off_key = 256;
+    off_begin = off_key + a256(n * 4);
+    off_perm = off_begin + a256((n + 1) * 4);
+    off_inv = off_perm + a256(n * 4);
+    off_xa = off_inv + a256(n * 4);
+    off_xs = off_xa + a256((size_t)rows * H * 2);
+    off_xr = off_xs + a256((size_t)rows * ((H + 255) / 256) * 32);
+    off_ha = off_xr + a256((size_t)rows * 4);
+    off_hs = off_ha + a256(n * I * 2);
+    off_he = off_hs + a256(n * ((I + 255) / 256) * 32);
+    off_dpart = off_he + a256(n * (I / kChunk));
+    total = off_dpart + (size_t)kparts * n * H * 4;
+}
+
+int naiwa_decode_mfma_rows_per_pass(int rows, int width, int H, int I, int kparts, size_t bytes) {
+    // 32-bit offsets into x and h
+    int r = rows;
+    auto fits = [&](int q) {
+        return NaiwaMfmaLayout(q, width, H, I, kparts).total <= bytes && (uint64_t)q * H * 2 <= UINT32_MAX &&
+               (uint64_t)q * width * I * 2 <= UINT32_MAX;
+    };
+    while (r > 1 && !fits(r)) r = (r + 1) / 2;
+    return r;
+}
+
+int naiwa_decode_mfma(const naiwa_bank* gate, const naiwa_bank* up, const naiwa_bank* down, const void* x, int x_dtype,
+                      const uint32_t* slot_ids, const float* w, int rows, int width, int act, float* out,
+                      int accumulate, uint16_t* res, int ks, int kparts, uint8_t* ws, hipStream_t st) {
+    const int H = gate->k, I = gate->n, n = rows * width;
+    const NaiwaMfmaLayout L(rows, width, H, I, kparts);
+    Call c;
+    c.g = Bank{(const uint8_t*)gate->base, gate->slot_stride, naiwa_row_bytes(gate->dtype, H)};
+    c.u = Bank{(const uint8_t*)up->base, up->slot_stride, naiwa_row_bytes(up->dtype, H)};
+    c.d = Bank{(const uint8_t*)down->base, down->slot_stride, naiwa_row_bytes(down->dtype, I)};
+    c.H = H, c.I = I, c.rows = rows, c.n = n, c.segs = std::max(1, std::min(n, gate->slots));
+    c.ks = ks, c.kparts = kparts, c.act = act, c.st = st;
+    c.seg_count = (int*)ws;
+    c.seg_key = (uint32_t*)(ws + L.off_key);
+    c.seg_begin = (uint32_t*)(ws + L.off_begin);
+    c.tok = (uint32_t*)(ws + L.off_perm);
+    uint32_t* inv = (uint32_t*)(ws + L.off_inv);
+    c.xa = (_Float16*)(ws + L.off_xa), c.xs = (_Float16*)(ws + L.off_xs), c.xr = (float*)(ws + L.off_xr);
+    c.ha = (_Float16*)(ws + L.off_ha), c.hs = (_Float16*)(ws + L.off_hs), c.he = (int8_t*)(ws + L.off_he);
+    c.dpart = (float*)(ws + L.off_dpart);
+    const int xb = x_dtype == NAIWA_BF16;
+    const bool g4 = gate->dtype == NAIWA_Q4_K, d4 = down->dtype == NAIWA_Q4_K;
+    if (g4)
+        seg_prep_kernel<NAIWA_Q4_K><<<rows + 1, kThreads, 0, st>>>(slot_ids, w, n, width, gate->slots, c.tok, inv, c.seg_count,
+                                                                   c.seg_key, c.seg_begin, (int*)(ws + 4), x, xb, H,
+                                                                   c.xa, c.xs, c.xr);
+    else
+        seg_prep_kernel<NAIWA_Q8_0><<<rows + 1, kThreads, 0, st>>>(slot_ids, w, n, width, gate->slots, c.tok, inv, c.seg_count,
+                                                                   c.seg_key, c.seg_begin, (int*)(ws + 4), x, xb, H,
+                                                                   c.xa, c.xs, c.xr);
+    if (g4 && d4)
+        experts_rows<NAIWA_Q4_K, NAIWA_Q4_K>(c);
+    else if (g4)
+        experts_rows<NAIWA_Q4_K, NAIWA_Q8_0>(c);
+    else if (d4)
+        experts_rows<NAIWA_Q8_0, NAIWA_Q4_K>(c);
+    else
+        experts_rows<NAIWA_Q8_0, NAIWA_Q8_0>(c);
+    combine_mfma_kernel<<<dim3((H + 255) / 256, rows), 64, 0, st>>>(c.dpart, kparts, n, H, width, inv, w, accumulate, out,
+                                                                    res);
+    return naiwa_hip_rc(hipGetLastError());
+}

@@ -37,7 +37,6 @@
 // bf16 operands carry the f32 exponent range: any finite activation goes in
 // without clamping or scaling.
 #include "common.h"
-#include "decode_mfma.h"
 #include "workspace.h"
 
 namespace {
@@ -47,7 +46,6 @@ typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float float2v __attribute__((ext_vector_type(2)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kThreads = 256;  // gather helpers, prep, combine
@@ -589,293 +587,6 @@ combine_kernel(const float* ypair, const uint32_t* ids, int k, int H, int slots,
     }
 }
 
-// ---------------------------------------------------------------------------
-// Multi-token decode on the matrix cores
-// ---------------------------------------------------------------------------
-// naiwa_moe_decode calls with several tokens per expert run their expert GEMMs
-// here.  A block of 4 waves takes one slot segment (the sorted pairs of one
-// slot) and 64 features; chunks of up to 16 of the segment's tokens are the A
-// operand of v_mfma_f32_16x16x32_bf16 and each lane dequantises its own weight
-// values once into the B operand, so a weight costs the same whatever the
-// token count.  Lane l = 16 g + m holds A[m][8 g + 0..7] (token m of the
-// chunk), B[8 g + 0..7][m] (feature m of the wave's 16) and D[4 g + i][m].
-// Gate and up accumulate in the same wave, so h = act(g) * u is formed in
-// registers.
-//
-// K order of the 16x16x32 steps.  In every K-block lane group g reads:
-//   Q4_K (256 values): 64-value chunk g; step s = 2 p + t takes its quant bytes
-//        8 p + 0..7, low nibbles for t = 0 and high ones for t = 1: values
-//        64 g + 32 t + 8 p + (0 2 1 3 4 6 5 7);
-//   Q8_0 (128 values, 4 blocks): block g; step s takes its values 8 s + 0..7.
-// The activations (x for gate/up, h for down) are stored as groups G = 4 s + g
-// of 8 f16 in that order.
-constexpr int kDecM = 16;        // tokens per MFMA tile
-constexpr int kDecThreads = 256; // 4 waves of 16 features
-constexpr int kDecF = 64;        // features (gate/up) or output rows (down) per block
-
-template <int DT> struct K16;
-template <> struct K16<NAIWA_Q4_K> {
-    static constexpr int kVals = 256, kSteps = 8;
-};
-template <> struct K16<NAIWA_Q8_0> {
-    static constexpr int kVals = 128, kSteps = 4;
-};
-
-// Position, in the laid-out row, of value f of the original row.
-template <int DT>
-__host__ __device__ inline int laid16(int f) {
-    constexpr int KV = K16<DT>::kVals;
-    const int kb = f / KV, r = f % KV;
-    if (DT == NAIWA_Q4_K) {
-        const int g = r / 64, t = (r % 64) / 32, p = (r % 32) / 8;
-        return kb * KV + 8 * (4 * (2 * p + t) + g) + q4_elem(r % 8);
-    }
-    const int g = r / 32, st = (r % 32) / 8;
-    return kb * KV + 8 * (4 * st + g) + r % 8;
-}
-
-// Per-K-block scale state of one lane (Q4_K: its two sub-blocks 2 g and 2 g + 1).
-struct Scl {
-    float sc[2], mn[2];
-};
-
-// One lane's weights of one K-block (row `row`, lane group g).
-template <int DT> struct W16;
-
-template <> struct W16<NAIWA_Q4_K> {
-    u32x4 hd, q0, q1; // header; quant bytes 0-15 and 16-31 of chunk g
-    __device__ __forceinline__ void load(const uint8_t* row, int kb, int g) {
-        const uint8_t* blk = row + (size_t)kb * NAIWA_Q4_K_BYTES;
-        hd = *reinterpret_cast<const u32x4*>(blk);
-        q0 = *reinterpret_cast<const u32x4*>(blk + 16 + 32 * g);
-        q1 = *reinterpret_cast<const u32x4*>(blk + 32 + 32 * g);
-    }
-    __device__ __forceinline__ void prep(int g, Scl& c) const {
-        q4k_scale_min(hd, 2 * g, c.sc[0], c.mn[0]);
-        q4k_scale_min(hd, 2 * g + 1, c.sc[1], c.mn[1]);
-    }
-    __device__ __forceinline__ bf16x8 step(int s, const Scl& c, const NibMask& nm) const {
-        const int p = s >> 1, t = s & 1;
-        const u32x4& q = p < 2 ? q0 : q1;
-        const uint32_t da = (p & 1) ? q.z : q.x, db = (p & 1) ? q.w : q.y;
-        return q4k_unpack(da, db, t, nm, c.sc[t], c.mn[t]);
-    }
-};
-
-template <> struct W16<NAIWA_Q8_0> {
-    uint32_t w[9]; // block 4 kb + g: 9 words from its aligned start
-    int sh;        // its byte offset within the first word (0 or 2)
-    __device__ __forceinline__ void load(const uint8_t* row, int kb, int g) {
-        const int off = (4 * kb + g) * NAIWA_Q8_0_BYTES;
-        sh = off & 3;
-        const uint32_t* p = reinterpret_cast<const uint32_t*>(row + (off & ~3));
-#pragma unroll
-        for (int i = 0; i < 9; ++i) w[i] = p[i];
-    }
-    __device__ __forceinline__ void prep(int, Scl&) const {}
-    __device__ __forceinline__ bf16x8 step(int s, const Scl&, const NibMask&) const {
-        const uint32_t d0 = sh ? w[2 * s + 1] : __builtin_amdgcn_alignbyte(w[2 * s + 1], w[2 * s], 2);
-        const uint32_t d1 = sh ? w[2 * s + 2] : __builtin_amdgcn_alignbyte(w[2 * s + 2], w[2 * s + 1], 2);
-        const uint32_t dbits = sh ? (w[0] >> 16) : (w[0] & 0xffffu);
-        return q8_unpack(d0, d1, naiwa_f16_to_f32(dbits));
-    }
-};
-
-// LDS A tile of one K-block: group G of token row m at [G][m ^ (G % 16)].
-// MT subtiles of 16 token rows (a chunk of 16 MT tokens); the XOR keeps a row in its subtile.
-template <int DT, int MT> struct ATile16 {
-    static constexpr int kGroups = 4 * K16<DT>::kSteps;
-    u32x4 v[kGroups][kDecM * MT];
-    __device__ __forceinline__ u32x4& at(int G, int m) { return v[G][m ^ (G & 15)]; }
-    __device__ __forceinline__ const u32x4& at(int G, int m) const { return v[G][m ^ (G & 15)]; }
-};
-
-// Thread tid's pieces of one K-block of the A tile: piece p = tid + kDecThreads * i is
-// row p / G, group p % G (the lanes of a load cover whole rows); rows[m] < 0 is a zero row.
-template <int DT, int MT> struct AStage16 {
-    static constexpr int G = ATile16<DT, MT>::kGroups;
-    static constexpr int kRows = kDecM * MT;
-    static constexpr int kPer = (G * kRows + kDecThreads - 1) / kDecThreads;
-    u32x4 r[kPer];
-    __device__ __forceinline__ void load(const uint16_t* base, const int* rows, int kb, int tid) {
-#pragma unroll
-        for (int i = 0; i < kPer; ++i) {
-            const int p = tid + kDecThreads * i;
-            r[i] = u32x4{0u, 0u, 0u, 0u};
-            if (p < G * kRows) {
-                const int ro = rows[p / G];
-                if (ro >= 0) r[i] = *reinterpret_cast<const u32x4*>(base + ro + kb * K16<DT>::kVals + 8 * (p % G));
-            }
-        }
-    }
-    __device__ __forceinline__ void store(ATile16<DT, MT>& a, int tid) const {
-#pragma unroll
-        for (int i = 0; i < kPer; ++i) {
-            const int p = tid + kDecThreads * i;
-            if (p < G * kRows) a.at(p % G, p / G) = r[i];
-        }
-    }
-};
-
-// x (bf16 or f32) [T, H] -> xl bf16 [T, H] in the 16x16x32 K order of DT, one thread
-// per run of 8 values (bf16 input unchanged, f32 rounded to nearest-even bf16).
-template <int DT>
-__global__ void __launch_bounds__(kThreads) dec_prep_kernel(const void* x, int x_bf16, int T, int H, uint16_t* xl) {
-    const int runs = H / 8;
-    const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-    const bool in = i < (int64_t)T * runs;
-    const int t = in ? (int)(i / runs) : 0, run = in ? (int)(i % runs) : 0;
-    float f[8] = {};
-    if (in) {
-        if (x_bf16) {
-            const uint4 v = *reinterpret_cast<const uint4*>((const uint16_t*)x + (size_t)t * H + 8 * run);
-            const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                f[2 * j] = __uint_as_float(w[j] << 16);
-                f[2 * j + 1] = __uint_as_float(w[j] & 0xffff0000u);
-            }
-        } else {
-            const float4* src = reinterpret_cast<const float4*>((const float*)x + (size_t)t * H + 8 * run);
-            const float4 a = src[0], b = src[1];
-            f[0] = a.x; f[1] = a.y; f[2] = a.z; f[3] = a.w;
-            f[4] = b.x; f[5] = b.y; f[6] = b.z; f[7] = b.w;
-        }
-    }
-    if (!in) return;
-    float g[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) g[e] = f[DT == NAIWA_Q4_K ? q4_elem(e) : e];
-    uint4 o;
-    o.x = bf16x2_bits(g[0], g[1]);
-    o.y = bf16x2_bits(g[2], g[3]);
-    o.z = bf16x2_bits(g[4], g[5]);
-    o.w = bf16x2_bits(g[6], g[7]);
-    *reinterpret_cast<uint4*>(xl + (size_t)t * H + laid16<DT>(8 * run)) = o;
-}
-
-// The K-block loop of one chunk of 16 MT tokens: NP weight rows (gate and up, or down)
-// against the A rows listed in `rows`, K-blocks kb0 .. kb0 + nkb - 1; each step's
-// dequantised B operand serves the MT subtiles.
-template <int DT, int NP, int MT>
-__device__ __forceinline__ void dec_chunk(const uint16_t* abase, const int* rows, const uint8_t* const* wrow,
-                                          int kb0, int nkb, ATile16<DT, MT>* as, int tid, int g, int m,
-                                          floatx4 (&acc)[NP][MT]) {
-    AStage16<DT, MT> st;
-    W16<DT> cur[NP], nxt[NP];
-    const NibMask nm = nib_mask();
-    st.load(abase, rows, kb0, tid);
-#pragma unroll
-    for (int q = 0; q < NP; ++q) cur[q].load(wrow[q], kb0, g);
-    st.store(as[0], tid);
-    __syncthreads();
-    // one K-block; the next one's loads are unconditional (the last block reloads
-    // itself) so the compiler waits only for this block's registers
-    auto block = [&](int j, const W16<DT>* bw, W16<DT>* nw) {
-        const int kn = kb0 + min(j + 1, nkb - 1);
-        st.load(abase, rows, kn, tid);
-#pragma unroll
-        for (int q = 0; q < NP; ++q) nw[q].load(wrow[q], kn, g);
-        Scl c[NP];
-#pragma unroll
-        for (int q = 0; q < NP; ++q) bw[q].prep(g, c[q]);
-        const ATile16<DT, MT>& a = as[j & 1];
-#pragma unroll
-        for (int s = 0; s < K16<DT>::kSteps; ++s) {
-            bf16x8 x8[MT];
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt) x8[mt] = __builtin_bit_cast(bf16x8, a.at(4 * s + g, kDecM * mt + m));
-#pragma unroll
-            for (int q = 0; q < NP; ++q) {
-                const bf16x8 b = bw[q].step(s, c[q], nm);
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt)
-                    acc[q][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x8[mt], b, acc[q][mt], 0, 0, 0);
-            }
-        }
-        st.store(as[(j + 1) & 1], tid);
-        lds_barrier();
-    };
-    int j = 0;
-    for (; j + 2 <= nkb; j += 2) {
-        block(j, cur, nxt);
-        block(j + 1, nxt, cur);
-    }
-    if (j < nkb) block(j, cur, nxt);
-}
-
-// gate/up: block (64 features, slot segment); h = act(gate) * up as bf16 at the
-// pair's sorted position, in the 16x16x32 K order of DD.
-template <int DG, int DD, int MT>
-__global__ void __launch_bounds__(kDecThreads, 2)
-dec_gateup_kernel(Bank gate, Bank up, const uint16_t* xl, int H, int I, int width, const int* seg_count,
-                  const uint32_t* seg_key, const uint32_t* seg_begin, const uint32_t* perm, int act, uint16_t* hl) {
-    constexpr int CM = kDecM * MT; // tokens per chunk
-    __shared__ ATile16<DG, MT> as[2];
-    __shared__ int rows[CM];
-    const int sg = blockIdx.y;
-    if (sg >= *seg_count) return;
-    const int tid = threadIdx.x, lane = tid & 63, m = lane & 15, g = lane >> 4;
-    const uint32_t slot = seg_key[sg];
-    const int b = (int)seg_begin[sg], e = (int)seg_begin[sg + 1];
-    const int n = blockIdx.x * kDecF + 16 * (tid >> 6) + m;
-    const uint8_t* wrow[2] = {gate.base + (int64_t)slot * gate.stride + (int64_t)n * gate.row_bytes,
-                              up.base + (int64_t)slot * up.stride + (int64_t)n * up.row_bytes};
-    const int col = laid16<DD>(n);
-    for (int c0 = b; c0 < e; c0 += CM) {
-        const int cnt = min(CM, e - c0);
-        __syncthreads(); // the previous chunk is done with rows and the A tiles
-        if (tid < CM) rows[tid] = tid < cnt ? (int)(perm[c0 + tid] / (uint32_t)width) * H : -1;
-        __syncthreads();
-        floatx4 acc[2][MT] = {};
-        dec_chunk<DG, 2, MT>(xl, rows, wrow, 0, H / K16<DG>::kVals, as, tid, g, m, acc);
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int mm = kDecM * mt + 4 * g + i;
-                if (mm < cnt)
-                    hl[(size_t)(c0 + mm) * I + col] =
-                        (uint16_t)bf16x2_bits(naiwa_act(act, acc[0][mt][i]) * acc[1][mt][i], 0.0f);
-            }
-    }
-}
-
-// down: block (64 output rows, K part, slot segment); the unweighted partial dot of
-// (K part, sorted position, row) into dpart.
-template <int DD, int MT>
-__global__ void __launch_bounds__(kDecThreads, 2)
-dec_down_kernel(Bank down, const uint16_t* hl, int H, int I, int ks, int npairs, const int* seg_count,
-                const uint32_t* seg_key, const uint32_t* seg_begin, float* dpart) {
-    constexpr int CM = kDecM * MT;
-    __shared__ ATile16<DD, MT> as[2];
-    __shared__ int rows[CM];
-    const int sg = blockIdx.z;
-    if (sg >= *seg_count) return;
-    const int tid = threadIdx.x, lane = tid & 63, m = lane & 15, g = lane >> 4;
-    const uint32_t slot = seg_key[sg];
-    const int b = (int)seg_begin[sg], e = (int)seg_begin[sg + 1];
-    const int kp = blockIdx.y, k0 = kp * ks;
-    const int r = blockIdx.x * kDecF + 16 * (tid >> 6) + m;
-    const uint8_t* wrow[1] = {down.base + (int64_t)slot * down.stride + (int64_t)r * down.row_bytes};
-    for (int c0 = b; c0 < e; c0 += CM) {
-        const int cnt = min(CM, e - c0);
-        __syncthreads();
-        if (tid < CM) rows[tid] = tid < cnt ? (c0 + tid) * I : -1;
-        __syncthreads();
-        floatx4 acc[1][MT] = {};
-        dec_chunk<DD, 1, MT>(hl, rows, wrow, k0 / K16<DD>::kVals, min(ks, I - k0) / K16<DD>::kVals, as, tid, g, m,
-                             acc);
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int mm = kDecM * mt + 4 * g + i;
-                if (mm < cnt) dpart[((size_t)kp * npairs + c0 + mm) * H + r] = acc[0][mt][i];
-            }
-    }
-}
-
 // K of a projection in this format: whole K-blocks.
 bool fmt_ok(int dtype, int kdim) {
     return (dtype == NAIWA_Q4_K && kdim % KBlock<NAIWA_Q4_K>::kVals == 0) ||
@@ -888,75 +599,7 @@ void launch_gateup(dim3 g, hipStream_t st, Bank bg, Bank bu, const uint16_t* xp,
     gateup_kernel<DG, DD><<<g, kGemm, 0, st>>>(bg, bu, xp, H, I, k, perm, tl, act, hp, xcd);
 }
 
-template <int MT>
-void dec_experts(bool g4, bool d4, dim3 g1, dim3 g2, Bank bg, Bank bu, Bank bd, const uint16_t* xl, uint16_t* hl,
-                 int H, int I, int width, int ks, int n, const int* seg_count, const uint32_t* seg_key,
-                 const uint32_t* seg_begin, const uint32_t* perm, int act, float* dpart, hipStream_t st) {
-    if (g4 && d4)
-        dec_gateup_kernel<NAIWA_Q4_K, NAIWA_Q4_K, MT><<<g1, kDecThreads, 0, st>>>(bg, bu, xl, H, I, width, seg_count,
-                                                                                  seg_key, seg_begin, perm, act, hl);
-    else if (g4)
-        dec_gateup_kernel<NAIWA_Q4_K, NAIWA_Q8_0, MT><<<g1, kDecThreads, 0, st>>>(bg, bu, xl, H, I, width, seg_count,
-                                                                                  seg_key, seg_begin, perm, act, hl);
-    else if (d4)
-        dec_gateup_kernel<NAIWA_Q8_0, NAIWA_Q4_K, MT><<<g1, kDecThreads, 0, st>>>(bg, bu, xl, H, I, width, seg_count,
-                                                                                  seg_key, seg_begin, perm, act, hl);
-    else
-        dec_gateup_kernel<NAIWA_Q8_0, NAIWA_Q8_0, MT><<<g1, kDecThreads, 0, st>>>(bg, bu, xl, H, I, width, seg_count,
-                                                                                  seg_key, seg_begin, perm, act, hl);
-    if (d4)
-        dec_down_kernel<NAIWA_Q4_K, MT><<<g2, kDecThreads, 0, st>>>(bd, hl, H, I, ks, n, seg_count, seg_key, seg_begin,
-                                                                     dpart);
-    else
-        dec_down_kernel<NAIWA_Q8_0, MT><<<g2, kDecThreads, 0, st>>>(bd, hl, H, I, ks, n, seg_count, seg_key, seg_begin,
-                                                                     dpart);
-}
-
 } // namespace
-
-bool naiwa_decode_mfma_ok(const naiwa_bank* gate, const naiwa_bank* up, const naiwa_bank* down, const void* x) {
-    const int H = gate->k, I = gate->n;
-    auto fmt = [](int dt, int k) {
-        return (dt == NAIWA_Q4_K && k % K16<NAIWA_Q4_K>::kVals == 0) ||
-               (dt == NAIWA_Q8_0 && k % K16<NAIWA_Q8_0>::kVals == 0);
-    };
-    if (gate->dtype != up->dtype || !fmt(gate->dtype, H) || !fmt(down->dtype, I)) return false;
-    if (H % kDecF || I % kDecF) return false;
-    return ((uintptr_t)x & 15) == 0; // 16-byte loads of x
-}
-
-size_t naiwa_decode_mfma_bytes(int rows, int n, int H, int I) {
-    return (((size_t)rows * H * 2 + 255) & ~size_t(255)) + (size_t)n * I * 2;
-}
-
-int naiwa_decode_mfma_experts(const naiwa_bank* gate, const naiwa_bank* up, const naiwa_bank* down, const void* x,
-                              int x_dtype, int rows, int width, int act, int n, int seg_bound, int ks,
-                              const int* seg_count, const uint32_t* seg_key, const uint32_t* seg_begin,
-                              const uint32_t* perm, uint8_t* ws, float* dpart, hipStream_t st) {
-    const int H = gate->k, I = gate->n;
-    uint16_t* xl = (uint16_t*)ws;
-    uint16_t* hl = (uint16_t*)(ws + (((size_t)rows * H * 2 + 255) & ~size_t(255)));
-    const Bank bg{(const uint8_t*)gate->base, gate->slot_stride, naiwa_row_bytes(gate->dtype, H)};
-    const Bank bu{(const uint8_t*)up->base, up->slot_stride, naiwa_row_bytes(up->dtype, H)};
-    const Bank bd{(const uint8_t*)down->base, down->slot_stride, naiwa_row_bytes(down->dtype, I)};
-    const int xb = x_dtype == NAIWA_BF16;
-    const unsigned pb = (unsigned)(((int64_t)rows * (H / 8) + kThreads - 1) / kThreads);
-    const bool g4 = gate->dtype == NAIWA_Q4_K, d4 = down->dtype == NAIWA_Q4_K;
-    if (g4)
-        dec_prep_kernel<NAIWA_Q4_K><<<pb, kThreads, 0, st>>>(x, xb, rows, H, xl);
-    else
-        dec_prep_kernel<NAIWA_Q8_0><<<pb, kThreads, 0, st>>>(x, xb, rows, H, xl);
-    const dim3 g1(I / kDecF, seg_bound), g2(H / kDecF, (I + ks - 1) / ks, seg_bound);
-    // two 16-token subtiles per chunk when the segments average more than 8 tokens:
-    // each weight is then dequantised once per 32 tokens instead of 16
-    if (n > 8 * seg_bound)
-        dec_experts<2>(g4, d4, g1, g2, bg, bu, bd, xl, hl, H, I, width, ks, n, seg_count, seg_key, seg_begin, perm,
-                       act, dpart, st);
-    else
-        dec_experts<1>(g4, d4, g1, g2, bg, bu, bd, xl, hl, H, I, width, ks, n, seg_count, seg_key, seg_begin, perm,
-                       act, dpart, st);
-    return naiwa_hip_rc(hipGetLastError());
-}
 
 extern "C" int naiwa_moe_prefill(const naiwa_bank* gate, const naiwa_bank* up, const naiwa_bank* down, const void* x,
                                  const uint32_t* slot_ids, const float* w, int T, int k, int act, float* out,

@@ -22,11 +22,13 @@ struct NaiwaSegSmem {
 
 // keys[n]; weights (may be null): an entry with weight 0 is skipped.
 // Outputs (each may be null): perm[valid entries], offsets[nkeys + 1],
-// seg_count[1], seg_key[segments], seg_begin[segments + 1], bad[1].
+// seg_count[1], seg_key[segments], seg_begin[segments + 1], bad[1], inv[n] (the
+// entry's place in perm, all ones for one left out).  per_token > 1: perm holds the entries'
+// tokens (index / per_token) instead.
 __device__ inline void naiwa_segment(NaiwaSegSmem& sm, const uint32_t* keys, const float* weights,
                                      int n, int nkeys, uint32_t* perm, uint32_t* offsets,
                                      int* seg_count, uint32_t* seg_key, uint32_t* seg_begin,
-                                     int* bad) {
+                                     int* bad, uint32_t* inv = nullptr, int per_token = 1) {
     const int tid = threadIdx.x;
     for (int b = tid; b < nkeys; b += NAIWA_SEG_THREADS) {
         sm.hist[b] = 0;
@@ -81,8 +83,8 @@ __device__ inline void naiwa_segment(NaiwaSegSmem& sm, const uint32_t* keys, con
     }
     __syncthreads();
     // Stable scatter, one chunk of 256 entries at a time.  An entry's rank among
-    // the chunk's entries of its key = its rank inside its wave (one ballot per
-    // distinct key of the wave) + the counts of that key in the lower waves.
+    // the chunk's entries of its key = its rank inside its wave + the counts of that
+    // key in the lower waves.
     const int lane = tid & 63, wave = tid >> 6;
     const uint64_t below = (1ull << lane) - 1ull;
     for (int c0 = 0; c0 < n; c0 += NAIWA_SEG_THREADS) {
@@ -92,23 +94,24 @@ __device__ inline void naiwa_segment(NaiwaSegSmem& sm, const uint32_t* keys, con
             const uint32_t kk = keys[i];
             if (kk < (uint32_t)nkeys && (!weights || weights[i] != 0.0f)) k = kk;
         }
-        uint32_t rank = 0, lead_cnt = 0; // lead_cnt: the wave's count of k, on the key's first lane
-        uint64_t todo = __ballot(k != 0xffffffffu);
-        while (todo) {
-            const int first = __ffsll((long long)todo) - 1;
-            const uint32_t key = (uint32_t)__builtin_amdgcn_readlane((int)k, first);
-            const uint64_t same = __ballot(k == key);
-            if (k == key) rank = (uint32_t)__popcll(same & below);
-            if (lane == first) lead_cnt = (uint32_t)__popcll(same);
-            todo &= ~same;
+        // the lanes with this lane's key: one ballot per key bit
+        uint64_t same = __ballot(k != 0xffffffffu);
+        for (int bit = 0; (nkeys - 1) >> bit; ++bit) {
+            const uint64_t ones = __ballot((k >> bit) & 1u);
+            same &= ((k >> bit) & 1u) ? ones : ~ones;
         }
+        uint32_t rank = (uint32_t)__popcll(same & below), lead_cnt = 0; // lead_cnt: the wave's count of k, on its first lane
+        if (k != 0xffffffffu && rank == 0) lead_cnt = (uint32_t)__popcll(same);
         if (lead_cnt) sm.wcnt[wave][k] = (uint16_t)lead_cnt;
         __syncthreads();
         if (k != 0xffffffffu) {
 #pragma unroll
             for (int w = 0; w < NAIWA_SEG_THREADS / 64; ++w)
                 if (w < wave) rank += sm.wcnt[w][k];
-            if (perm) perm[sm.hist[k] + rank] = (uint32_t)i;
+            if (perm) perm[sm.hist[k] + rank] = (uint32_t)i / (uint32_t)per_token;
+            if (inv) inv[i] = sm.hist[k] + rank;
+        } else if (inv && i < n) {
+            inv[i] = 0xffffffffu;
         }
         __syncthreads();
         if (lead_cnt) {

@@ -1,0 +1,97 @@
+"""The matrix-core decode (calls of 4 rows or more) against the oracle at the edges of its
+tiles: 8-, 16- and 32-row activation tiles and chunks past them, one and two weight strips,
+short last K parts, more than 512 pairs, rows of very different magnitudes, and the
+no-alloc entry point's passes over the rows."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import oracle as O
+import synthetic as S
+
+pytestmark = pytest.mark.gpu
+Q4, Q8 = O.Q4_K, O.Q8_0
+# Weights enter as exact integers with f32 scales, a bf16 x is kept exactly, h is rounded once to
+# f16 (relative 2^-11 a value): a row's error stays below 2^-11 sum |h w| w_j, within 1e-3 of the
+# largest output (f32 x is rounded to f16 as well: the same bound again).
+TOL = 1e-3
+
+
+def _layer(nm, seed, E, H, I, dt):
+    g, u, d, r = S.layer(seed, E, H, I, dt)
+    banks = nm.LayerBanks(E, H, I, dt)
+    for e in range(E):
+        banks.load(e, g[e], u[e], d[e])
+    # the stacks point into the arrays: the caller keeps those
+    return banks, (O.stack(g, dt[0], I, H), O.stack(u, dt[1], I, H), O.stack(d, dt[2], H, I)), (g, u, d)
+
+
+@pytest.mark.parametrize("dt,H,I,E,k,rows,x_f32", [
+    ((Q4, Q4, Q4), 256, 256, 4, 2, 4, False),       # one K-block each way
+    ((Q4, Q4, Q8), 512, 384, 5, 3, 7, True),        # 8-row tile, odd rows, f32 x
+    ((Q8, Q8, Q8), 384, 128, 3, 2, 9, False),       # 16-row tile
+    ((Q8, Q8, Q4), 128, 512, 16, 2, 17, False),
+    ((Q4, Q4, Q4), 256, 2304, 4, 2, 33, False),     # two K parts, the last 256; chunks of 32
+    ((Q4, Q4, Q8), 256, 2176, 2, 1, 65, True),      # the last K part 128; segments past 32 rows
+    ((Q4, Q4, Q4), 512, 256, 16, 8, 150, False),    # 1,200 pairs
+    ((Q8, Q8, Q8), 256, 256, 8, 16, 40, False),     # 640 pairs, the widest row of pairs
+])
+def test_exact_weights_at_tile_edges(gpu, dt, H, I, E, k, rows, x_f32):
+    nm = gpu
+    banks, stacks, keep = _layer(nm, 8100 + rows, E, H, I, dt)
+    x = S.activations_bf16(8200 + rows, rows, H)
+    xf = O.from_bf16(x)
+    rng = np.random.default_rng(rows)
+    ids = rng.integers(0, E, (rows, k)).astype(np.uint32)   # repeated slots among them
+    w = rng.random((rows, k)).astype(np.float32)
+    w[0, -1] = 0.0                                          # a padded pair
+    if x_f32:
+        xf = (xf * 1.0001).astype(np.float32)
+    xd = nm.DeviceBuffer.from_array(xf if x_f32 else x)
+    ids_d, w_d = nm.DeviceBuffer.from_array(ids), nm.DeviceBuffer.from_array(w)
+    out = nm.DeviceBuffer(rows * H * 4)
+    print(f"[mfma decode {dt} H={H} I={I} E={E} k={k} rows={rows}]", flush=True)
+    nm.indexed_moe_fused_decode(banks, xd, nm.F32 if x_f32 else nm.BF16, ids_d, w_d, rows, k, out)
+    got = out.download(np.float32).reshape(rows, H)
+    err = S.max_rel_err(got, O.fused_moe_decode(*stacks, xf, ids, w))
+    print(f"  max_rel_err={err:.3e}", flush=True)
+    assert err < TOL
+
+
+def test_rows_of_any_magnitude(gpu):
+    nm = gpu
+    E, H, I, k = 4, 256, 256, 2
+    scales = np.array([0.0, 1e-12, 1e-3, 1.0, 1e6, 1e14], np.float32)
+    banks, stacks, keep = _layer(nm, 8300, E, H, I, (Q4, Q4, Q4))
+    x = O.to_bf16(O.from_bf16(S.activations_bf16(8301, len(scales), H)) * scales[:, None])
+    ids = np.tile(np.arange(k, dtype=np.uint32), (len(scales), 1))
+    w = np.full((len(scales), k), 0.5, np.float32)
+    bufs = [nm.DeviceBuffer.from_array(a) for a in (x, ids, w)]
+    out = nm.DeviceBuffer(len(scales) * H * 4)
+    nm.indexed_moe_fused_decode(banks, bufs[0], nm.BF16, bufs[1], bufs[2], len(scales), k, out)
+    got = out.download(np.float32).reshape(len(scales), H)
+    want = O.fused_moe_decode(*stacks, O.from_bf16(x), ids, w)
+    assert not got[0].any()
+    for i in range(1, len(scales)):
+        assert S.max_rel_err(got[i], want[i]) < TOL, scales[i]
+
+
+def test_noalloc_passes_give_the_bits_of_one_pass(gpu):
+    nm = gpu
+    E, H, I, k, rows = 8, 512, 256, 8, 600     # 4,800 pairs: more than the fixed array holds in one pass
+    banks, stacks, keep = _layer(nm, 8400, E, H, I, (Q4, Q4, Q4))
+    x = S.activations_bf16(8401, rows, H)
+    rng = np.random.default_rng(1)
+    ids = rng.integers(0, E, (rows, k)).astype(np.uint32)
+    w = rng.random((rows, k)).astype(np.float32)
+    bufs = [nm.DeviceBuffer.from_array(a) for a in (x, ids, w)]
+    ref, got = nm.DeviceBuffer(rows * H * 4), nm.DeviceBuffer(rows * H * 4)
+    g, u, d = banks.gate.desc(), banks.up.desc(), banks.down.desc()
+    for fn, out in (("naiwa_moe_decode_ex", ref), ("naiwa_moe_decode_noalloc", got)):
+        rc = getattr(nm.lib(), fn)(C.byref(g), C.byref(u), C.byref(d), bufs[0].ptr, nm.BF16, bufs[1].ptr, bufs[2].ptr,
+                                   rows, k, nm.ACT_SILU, out.ptr, 0, 0)
+        assert rc == 0, fn
+    a, b = ref.download(np.float32), got.download(np.float32)
+    assert np.array_equal(a, b)
+    assert S.max_rel_err(a.reshape(rows, H)[:16], O.fused_moe_decode(*stacks, O.from_bf16(x[:16]), ids[:16], w[:16])) < TOL
