@@ -682,12 +682,12 @@ int forward_impl(naiwa_cached_layer* L, naiwa_cached_layer* next, int swaps_per_
         // staged pairs added on top: ring slots sort after cache slots, so the two calls
         // add the terms of one call in its order (src/moe/decode.rs:226-233 runs the
         // resident experts before the staging wait for the same reason)
-        if ((rc = naiwa_moe_decode_ex(&d.gate, &d.up, &d.down, x, NAIWA_BF16, L->slots_dev, L->wsplit_dev, rows, k,
-                                      d.act, out, 0, stream)))
+        if ((rc = naiwa_moe_decode_chain(&d.gate, &d.up, &d.down, x, L->slots_dev, L->wsplit_dev, rows, k, d.act,
+                                         out, 0, stream)))
             return rc;
         if ((rc = wait_staged())) return rc;
-        if ((rc = naiwa_moe_decode_ex(&d.gate, &d.up, &d.down, x, NAIWA_BF16, L->slots_dev, L->wsplit_dev + n, rows,
-                                      k, d.act, out, NAIWA_DECODE_ACCUMULATE, stream)))
+        if ((rc = naiwa_moe_decode_chain(&d.gate, &d.up, &d.down, x, L->slots_dev, L->wsplit_dev + n, rows, k, d.act,
+                                         out, NAIWA_DECODE_ACCUMULATE, stream)))
             return rc;
     }
     // promotion: staged -> cache slot copies, ordered after the kernel by the stream

@@ -3,7 +3,13 @@
 
 #include "../../include/naiwa_moe.h"
 
-// naiwa_moe_decode of bf16 x [rows, H] followed by x = bf16(x + y), x updated in place:
+// naiwa_moe_decode_ex of bf16 x as a layer of a whole step.  The calls of this file give the
+// same bits for the same layer; past 3 rows naiwa_moe_decode rounds less (decode_mfma.hip).
+int naiwa_moe_decode_chain(const naiwa_bank* gate, const naiwa_bank* up, const naiwa_bank* down, const void* x,
+                           const uint32_t* slot_ids, const float* w, int rows, int width, int act, float* out,
+                           int flags, int64_t stream);
+
+// naiwa_moe_decode_chain of bf16 x [rows, H] followed by x = bf16(x + y), x updated in place:
 // the residual is folded into the ordered combine when the call takes the staged paths
 // (y, f32 [rows, H], is then written only with keep_y), else it goes through y and a
 // residual launch.  The same bits either way.
@@ -26,7 +32,7 @@ struct naiwa_decode_wait {
     uint32_t* fail;
 };
 
-// naiwa_moe_decode with a folded wait (see naiwa_decode_wait).
+// naiwa_moe_decode_chain with a folded wait (see naiwa_decode_wait).
 int naiwa_moe_decode_wait(const naiwa_bank* gate, const naiwa_bank* up, const naiwa_bank* down, const void* x,
                           int x_dtype, const uint32_t* slot_ids, const float* w, int rows, int width, int act,
                           float* out, int64_t stream, const naiwa_decode_wait* wait);

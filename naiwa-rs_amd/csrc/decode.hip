@@ -757,19 +757,21 @@ __global__ void zero_f32_kernel(float* p, int64_t n) {
 
 // Calls of several rows whose formats fit run on the matrix cores, in passes over the rows
 // when one pass would need more than `cap` bytes of scratch.  Which path a call takes, and
-// its bits, depend on neither cap nor the weights.
+// its bits, depend on neither cap nor the weights.  chain: a layer of a whole step, which
+// keeps the bf16 rounding that its bits have (decode_mfma.hip) up to the pair count that
+// the rounding was used at; past it the step had f32 weights.
 struct MfmaPlan {
-    bool on;
+    bool on, bf16;
     int rows; // per pass
     size_t bytes;
 };
 constexpr size_t kMfmaScratchMax = size_t(256) << 20; // the K parts' dots of a large call stay in the caches
 MfmaPlan mfma_plan(const naiwa_bank* gate, const naiwa_bank* up, const naiwa_bank* down, const void* x, int rows,
-                   int width, size_t cap) {
+                   int width, size_t cap, bool chain) {
     const int mr = mfma_rows();
     MfmaPlan p{mr > 0 && rows >= mr && width > 0 && width <= NAIWA_MFMA_MAX_WIDTH &&
                    naiwa_decode_mfma_ok(gate, up, down, x),
-               0, 0};
+               chain && split_path(rows * width, width), 0, 0};
     if (!p.on) return p;
     const int H = gate->k, I = gate->n;
     p.rows = naiwa_decode_mfma_rows_per_pass(rows, width, H, I, split_parts(I), cap);
@@ -921,7 +923,7 @@ int decode_launch(const naiwa_bank* gate, const naiwa_bank* up, const naiwa_bank
             const void* xr = (const uint8_t*)x + o * (x_dtype == NAIWA_BF16 ? 2 : 4);
             const int rc = naiwa_decode_mfma(gate, up, down, xr, x_dtype, slot_ids + p, w + p,
                                              std::min(mfma.rows, rows - r0), width, act, out ? out + o : nullptr,
-                                             accumulate, res ? res + o : nullptr, split_ks(I), split_parts(I), ws, st);
+                                             accumulate, res ? res + o : nullptr, split_ks(I), split_parts(I), mfma.bf16, ws, st);
             if (rc) return rc;
         }
         return NAIWA_OK;
@@ -1033,19 +1035,35 @@ int noalloc_scratch(uint8_t** out) {
 
 } // namespace
 
-extern "C" int naiwa_moe_decode_ex(const naiwa_bank* gate, const naiwa_bank* up, const naiwa_bank* down,
-                                   const void* x, int x_dtype, const uint32_t* slot_ids, const float* w, int rows,
-                                   int width, int act, float* out, int flags, int64_t stream) {
+namespace {
+
+int decode_call(const naiwa_bank* gate, const naiwa_bank* up, const naiwa_bank* down, const void* x, int x_dtype,
+                const uint32_t* slot_ids, const float* w, int rows, int width, int act, float* out, int flags,
+                bool chain, int64_t stream) {
     int rc = check_args(gate, up, down, x, x_dtype, slot_ids, w, rows, width, act, out, flags);
     if (rc || rows == 0) return rc;
     uint8_t* ws = nullptr;
-    const MfmaPlan mfma = mfma_plan(gate, up, down, x, rows, width, kMfmaScratchMax);
+    const MfmaPlan mfma = mfma_plan(gate, up, down, x, rows, width, kMfmaScratchMax, chain);
     if (width > 0) {
         ws = (uint8_t*)naiwa_scratch(NAIWA_SCRATCH_DECODE, call_bytes(mfma, gate, down, rows, width), &rc);
         if (!ws) return rc;
     }
     return decode_launch(gate, up, down, x, x_dtype, slot_ids, w, rows, width, act, out, flags, mfma, ws,
                          (hipStream_t)stream);
+}
+
+} // namespace
+
+extern "C" int naiwa_moe_decode_ex(const naiwa_bank* gate, const naiwa_bank* up, const naiwa_bank* down,
+                                   const void* x, int x_dtype, const uint32_t* slot_ids, const float* w, int rows,
+                                   int width, int act, float* out, int flags, int64_t stream) {
+    return decode_call(gate, up, down, x, x_dtype, slot_ids, w, rows, width, act, out, flags, false, stream);
+}
+
+int naiwa_moe_decode_chain(const naiwa_bank* gate, const naiwa_bank* up, const naiwa_bank* down, const void* x,
+                           const uint32_t* slot_ids, const float* w, int rows, int width, int act, float* out,
+                           int flags, int64_t stream) {
+    return decode_call(gate, up, down, x, NAIWA_BF16, slot_ids, w, rows, width, act, out, flags, true, stream);
 }
 
 extern "C" int naiwa_moe_decode_noalloc(const naiwa_bank* gate, const naiwa_bank* up, const naiwa_bank* down,
@@ -1057,7 +1075,7 @@ extern "C" int naiwa_moe_decode_noalloc(const naiwa_bank* gate, const naiwa_bank
         return NAIWA_E_TOO_LARGE;
     // on the matrix cores in passes that fit: an accepted call has at least 4 rows there, so
     // one row takes little more than a quarter of the array
-    const MfmaPlan mfma = mfma_plan(gate, up, down, x, rows, width, kNoAllocScratchBytes);
+    const MfmaPlan mfma = mfma_plan(gate, up, down, x, rows, width, kNoAllocScratchBytes, false);
     if (mfma.on && mfma.bytes > kNoAllocScratchBytes) return NAIWA_E_TOO_LARGE;
     uint8_t* ws = nullptr;
     if ((rc = noalloc_scratch(&ws))) return rc;
@@ -1078,7 +1096,7 @@ int naiwa_moe_decode_residual(const naiwa_bank* gate, const naiwa_bank* up, cons
     int rc = check_args(gate, up, down, x, NAIWA_BF16, slot_ids, w, rows, width, act, y, 0);
     if (rc || rows == 0 || width == 0) return rc;
     if (wait && (!wait->flag || !wait->fail)) return NAIWA_E_INVALID;
-    const MfmaPlan mfma = mfma_plan(gate, up, down, x, rows, width, kMfmaScratchMax);
+    const MfmaPlan mfma = mfma_plan(gate, up, down, x, rows, width, kMfmaScratchMax, true);
     uint8_t* ws = (uint8_t*)naiwa_scratch(NAIWA_SCRATCH_DECODE, call_bytes(mfma, gate, down, rows, width), &rc);
     if (!ws) return rc;
     if (mfma.on || split_path(rows * width, width))
@@ -1097,7 +1115,7 @@ int naiwa_moe_decode_wait(const naiwa_bank* gate, const naiwa_bank* up, const na
     if (rc || rows == 0) return rc;
     if (wait && (!wait->flag || !wait->fail)) return NAIWA_E_INVALID;
     uint8_t* ws = nullptr;
-    const MfmaPlan mfma = mfma_plan(gate, up, down, x, rows, width, kMfmaScratchMax);
+    const MfmaPlan mfma = mfma_plan(gate, up, down, x, rows, width, kMfmaScratchMax, true);
     if (width > 0) {
         ws = (uint8_t*)naiwa_scratch(NAIWA_SCRATCH_DECODE, call_bytes(mfma, gate, down, rows, width), &rc);
         if (!ws) return rc;

@@ -26,6 +26,8 @@ int naiwa_decode_mfma_rows_per_pass(int rows, int width, int H, int I, int kpart
 // One pass over scratch ws (NaiwaMfmaLayout(rows, ...).total bytes): out = (accumulate ? out
 // : 0) + the weighted experts, and with res (bf16 [rows, H]) x = bf16(x + out) in place
 // (out may then be null).  K parts of ks values of I, kparts of them.
+// bf16: x, h and the weights are rounded to bf16 (a layer of a chain), otherwise the weights
+// are exact.
 int naiwa_decode_mfma(const naiwa_bank* gate, const naiwa_bank* up, const naiwa_bank* down, const void* x, int x_dtype,
                       const uint32_t* slot_ids, const float* w, int rows, int width, int act, float* out,
-                      int accumulate, uint16_t* res, int ks, int kparts, uint8_t* ws, hipStream_t st);
+                      int accumulate, uint16_t* res, int ks, int kparts, bool bf16, uint8_t* ws, hipStream_t st);

@@ -35,6 +35,11 @@
 //   h: one scale per (pair, 64 features), the block's own strip, stored beside it;
 //      the down kernel brings a row's strips to one scale as it reads the A operand.
 //
+// Rounded operands (BF).  The layers of a chain route on activations that the layers before
+// them rounded, so any change of rounding flips an expert near the cut of a top-k somewhere
+// and with it all that follows: whole steps (the layered stack, the partial cache) keep x, h
+// and the dequantised weights in bf16, and with them their results bit for bit.
+//
 // K order: group G = 4 s + g of 8 f16 is lane group g's A operand at step s.
 //   Q4_K (256 values): lane group g takes 64-value chunk g; step s = 2 p + t its
 //        quant bytes 8 p + 0..7, low nibbles for t = 0 and high ones for t = 1:
@@ -44,17 +49,16 @@
 #include "decode_mfma.h"
 #include "common.h"
 #include "segments.h"
+#include "unpack_bf16.h"
 
 #include <algorithm>
 
 namespace {
 
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef _Float16 half4v __attribute__((ext_vector_type(4)));
 typedef _Float16 half8v __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kThreads = 256; // 4 waves of 16 weight rows (per matrix)
 constexpr int kF = 64;        // weight rows per block and matrix
@@ -73,9 +77,6 @@ template <> struct KB<NAIWA_Q4_K> {
 template <> struct KB<NAIWA_Q8_0> {
     static constexpr int kVals = 128, kSteps = 4, kGroups = 16, kBytes = 4 * NAIWA_Q8_0_BYTES;
 };
-
-// Element i of a laid-out Q4_K run of 8 values holds value q4_elem(i) of the run (an involution).
-__host__ __device__ constexpr int q4_elem(int i) { return (i == 1 || i == 2 || i == 5 || i == 6) ? (i ^ 3) : i; }
 
 // The group that holds run r (values 8 r .. 8 r + 7) of a K-block.
 template <int DT>
@@ -107,6 +108,15 @@ __device__ __forceinline__ half8v pack_run(const float (&f)[8], float scale, flo
     return o;
 }
 
+// The same in bf16, unscaled.
+template <int DT>
+__device__ __forceinline__ half8v pack_run_bf16(const float (&f)[8]) {
+    float o[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) o[i] = f[DT == NAIWA_Q4_K ? q4_elem(i) : i];
+    return __builtin_bit_cast(half8v, to_bf16x8(o));
+}
+
 // Slot of sub-block sum j (0..7) of a K-block: f16 halves hi [0..7] and lo [8..15].
 __device__ __forceinline__ void put_sum(_Float16* s16, int j, float sum) {
     const _Float16 hi = (_Float16)sum;
@@ -121,7 +131,7 @@ __device__ __forceinline__ void put_sum(_Float16* s16, int j, float sum) {
 // f16 groups xa [rows][H], sub-block sums xs [rows][H / 256][16] (Q4_K) and the
 // row's inverse scale xr [rows].  The two parts share nothing, and a launch of its
 // own costs each about 4.5 us of a 60 us call.
-template <int DT>
+template <int DT, bool BF>
 __global__ void __launch_bounds__(kThreads)
 seg_prep_kernel(const uint32_t* slot_ids, const float* w, int n, int width, int nslots, uint32_t* tok, uint32_t* inv,
                 int* seg_count, uint32_t* seg_key, uint32_t* seg_begin, int* bad, const void* x, int x_bf16, int H,
@@ -151,6 +161,16 @@ seg_prep_kernel(const uint32_t* slot_ids, const float* w, int n, int width, int 
             }
         }
     };
+    constexpr int R = KB<DT>::kVals / 8;
+    if constexpr (BF) {
+        for (int run = tid; run < runs; run += kThreads) {
+            float f[8];
+            run_of(run, f);
+            *reinterpret_cast<half8v*>(xa + (size_t)t * H + run / R * KB<DT>::kVals + 8 * group_of_run<DT>(run % R)) =
+                pack_run_bf16<DT>(f);
+        }
+        return;
+    }
     float mx = 0.0f;
     for (int run = tid; run < runs; run += kThreads) {
         float f[8];
@@ -174,7 +194,6 @@ seg_prep_kernel(const uint32_t* slot_ids, const float* w, int n, int width, int 
         float f[8] = {}, sum;
         if (in) run_of(run, f);
         const half8v o = pack_run<DT>(f, sc, sum);
-        constexpr int R = KB<DT>::kVals / 8;
         const int kb = run / R, r = run % R;
         if (in) *reinterpret_cast<half8v*>(xa + (size_t)t * H + kb * KB<DT>::kVals + 8 * group_of_run<DT>(r)) = o;
         if (DT == NAIWA_Q4_K) {
@@ -216,9 +235,9 @@ __device__ __forceinline__ void lds_barrier() {
 // each instruction's rows start 16 kRpd bytes further on, so the 16 rows' pieces of one
 // group fall on distinct banks while a step's read keeps a fixed offset from the lane's
 // own base: (m / kRpd) kStride + (m % kRpd) 16 kGroups + 16 (g ^ m % kRpd) + 64 s.
-template <int DT, int MR> struct ATile {
+template <int DT, int MR, bool BF> struct ATile {
     static constexpr int G = KB<DT>::kGroups, kRpd = 64 / G, kDma = MR / kRpd, kStride = 1024 + 16 * kRpd;
-    static constexpr bool kSums = DT == NAIWA_Q4_K;
+    static constexpr bool kSums = DT == NAIWA_Q4_K && !BF;
     __align__(16) uint8_t v[kDma * kStride];
     __align__(16) _Float16 sums[kSums ? MR * 16 : 8]; // [row][hi 0..7 | lo 0..7]
 };
@@ -233,15 +252,6 @@ template <int DT, int NP> struct WTile {
 };
 
 // The lane's unpacking of its weight row's K-block, from LDS into B operands and scales.
-struct NibMask {
-    uint32_t lo, hi;
-};
-__device__ __forceinline__ NibMask nib_mask() {
-    NibMask n{0x000F000Fu, 0x00F000F0u};
-    asm("" : "+v"(n.lo)); // masks in VGPRs: (w & mask) | magic is then one v_and_or_b32
-    asm("" : "+v"(n.hi));
-    return n;
-}
 __device__ __forceinline__ half2v h2(uint32_t v) { return __builtin_bit_cast(half2v, v); }
 __device__ __forceinline__ half2v splat(_Float16 v) { return half2v{v, v}; }
 
@@ -294,10 +304,11 @@ template <int NP> struct WRegs<NAIWA_Q8_0, NP> {
 
 // One K-block of a wave: acc[q][mt] += rows q of the weights times the A tile's subtiles.
 // fac (h only): the row's per-chunk f16 factors from this K-block's chunk on.
-template <int DT, int NP, int MT, int MR, bool HF>
-__device__ __forceinline__ void kblock(const WRegs<DT, NP>& wr, const ATile<DT, MR>& at, const uint16_t* fac, int fst,
-                                       int g, int m, const NibMask& nm, floatx4 (&acc)[NP][MT]) {
-    using A = ATile<DT, MR>;
+// BF: activations and dequantised weights rounded to bf16, accumulated over the K-blocks.
+template <int DT, int NP, int MT, int MR, bool HF, bool BF>
+__device__ __forceinline__ void kblock(const WRegs<DT, NP>& wr, const ATile<DT, MR, BF>& at, const uint16_t* fac,
+                                       int fst, int g, int m, const NibMask& nm, floatx4 (&acc)[NP][MT]) {
+    using A = ATile<DT, MR, BF>;
     auto arow = [&](int mt) { return MR < 16 ? (m & (MR - 1)) : 16 * mt + m; };
     const uint8_t* abase[MT];
 #pragma unroll
@@ -308,7 +319,34 @@ __device__ __forceinline__ void kblock(const WRegs<DT, NP>& wr, const ATile<DT, 
     auto ld_a = [&](int mt, int s) {
         return __builtin_bit_cast(half8v, *reinterpret_cast<const u32x4*>(abase[mt] + 64 * s));
     };
-    if constexpr (DT == NAIWA_Q4_K) {
+    if constexpr (BF) {
+        float sc[NP][2], mn[NP][2];
+        if constexpr (DT == NAIWA_Q4_K)
+#pragma unroll
+            for (int q = 0; q < NP; ++q)
+#pragma unroll
+                for (int t = 0; t < 2; ++t) q4k_scale_min(wr.hd[q], 2 * g + t, sc[q][t], mn[q][t]);
+#pragma unroll
+        for (int s = 0; s < KB<DT>::kSteps; ++s) {
+            bf16x8 a8[MT];
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) a8[mt] = __builtin_bit_cast(bf16x8, ld_a(mt, s));
+#pragma unroll
+            for (int q = 0; q < NP; ++q) {
+                bf16x8 b8;
+                if constexpr (DT == NAIWA_Q4_K) {
+                    const int p = s >> 1, t = s & 1;
+                    const u32x4& qv = p < 2 ? wr.q0[q] : wr.q1[q];
+                    b8 = q4k_unpack((p & 1) ? qv.z : qv.x, (p & 1) ? qv.w : qv.y, t, nm, sc[q][t], mn[q][t]);
+                } else {
+                    b8 = q8_unpack(wr.code(q, s, 0), wr.code(q, s, 1), wr.d(q, s));
+                }
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+                    acc[q][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a8[mt], b8, acc[q][mt], 0, 0, 0);
+            }
+        }
+    } else if constexpr (DT == NAIWA_Q4_K) {
         half2v sc[NP];
         half4v m6[NP];
         float d[NP], dmin[NP];
@@ -362,7 +400,7 @@ __device__ __forceinline__ void kblock(const WRegs<DT, NP>& wr, const ATile<DT, 
                 const u32x4& qv = p < 2 ? wr.q0[q] : wr.q1[q];
                 const uint32_t w[2] = {(p & 1) ? qv.z : qv.x, (p & 1) ? qv.w : qv.y};
                 // (magic + nibble) * sc - magic * sc = sc * nibble, exact in one f16 fma
-                const uint32_t mk = t ? nm.hi : nm.lo, magic = t ? 0x54005400u : 0x64006400u;
+                const uint32_t mk = nm.m[t], magic = t ? 0x54005400u : 0x64006400u;
                 const half2v s2 = splat(sc[q][t]), o2 = s2 * splat((_Float16)(t ? -64.0f : -1024.0f));
                 u32x4 b;
 #pragma unroll
@@ -429,9 +467,9 @@ __device__ __forceinline__ void kblock(const WRegs<DT, NP>& wr, const ATile<DT, 
 // LDS of one block: a weight stage per wave and two A tiles.  More weight stages cost
 // blocks: with 2 the 8- and 96-row calls at H 2048, I 768 took 63 and 131 us against 61
 // and 120, and 16 and 64 rows at H 4096, I 14336 the same 188 and 227.
-template <int DT, int NP, int MR> struct Smem {
+template <int DT, int NP, int MR, bool BF> struct Smem {
     WTile<DT, NP> w[kThreads / 64];
-    ATile<DT, MR> a[2];
+    ATile<DT, MR, BF> a[2];
 };
 
 // A value every lane of the wave reads, through the scalar cache (its own counter, so it
@@ -446,12 +484,12 @@ __device__ __forceinline__ uint32_t scalar_ld(const uint32_t* p) {
 // vmcnt), the barrier makes every wave's part of the A tile visible and frees the other A
 // buffer, the next A copies go out, the lanes take their weight words, the next K-block's
 // copies go out into the freed stage, and the K-block is computed.
-template <int DT, int NP, int MT, int MR> struct KLoop {
-    using A = ATile<DT, MR>;
+template <int DT, int NP, int MT, int MR, bool BF> struct KLoop {
+    using A = ATile<DT, MR, BF>;
     using W = WTile<DT, NP>;
     static constexpr int PB = W::k16 ? 16 : 4, kPer = KB<DT>::kBytes / PB; // pieces per row
     static constexpr int kAd = (A::kDma + 3) / 4; // A copies of a wave: instructions wave, wave + 4, ...
-    Smem<DT, NP, MR>& sm;
+    Smem<DT, NP, MR, BF>& sm;
     const uint8_t *abase, *sums;
     const uint8_t* wrow[NP];
     int kb0, nkb, lane, wave;
@@ -520,7 +558,7 @@ template <int DT, int NP, int MT, int MR> struct KLoop {
             wr.load(sm.w[wave], g, m);
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // held in registers: the stage is free
             issue_w(kb0 + jn);
-            kblock<DT, NP, MT, MR, HF>(wr, sm.a[j & 1], HF ? &fac[0][j * (KB<DT>::kVals / kChunk)] : nullptr, NFAC, g, m,
+            kblock<DT, NP, MT, MR, HF, BF>(wr, sm.a[j & 1], HF ? &fac[0][j * (KB<DT>::kVals / kChunk)] : nullptr, NFAC, g, m,
                                        nm, acc);
         }
         // the last K-block's copies went out once more: they land before the LDS is used for
@@ -532,13 +570,13 @@ template <int DT, int NP, int MT, int MR> struct KLoop {
 
 // gate/up: block (64 features, slot segment); h = act(gate) * up of the pair at its sorted
 // position, f16 in the K order of DD with a scale per (pair, 64 features).
-template <int DG, int DD, int MT, int MR>
+template <int DG, int DD, int MT, int MR, bool BF>
 __global__ void __launch_bounds__(kThreads, 2)
 gateup_mfma_kernel(Bank gate, Bank up, const _Float16* xa, const _Float16* xs, const float* xr, int H, int I,
                    const int* seg_count, const uint32_t* seg_key, const uint32_t* seg_begin, const uint32_t* tok,
                    int act, _Float16* ha, _Float16* hs, int8_t* he) {
     constexpr int kHt = kF + 4; // floats per row of the h exchange
-    __shared__ Smem<DG, 2, MR> sm;
+    __shared__ Smem<DG, 2, MR, BF> sm;
     static_assert(sizeof(float) * MR * kHt <= sizeof(sm), "the h exchange reuses the tiles");
     const int sg = blockIdx.y;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -551,7 +589,7 @@ gateup_mfma_kernel(Bank gate, Bank up, const _Float16* xa, const _Float16* xs, c
     if (sg >= segs) return;
     const int n0 = blockIdx.x * kF;
     const int64_t r0 = n0 + 16 * wave;
-    KLoop<DG, 2, MT, MR> kl{sm, (const uint8_t*)xa, (const uint8_t*)xs,
+    KLoop<DG, 2, MT, MR, BF> kl{sm, (const uint8_t*)xa, (const uint8_t*)xs,
                                  {gate.base + (int64_t)slot * gate.stride + r0 * gate.row_bytes,
                                   up.base + (int64_t)slot * up.stride + r0 * up.row_bytes},
                                  0, H / KB<DG>::kVals, lane, wave};
@@ -564,7 +602,7 @@ gateup_mfma_kernel(Bank gate, Bank up, const _Float16* xa, const _Float16* xs, c
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) rs[mt][i] = xr[tok[c0 + min(16 * mt + 4 * g + i, cnt - 1)]];
+            for (int i = 0; i < 4; ++i) rs[mt][i] = BF ? 1.0f : xr[tok[c0 + min(16 * mt + 4 * g + i, cnt - 1)]];
         floatx4 acc[2][MT] = {};
         kl.template run<false, 2>(nullptr, acc);
         float* ht = reinterpret_cast<float*>(&sm);
@@ -583,19 +621,24 @@ gateup_mfma_kernel(Bank gate, Bank up, const _Float16* xa, const _Float16* xs, c
         for (int u0 = 0; u0 < MR * 8; u0 += kThreads) {
             const int u = u0 + tid, mm = u >> 3, run = u & 7;
             if (MR * 8 < kThreads && u >= MR * 8) break;
+            constexpr int KV = KB<DD>::kVals;
+            const int kb = n0 / KV, r = (n0 % KV) / 8 + run;
+            const size_t pos = c0 + mm;
             float f[8], mx = 0.0f, sum;
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 f[j] = ht[mm * kHt + 8 * run + j];
                 mx = fmaxf(mx, fabsf(f[j]));
             }
+            if constexpr (BF) {
+                if (mm < cnt)
+                    *reinterpret_cast<half8v*>(ha + pos * I + kb * KV + 8 * group_of_run<DD>(r)) = pack_run_bf16<DD>(f);
+                continue;
+            }
 #pragma unroll
             for (int k = 1; k < 8; k <<= 1) mx = fmaxf(mx, __shfl_xor(mx, k, 64));
             const int ex = scale_exp(mx);
             const half8v o = pack_run<DD>(f, pow2f(ex), sum);
-            constexpr int KV = KB<DD>::kVals;
-            const int kb = n0 / KV, r = (n0 % KV) / 8 + run;
-            const size_t pos = c0 + mm;
             if (DD == NAIWA_Q4_K) {
                 sum += __shfl_xor(sum, 1, 64);
                 sum += __shfl_xor(sum, 2, 64);
@@ -612,15 +655,15 @@ gateup_mfma_kernel(Bank gate, Bank up, const _Float16* xa, const _Float16* xs, c
 
 // down: block (128 rows, K part, slot segment); the unweighted partial dot of (K part,
 // sorted position, row) into dpart.
-template <int DD, int MT, int MR>
+template <int DD, int MT, int MR, bool BF>
 __global__ void __launch_bounds__(kThreads, 2)
 down_mfma_kernel(Bank down, const _Float16* ha, const _Float16* hs, const int8_t* he, int H, int I, int ks, int npairs,
                  const int* seg_count, const uint32_t* seg_key, const uint32_t* seg_begin, float* dpart) {
     constexpr int NP = 2;    // two strips of 64 rows: H is a multiple of 128 in every served format
     constexpr int kFac = 34; // K parts of at most 2048: 32 chunks, rows an odd number of words apart
-    __shared__ Smem<DD, NP, MR> sm;
-    __shared__ uint16_t fac[MR][kFac];
-    __shared__ float rs[MR];
+    __shared__ Smem<DD, NP, MR, BF> sm;
+    __shared__ uint16_t fac[BF ? 1 : MR][kFac];
+    __shared__ float rs[BF ? 1 : MR];
     const int sg = blockIdx.z;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 4, m = lane & 15;
@@ -631,7 +674,7 @@ down_mfma_kernel(Bank down, const _Float16* ha, const _Float16* hs, const int8_t
     if (sg >= segs) return;
     const int kp = blockIdx.y, k0 = kp * ks, kn = min(ks, I - k0);
     const int64_t r0 = (int64_t)blockIdx.x * (NP * kF) + 16 * wave; // matrix q: rows r0 + 64 q
-    KLoop<DD, NP, MT, MR> kl{sm, (const uint8_t*)ha, (const uint8_t*)hs, {}, k0 / KB<DD>::kVals,
+    KLoop<DD, NP, MT, MR, BF> kl{sm, (const uint8_t*)ha, (const uint8_t*)hs, {}, k0 / KB<DD>::kVals,
                                   kn / KB<DD>::kVals, lane, wave};
 #pragma unroll
     for (int q = 0; q < NP; ++q)
@@ -641,6 +684,7 @@ down_mfma_kernel(Bank down, const _Float16* ha, const _Float16* hs, const int8_t
         kl.start(down.row_bytes, (uint32_t)I * 2, (uint32_t)(I / 256) * 32,
                  [&](int r) { return (uint32_t)(c0 + min(r, cnt - 1)); });
         // each row's scales over the K part to the smallest one of them: 32 lanes a row
+        if constexpr (!BF)
 #pragma unroll
         for (int i = 0; i < MR; i += kThreads / 32) {
             const int r = i + (tid >> 5), c = tid & 31;
@@ -653,7 +697,7 @@ down_mfma_kernel(Bank down, const _Float16* ha, const _Float16* hs, const int8_t
             if (c == 0) rs[r] = pow2f(-lo);
         }
         floatx4 acc[NP][MT] = {};
-        kl.template run<true, kFac>(fac, acc);
+        kl.template run<!BF, kFac>(fac, acc);
 #pragma unroll
         for (int q = 0; q < NP; ++q)
 #pragma unroll
@@ -661,7 +705,8 @@ down_mfma_kernel(Bank down, const _Float16* ha, const _Float16* hs, const int8_t
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const int mm = 16 * mt + 4 * g + i;
-                    if (mm < cnt) dpart[((size_t)kp * npairs + c0 + mm) * H + r0 + kF * q + m] = acc[q][mt][i] * rs[mm];
+                    if (mm < cnt) dpart[((size_t)kp * npairs + c0 + mm) * H + r0 + kF * q + m] =
+                            BF ? acc[q][mt][i] : acc[q][mt][i] * rs[mm];
                 }
         __syncthreads(); // the scales are free for the next chunk
     }
@@ -758,25 +803,33 @@ struct Call {
     hipStream_t st;
 };
 
-template <int DG, int DD, int MT, int MR>
+template <int DG, int DD, int MT, int MR, bool BF>
 void experts(const Call& c) {
-    gateup_mfma_kernel<DG, DD, MT, MR><<<dim3(c.I / kF, c.segs), kThreads, 0, c.st>>>(
+    gateup_mfma_kernel<DG, DD, MT, MR, BF><<<dim3(c.I / kF, c.segs), kThreads, 0, c.st>>>(
         c.g, c.u, c.xa, c.xs, c.xr, c.H, c.I, c.seg_count, c.seg_key, c.seg_begin, c.tok, c.act, c.ha, c.hs, c.he);
-    down_mfma_kernel<DD, MT, MR><<<dim3(c.H / (2 * kF), c.kparts, c.segs), kThreads, 0, c.st>>>(
+    down_mfma_kernel<DD, MT, MR, BF><<<dim3(c.H / (2 * kF), c.kparts, c.segs), kThreads, 0, c.st>>>(
         c.d, c.ha, c.hs, c.he, c.H, c.I, c.ks, c.n, c.seg_count, c.seg_key, c.seg_begin, c.dpart);
 }
 
 // Token rows of the A tile.  8: a segment of a call of at most 8 rows holds no more (unless
 // a token repeats a slot), and the smaller tile lets a fifth block fit on a CU.  32 when
 // segments average more than 8 tokens: a weight is then unpacked once per 32 tokens.
-template <int DG, int DD>
+template <int DG, int DD, bool BF>
 void experts_rows(const Call& c) {
     if (c.rows <= 8)
-        experts<DG, DD, 1, 8>(c);
+        experts<DG, DD, 1, 8, BF>(c);
     else if (c.n > 8 * c.segs)
-        experts<DG, DD, 2, 32>(c);
+        experts<DG, DD, 2, 32, BF>(c);
     else
-        experts<DG, DD, 1, 16>(c);
+        experts<DG, DD, 1, 16, BF>(c);
+}
+
+template <int DG, int DD>
+void experts_rounding(const Call& c, bool bf) {
+    if (bf)
+        experts_rows<DG, DD, true>(c);
+    else
+        experts_rows<DG, DD, false>(c);
 }
 
 bool fmt_ok(int dt, int k) {
@@ -825,7 +878,7 @@ int naiwa_decode_mfma_rows_per_pass(int rows, int width, int H, int I, int kpart
 
 int naiwa_decode_mfma(const naiwa_bank* gate, const naiwa_bank* up, const naiwa_bank* down, const void* x, int x_dtype,
                       const uint32_t* slot_ids, const float* w, int rows, int width, int act, float* out,
-                      int accumulate, uint16_t* res, int ks, int kparts, uint8_t* ws, hipStream_t st) {
+                      int accumulate, uint16_t* res, int ks, int kparts, bool bf16, uint8_t* ws, hipStream_t st) {
     const int H = gate->k, I = gate->n, n = rows * width;
     const NaiwaMfmaLayout L(rows, width, H, I, kparts);
     Call c;
@@ -844,22 +897,18 @@ int naiwa_decode_mfma(const naiwa_bank* gate, const naiwa_bank* up, const naiwa_
     c.dpart = (float*)(ws + L.off_dpart);
     const int xb = x_dtype == NAIWA_BF16;
     const bool g4 = gate->dtype == NAIWA_Q4_K, d4 = down->dtype == NAIWA_Q4_K;
-    if (g4)
-        seg_prep_kernel<NAIWA_Q4_K><<<rows + 1, kThreads, 0, st>>>(slot_ids, w, n, width, gate->slots, c.tok, inv, c.seg_count,
-                                                                   c.seg_key, c.seg_begin, (int*)(ws + 4), x, xb, H,
-                                                                   c.xa, c.xs, c.xr);
-    else
-        seg_prep_kernel<NAIWA_Q8_0><<<rows + 1, kThreads, 0, st>>>(slot_ids, w, n, width, gate->slots, c.tok, inv, c.seg_count,
-                                                                   c.seg_key, c.seg_begin, (int*)(ws + 4), x, xb, H,
-                                                                   c.xa, c.xs, c.xr);
+    auto* prep = g4 ? (bf16 ? seg_prep_kernel<NAIWA_Q4_K, true> : seg_prep_kernel<NAIWA_Q4_K, false>)
+                    : (bf16 ? seg_prep_kernel<NAIWA_Q8_0, true> : seg_prep_kernel<NAIWA_Q8_0, false>);
+    prep<<<rows + 1, kThreads, 0, st>>>(slot_ids, w, n, width, gate->slots, c.tok, inv, c.seg_count, c.seg_key,
+                                        c.seg_begin, (int*)(ws + 4), x, xb, H, c.xa, c.xs, c.xr);
     if (g4 && d4)
-        experts_rows<NAIWA_Q4_K, NAIWA_Q4_K>(c);
+        experts_rounding<NAIWA_Q4_K, NAIWA_Q4_K>(c, bf16);
     else if (g4)
-        experts_rows<NAIWA_Q4_K, NAIWA_Q8_0>(c);
+        experts_rounding<NAIWA_Q4_K, NAIWA_Q8_0>(c, bf16);
     else if (d4)
-        experts_rows<NAIWA_Q8_0, NAIWA_Q4_K>(c);
+        experts_rounding<NAIWA_Q8_0, NAIWA_Q4_K>(c, bf16);
     else
-        experts_rows<NAIWA_Q8_0, NAIWA_Q8_0>(c);
+        experts_rounding<NAIWA_Q8_0, NAIWA_Q8_0>(c, bf16);
     combine_mfma_kernel<<<dim3((H + 255) / 256, rows), 64, 0, st>>>(c.dpart, kparts, n, H, width, inv, w, accumulate, out,
                                                                     res);
     return naiwa_hip_rc(hipGetLastError());

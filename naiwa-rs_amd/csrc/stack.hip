@@ -2,7 +2,7 @@
 // x <- bf16(x + MoE_l(x)), with routing kept on the device.
 //
 // NAIWA_STACK_LAYERED chains the standalone entry points (router top-k,
-// slot lookup, naiwa_moe_decode, residual) per layer.
+// slot lookup, the decode of one layer, residual) per layer.
 #include "decode.h"
 #include "router.h"
 #include "rowdot.h"
@@ -88,8 +88,7 @@ extern "C" int naiwa_stack_decode_y(const naiwa_layer* layers, int n_layers, voi
                 return rc;
             continue;
         }
-        if ((rc = naiwa_moe_decode(&L.gate, &L.up, &L.down, x, NAIWA_BF16, dec_ids, dec_w, rows, k, act, y,
-                                   stream)))
+        if ((rc = naiwa_moe_decode_chain(&L.gate, &L.up, &L.down, x, dec_ids, dec_w, rows, k, act, y, 0, stream)))
             return rc;
         if ((rc = naiwa_hip_rc(hipMemcpyAsync(y_out + (size_t)l * rows * H, y, (size_t)rows * H * 4,
                                               hipMemcpyDeviceToDevice, st))))

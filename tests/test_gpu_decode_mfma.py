@@ -95,3 +95,35 @@ def test_noalloc_passes_give_the_bits_of_one_pass(gpu):
     a, b = ref.download(np.float32), got.download(np.float32)
     assert np.array_equal(a, b)
     assert S.max_rel_err(a.reshape(rows, H)[:16], O.fused_moe_decode(*stacks, O.from_bf16(x[:16]), ids[:16], w[:16])) < TOL
+
+
+@pytest.mark.parametrize("dt,H,I,E,k,rows", [
+    ((Q4, Q4, Q4), 256, 256, 8, 2, 5),       # 8-row tile
+    ((Q4, Q4, Q8), 512, 384, 16, 3, 11),     # 16-row tile
+    ((Q8, Q8, Q4), 256, 2304, 4, 2, 35),     # two K parts; chunks of 32 rows and past them
+    ((Q8, Q8, Q8), 384, 128, 8, 4, 17),
+])
+def test_chain_rounding_at_tile_edges(gpu, dt, H, I, E, k, rows):
+    """A layer of a layered step rounds x, h and the weights to bf16: within 1e-2 of the oracle,
+    and the residual in the combine gives the bits of a residual launch."""
+    nm = gpu
+    banks, stacks, keep = _layer(nm, 8500 + rows, E, H, I, dt)
+    router = S.layer(8500 + rows, E, H, I, dt)[3]
+    rd = nm.DeviceBuffer.from_array(router)
+    desc = (nm._lib.Layer * 1)(nm.layer_desc(rd, banks))
+    x = S.activations_bf16(8501 + rows, rows, H)
+    print(f"[chain {dt} H={H} I={I} E={E} k={k} rows={rows}]", flush=True)
+    got = []
+    for want_y in (True, False):
+        xd, y = nm.DeviceBuffer.from_array(x), nm.DeviceBuffer(rows * H * 4)
+        nm.stack_decode(desc, xd, rows, H, E, k, mode=O.ROUTE_SOFTMAX_TOPK_RENORM, fused=False,
+                        y_out=y if want_y else None)
+        nm.synchronize()
+        got.append(xd.download(np.uint16))
+        if want_y:
+            ids, w = O.topk(O.router_logits(O.from_bf16(x), router), k, O.ROUTE_SOFTMAX_TOPK_RENORM)
+            err = S.max_rel_err(y.download(np.float32).reshape(rows, H),
+                                O.fused_moe_decode(*stacks, O.from_bf16(x), ids, w))
+            print(f"  max_rel_err={err:.3e}", flush=True)
+            assert err < 1e-2
+    assert np.array_equal(got[0], got[1])
