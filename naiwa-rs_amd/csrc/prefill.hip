@@ -3,7 +3,8 @@
 // MoEExperts::forward called from src/prefill_stream.rs:2080-2102.
 //
 //   1. gather:   (token, k) pairs sorted by slot (stable), offsets per slot;
-//   2. tiles:    the sorted pairs cut into tiles of 64 pairs of one slot;
+//   2. tiles:    the sorted pairs cut into tiles of up to 64 or 128 pairs of one
+//                slot;
 //   3. prep:     x (bf16) laid out once in the K order of the gate/up weight
 //                format (below);
 //   4. gate/up:  per (tile, 128 intermediate features): 64 x rows times the
@@ -40,6 +41,8 @@
 #include "unpack_bf16.h"
 #include "workspace.h"
 
+#include <algorithm>
+
 namespace {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
@@ -52,10 +55,10 @@ constexpr int kTND = 256;      // down output features per block
 
 template <int DT> struct KBlock;
 template <> struct KBlock<NAIWA_Q4_K> {
-    static constexpr int kVals = 256, kSteps = 16;
+    static constexpr int kVals = 256, kSteps = 16, kBytes = NAIWA_Q4_K_BYTES;
 };
 template <> struct KBlock<NAIWA_Q8_0> {
-    static constexpr int kVals = 128, kSteps = 8;
+    static constexpr int kVals = 128, kSteps = 8, kBytes = 4 * NAIWA_Q8_0_BYTES;
 };
 
 // The group (2s + h) that holds run r of a K-block.
@@ -81,7 +84,7 @@ __host__ __device__ inline int laid_pos(int f) {
 
 struct Tiles {
     int* start; // first sorted position of the tile
-    int* count; // pairs in the tile (<= kTM)
+    int* count; // pairs in the tile (<= the tile size)
     int* slot;  // the tile's slot
     int* n;     // number of tiles
 };
@@ -109,14 +112,14 @@ __device__ __forceinline__ bool tile_col(int b, int ntiles, int ncol, int xcd, i
     return true;
 }
 
-// Cut the sorted pairs into tiles of <= kTM pairs of one slot.  One block.
-__device__ inline void tiles_block(const uint32_t* offsets, int slots, Tiles t) {
+// Cut the sorted pairs into tiles of <= tm pairs of one slot.  One block.
+__device__ inline void tiles_block(const uint32_t* offsets, int slots, int tm, Tiles t) {
     __shared__ int part[kThreads + 1];
     const int tid = threadIdx.x;
     const int per = (slots + kThreads - 1) / kThreads;
     const int s0 = min(slots, tid * per), s1 = min(slots, s0 + per);
     int mine = 0;
-    for (int s = s0; s < s1; ++s) mine += (int)((offsets[s + 1] - offsets[s] + kTM - 1) / kTM);
+    for (int s = s0; s < s1; ++s) mine += (int)((offsets[s + 1] - offsets[s] + tm - 1) / tm);
     part[tid] = mine;
     __syncthreads();
     if (tid == 0) {
@@ -133,9 +136,12 @@ __device__ inline void tiles_block(const uint32_t* offsets, int slots, Tiles t) 
     int at = part[tid];
     for (int s = s0; s < s1; ++s) {
         const int b = (int)offsets[s], n = (int)(offsets[s + 1] - offsets[s]);
-        for (int m = 0; m < n; m += kTM, ++at) {
-            t.start[at] = b + m;
-            t.count[at] = min(kTM, n - m);
+        // the fewest tiles, of about equal numbers of 32-row subtiles
+        const int subs = (n + 31) / 32, nt = (n + tm - 1) / tm;
+        for (int j = 0; j < nt; ++j, ++at) {
+            const int m0 = 32 * (subs * j / nt), m1 = min(n, 32 * (subs * (j + 1) / nt));
+            t.start[at] = b + m0;
+            t.count[at] = m1 - m0;
             t.slot[at] = s;
         }
     }
@@ -173,9 +179,9 @@ __device__ inline void prep_block(const uint16_t* x, int T, int H, uint16_t* xp,
 // in one launch: the two do not depend on each other.
 template <int DT>
 __global__ void __launch_bounds__(kThreads) prep_tiles_kernel(const uint16_t* x, int T, int H, uint16_t* xp,
-                                                              const uint32_t* offsets, int slots, Tiles t) {
+                                                              const uint32_t* offsets, int slots, int tm, Tiles t) {
     if (blockIdx.x == gridDim.x - 1)
-        tiles_block(offsets, slots, t);
+        tiles_block(offsets, slots, tm, t);
     else
         prep_block<DT>(x, T, H, xp, blockIdx.x);
 }
@@ -455,6 +461,12 @@ down_kernel(Bank down, const uint16_t* hp, int H, int I, const uint32_t* perm, c
         }
 }
 
+} // namespace
+
+#include "prefill_wide.h"
+
+namespace {
+
 // out[t] = sum over j = 0..k-1 of the pair rows whose slot id is valid, in j order.
 // V = 4: 16 bytes per thread (H % 4 == 0, out 16-byte aligned), the loads of up to
 // 8 pair rows issued before their sums; the same additions in the same order as V = 1.
@@ -509,10 +521,29 @@ bool fmt_ok(int dtype, int kdim) {
            (dtype == NAIWA_Q8_0 && kdim % KBlock<NAIWA_Q8_0>::kVals == 0);
 }
 
+struct Gemms { // one call's two grouped products
+    Bank gate, up, down;
+    const uint16_t* xp;
+    uint16_t* hp;
+    float* ypair;
+    const uint32_t* perm;
+    const float* w;
+    int H, I, k, act, xcd;
+    Tiles tl;
+};
+
 template <int DG, int DD>
-void launch_gateup(dim3 g, hipStream_t st, Bank bg, Bank bu, const uint16_t* xp, int H, int I, int k,
-                   const uint32_t* perm, Tiles tl, int act, uint16_t* hp, int xcd) {
-    gateup_kernel<DG, DD><<<g, kGemm, 0, st>>>(bg, bu, xp, H, I, k, perm, tl, act, hp, xcd);
+void launch_gemms(bool wide, unsigned tiles, hipStream_t st, const Gemms& g) {
+    const unsigned b1 = g.I / kTNG * tiles, b2 = g.H / kTND * tiles;
+    if (wide) {
+        wide_gateup_kernel<DG, DD><<<b1, kWide, 0, st>>>(g.gate, g.up, g.xp, g.H, g.I, g.k, g.perm, g.tl, g.act, g.hp,
+                                                         g.xcd);
+        wide_down_kernel<DD><<<b2, kWide, 0, st>>>(g.down, g.hp, g.H, g.I, g.perm, g.w, g.tl, g.ypair, g.xcd);
+    } else {
+        gateup_kernel<DG, DD><<<b1, kGemm, 0, st>>>(g.gate, g.up, g.xp, g.H, g.I, g.k, g.perm, g.tl, g.act, g.hp,
+                                                    g.xcd);
+        down_kernel<DD><<<b2, kGemm, 0, st>>>(g.down, g.hp, g.H, g.I, g.perm, g.w, g.tl, g.ypair, g.xcd);
+    }
 }
 
 } // namespace
@@ -544,7 +575,20 @@ extern "C" int naiwa_moe_prefill(const naiwa_bank* gate, const naiwa_bank* up, c
 
     // scratch: perm [n] | offsets [slots + 1] | bad | tiles 3 x max + n | xp bf16 [T, H] | h bf16 [n, I] |
     //          ypair f32 [n, H]
-    const int64_t max_tiles = (n + kTM - 1) / kTM + slots;
+    // 128-pair tiles where the experts average more pairs than a 64-pair tile holds and
+    // one launch gives every CU a block; below either line the 64-pair tiles' 8-wave blocks
+    // keep more loads in flight.  Whole calls, 64- and 128-pair tiles: H 2048, I 768, 128
+    // experts, 64 / 81 / 125 / 162 pairs an expert 311 / 390 / 515 / 652 us and 266 / 308 /
+    // 438 / 557; H 2048, I 1408, 66 experts (Q8_0 down) 62 / 85 / 133 pairs 253 / 328 / 447
+    // and 275 / 300 / 348; H 4096, I 14336, 8 experts, 64 / 256 / 1024 pairs 510 / 1,137 /
+    // 3,924 and 431 / 931 / 3,061.  Few blocks: H 2048, I 1024, 16 experts, 82 pairs (128
+    // blocks) 92 and 108; H 2560, I 1792, 18 experts of Q8_0, 100 pairs (252) 163 and 168;
+    // H 1024, I 512, 8 experts, 128 pairs (32) 54 and 62.
+    const int64_t wide_tiles = std::max<int64_t>((n + kWideM - 1) / kWideM, slots);
+    const bool wide = n > (int64_t)64 * slots && wide_tiles * (I / kTNG) >= 256 &&
+                      32 * std::max(rbg, rbd) <= (int64_t)UINT32_MAX; // a strip's row offsets have 32 bits
+    const int tm = wide ? kWideM : kTM;
+    const int64_t max_tiles = (n + tm - 1) / tm + slots;
     auto a256 = [](size_t b) { return (b + 255) & ~size_t(255); };
     const size_t o_perm = 0, o_off = a256(o_perm + (size_t)n * 4), o_bad = a256(o_off + (size_t)(slots + 1) * 4);
     const size_t o_tiles = a256(o_bad + 4), o_x = a256(o_tiles + (size_t)(3 * max_tiles + 1) * 4);
@@ -569,34 +613,30 @@ extern "C" int naiwa_moe_prefill(const naiwa_bank* gate, const naiwa_bank* up, c
     const unsigned prep_blocks = (unsigned)(((int64_t)T * (H / 8) + kThreads - 1) / kThreads);
     if (gate->dtype == NAIWA_Q4_K)
         prep_tiles_kernel<NAIWA_Q4_K><<<prep_blocks + 1, kThreads, 0, st>>>((const uint16_t*)x, T, H, xp, offsets,
-                                                                            slots, tl);
+                                                                            slots, tm, tl);
     else
         prep_tiles_kernel<NAIWA_Q8_0><<<prep_blocks + 1, kThreads, 0, st>>>((const uint16_t*)x, T, H, xp, offsets,
-                                                                            slots, tl);
+                                                                            slots, tm, tl);
     const Bank bg{(const uint8_t*)gate->base, gate->slot_stride, rbg}, bu{(const uint8_t*)up->base, up->slot_stride, rbg};
     const Bank bd{(const uint8_t*)down->base, down->slot_stride, rbd};
     const unsigned tiles8 = (unsigned)((max_tiles + 7) / 8 * 8);
-    const dim3 g1((unsigned)(I / kTNG) * tiles8), g2((unsigned)(H / kTND) * tiles8);
     // XCD order when the experts average at most two tiles (few weight strips to share
     // between tiles, activation rows shared by every column block); with many tiles an
     // expert (a 4096-token Mixtral chunk: 16), the plain order keeps a column's weight
     // strip in one XCD's L2 across the tiles running at once.  DeepSeek-V2-Lite chunk:
     // FETCH -27 % (gate/up) and -26 % (down) at the same time; Mixtral 4096 tokens in
     // XCD order: 27.8K against 32.8K tok/s.
-    const int xcd = n <= (int64_t)2 * kTM * slots ? 1 : 0;
+    const int xcd = n <= (int64_t)128 * slots ? 1 : 0;
     const bool g4 = gate->dtype == NAIWA_Q4_K, d4 = down->dtype == NAIWA_Q4_K;
+    const Gemms g{bg, bu, bd, xp, hp, ypair, perm, w, H, I, k, act, xcd, tl};
     if (g4 && d4)
-        launch_gateup<NAIWA_Q4_K, NAIWA_Q4_K>(g1, st, bg, bu, xp, H, I, k, perm, tl, act, hp, xcd);
+        launch_gemms<NAIWA_Q4_K, NAIWA_Q4_K>(wide, tiles8, st, g);
     else if (g4)
-        launch_gateup<NAIWA_Q4_K, NAIWA_Q8_0>(g1, st, bg, bu, xp, H, I, k, perm, tl, act, hp, xcd);
+        launch_gemms<NAIWA_Q4_K, NAIWA_Q8_0>(wide, tiles8, st, g);
     else if (d4)
-        launch_gateup<NAIWA_Q8_0, NAIWA_Q4_K>(g1, st, bg, bu, xp, H, I, k, perm, tl, act, hp, xcd);
+        launch_gemms<NAIWA_Q8_0, NAIWA_Q4_K>(wide, tiles8, st, g);
     else
-        launch_gateup<NAIWA_Q8_0, NAIWA_Q8_0>(g1, st, bg, bu, xp, H, I, k, perm, tl, act, hp, xcd);
-    if (d4)
-        down_kernel<NAIWA_Q4_K><<<g2, kGemm, 0, st>>>(bd, hp, H, I, perm, w, tl, ypair, xcd);
-    else
-        down_kernel<NAIWA_Q8_0><<<g2, kGemm, 0, st>>>(bd, hp, H, I, perm, w, tl, ypair, xcd);
+        launch_gemms<NAIWA_Q8_0, NAIWA_Q8_0>(wide, tiles8, st, g);
     const int acc = (flags & NAIWA_PREFILL_ACCUMULATE) ? 1 : 0;
     const unsigned cs4 = (unsigned)((H / 4 + kThreads - 1) / kThreads), cs1 = (unsigned)((H + kThreads - 1) / kThreads);
     uint16_t* res = (flags & NAIWA_PREFILL_RESIDUAL) ? (uint16_t*)const_cast<void*>(x) : nullptr;
