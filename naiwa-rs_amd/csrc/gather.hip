@@ -13,92 +13,60 @@ gather_kernel(const uint32_t* ids, int n, int E, uint32_t* perm, uint32_t* offse
     naiwa_segment(sm, ids, nullptr, n, E, perm, offsets, nullptr, nullptr, nullptr, bad);
 }
 
-// The same stable counting sort with one block per expert id e: its segment
-// starts at the number of valid ids below e, and its entries keep their flat
-// order by a block-wide running count of (id == e) over chunks of 256 entries.
-// O(n) per block, all ids in parallel: for many entries and few ids (a prefill
-// chunk's routing) it replaces the one-block sort's serial chunks.
-constexpr int kExpertThreads = 256;
+// The same stable counting sort with one block per expert id e: its segment starts at
+// the number of valid ids below e, and its entries keep their flat order.  All ids in
+// parallel: for many entries and few ids (a prefill chunk's routing) it replaces the
+// one-block sort's serial chunks.  Every block reads all n ids, once: wave w keeps the
+// contiguous entries 64 R w .. 64 R (w + 1) - 1 in registers, R a lane, counts its own, and
+// after one exchange of the waves' counts places them without another barrier.  (With
+// chunks of 256 entries and two barriers each, 16K pairs of 128 experts took 37 us.)
+constexpr int kExpertThreads = 1024, kExpertWaves = kExpertThreads / 64;
 
-constexpr int kIdsPerThread = 32; // ids a thread keeps in registers (calls of up to 8192 entries)
-
-template <bool CACHED>
+template <int R>
 __global__ void __launch_bounds__(kExpertThreads)
 gather_by_id_kernel(const uint32_t* ids, int n, int E, uint32_t* perm, uint32_t* offsets, int* bad) {
-    __shared__ uint32_t wsum[kExpertThreads / 64];
-    __shared__ uint32_t wsum2[kExpertThreads / 64];
+    __shared__ uint32_t sums[3][kExpertWaves]; // of each wave: ids below e, outside [0, E), equal to e
     const int e = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    // entry tid + 256 r: its id, read once (CACHED: all of this thread's loads issued
-    // together, then kept for the second pass)
-    uint32_t cache[CACHED ? kIdsPerThread : 1];
-    if (CACHED) {
+    const int i0 = 64 * R * wave + lane;
+    uint32_t id[R];
 #pragma unroll
-        for (int r = 0; r < kIdsPerThread; ++r) {
-            const int i = tid + kExpertThreads * r;
-            cache[r] = i < n ? ids[i] : 0u;
-        }
-    }
-    // valid ids below e, and ids outside [0, E) (block 0 reports them)
-    uint32_t below = 0, outside = 0;
-    auto count = [&](uint32_t v) {
-        below += v < (uint32_t)e;
-        outside += v >= (uint32_t)E;
-    };
-    if constexpr (CACHED) {
+    for (int r = 0; r < R; ++r) id[r] = i0 + 64 * r < n ? ids[i0 + 64 * r] : 0u;
+    uint32_t below = 0, outside = 0, mine = 0;
 #pragma unroll
-        for (int r = 0; r < kIdsPerThread; ++r)
-            if (tid + kExpertThreads * r < n) count(cache[r]);
-    } else {
-        for (int i = tid; i < n; i += kExpertThreads) count(ids[i]);
-    }
-    for (int m = 32; m >= 1; m >>= 1) {
-        below += __shfl_xor(below, m, 64);
-        outside += __shfl_xor(outside, m, 64);
+    for (int r = 0; r < R; ++r) {
+        const bool in = i0 + 64 * r < n;
+        below += (uint32_t)__popcll(__ballot(in && id[r] < (uint32_t)e));
+        outside += (uint32_t)__popcll(__ballot(in && id[r] >= (uint32_t)E));
+        mine += (uint32_t)__popcll(__ballot(in && id[r] == (uint32_t)e));
     }
     if (lane == 0) {
-        wsum[wave] = below;
-        wsum2[wave] = outside;
+        sums[0][wave] = below;
+        sums[1][wave] = outside;
+        sums[2][wave] = mine;
     }
     __syncthreads();
-    uint32_t start = 0, nbad = 0;
+    uint32_t start = 0, nbad = 0, before = 0, total = 0;
 #pragma unroll
-    for (int w = 0; w < kExpertThreads / 64; ++w) {
-        start += wsum[w];
-        nbad += wsum2[w];
+    for (int w = 0; w < kExpertWaves; ++w) {
+        start += sums[0][w];
+        nbad += sums[1][w];
+        total += sums[2][w];
+        if (w < wave) before += sums[2][w];
     }
-    __syncthreads();
     const uint64_t lower = (1ull << lane) - 1ull;
-    uint32_t run = 0;
-    // entries in chunks of 256: each block-wide chunk keeps the positions stable
-    auto chunk = [&](int i, uint32_t v) {
-        const bool mine = i < n && v == (uint32_t)e;
-        const uint64_t m = __ballot(mine);
-        if (lane == 0) wsum[wave] = (uint32_t)__popcll(m);
-        __syncthreads();
-        uint32_t before = run;
+    uint32_t at = start + before;
+    if (mine) { // the wave's count: uniform
 #pragma unroll
-        for (int w = 0; w < kExpertThreads / 64; ++w) {
-            if (w < wave) before += wsum[w];
-            run += wsum[w];
-        }
-        if (mine && perm) perm[start + before + (uint32_t)__popcll(m & lower)] = (uint32_t)i;
-        __syncthreads();
-    };
-    if constexpr (CACHED) {
-#pragma unroll
-        for (int r = 0; r < kIdsPerThread; ++r) {
-            if (kExpertThreads * r >= n) break; // uniform
-            chunk(tid + kExpertThreads * r, cache[r]);
-        }
-    } else {
-        for (int c0 = 0; c0 < n; c0 += kExpertThreads) {
-            const int i = c0 + tid;
-            chunk(i, i < n ? ids[i] : 0u);
+        for (int r = 0; r < R; ++r) {
+            const bool me = i0 + 64 * r < n && id[r] == (uint32_t)e;
+            const uint64_t m = __ballot(me);
+            if (me) perm[at + (uint32_t)__popcll(m & lower)] = (uint32_t)(i0 + 64 * r);
+            at += (uint32_t)__popcll(m);
         }
     }
     if (tid == 0) {
         offsets[e] = start;
-        if (e == E - 1) offsets[E] = start + run;
+        if (e == E - 1) offsets[E] = start + total;
         if (e == 0 && bad) *bad = (int)nbad;
     }
 }
@@ -111,12 +79,12 @@ extern "C" int naiwa_moe_gather(const uint32_t* ids, int n, int E, uint32_t* per
     if (!offsets_out || (n > 0 && (!ids || !perm_out))) return NAIWA_E_INVALID;
     // one block per id while that stays cheap (every block reads all n ids), else one block
     if (n > NAIWA_SEG_THREADS && (int64_t)n * E <= (int64_t)1 << 24) {
-        if (n <= kExpertThreads * kIdsPerThread)
-            gather_by_id_kernel<true><<<E, kExpertThreads, 0, (hipStream_t)stream>>>(ids, n, E, perm_out,
-                                                                                    offsets_out, bad_out);
-        else
-            gather_by_id_kernel<false><<<E, kExpertThreads, 0, (hipStream_t)stream>>>(ids, n, E, perm_out,
-                                                                                     offsets_out, bad_out);
+        const auto kernel = n <= 4 * kExpertThreads    ? gather_by_id_kernel<4>
+                            : n <= 8 * kExpertThreads  ? gather_by_id_kernel<8>
+                            : n <= 16 * kExpertThreads ? gather_by_id_kernel<16>
+                            : n <= 32 * kExpertThreads ? gather_by_id_kernel<32>
+                                                       : gather_by_id_kernel<64>;
+        kernel<<<E, kExpertThreads, 0, (hipStream_t)stream>>>(ids, n, E, perm_out, offsets_out, bad_out);
     } else
         gather_kernel<<<1, NAIWA_SEG_THREADS, 0, (hipStream_t)stream>>>(ids, n, E, perm_out, offsets_out,
                                                                          bad_out);
