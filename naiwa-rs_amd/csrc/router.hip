@@ -18,7 +18,7 @@ namespace {
 
 constexpr int kLogitThreads = 256;
 constexpr int kLogitPer = 4;      // chunk loads a thread issues before using any
-constexpr int kLogitRows = 16;    // rows per block of the many-row kernel: 4 per wave
+constexpr int kLogitRows = 16;    // rows per block of the wave-per-row kernel: 4 per wave
 constexpr int kLogitFewRows = 32; // up to this many rows, one block per (expert, row)
 
 // logits[t, e] for many rows: expert e = blockIdx.x and rows blockIdx.y * 16 + 0..15,
@@ -66,6 +66,136 @@ router_logits_rows_kernel(const void* x, int x_bf16, const float* W, const float
         }
         acc = naiwa_wave_sum_i64(acc);
         if (lane == 0) logits[(int64_t)t * E + e] = naiwa_router_fix_to_f32(acc) + (bias ? bias[e] : 0.0f);
+    }
+}
+
+// Logits of many rows: block (experts 4 blockIdx.x + 0..3, rows 64 blockIdx.y + 0..63),
+// lane = row, so a lane owns its logits and nothing is reduced across lanes; the 8 waves
+// take the units of K (128 bytes of every row) w, w + 8, ... and their int64 sums meet in
+// LDS.  A wave copies its unit's 64 row pieces to its own LDS (coalesced, the next unit's in
+// flight meanwhile) and each lane reads its row's chunks back; a chunk's router weights
+// are the same for all lanes: scalar loads.
+//
+// VALU-bound: a chunk is 8 fma and its rounding.  rint(p 2^32) is split as
+// a 2^22 + b, a = rint(p 2^10), b = rint((p - a 2^-10) 2^32), both by adding 1.5 2^23,
+// whose float bits then count a and b: exact while |p| < 2^12 (the first product stays below
+// 2^22, the remainder and its product are exact, and a 2^22 is even, so ties go the same
+// way), and 6 operations instead of a float-to-int64 conversion's 12 or more.  A lane adds
+// up |p|; where that sum is not below 2^12 (NaN too), its chunks are summed again by
+// naiwa_router_chunk.  A wave's b sums stay in 32 bits for up to 1023 chunks.
+// A wave per row and expert (the kernel above) converts x for every expert and reduces 64-bit sums
+// over its lanes: 1,999 rows of 128 experts, H 2048, 111 us against 42-52 here.
+constexpr int kManyThreads = 512, kManyWaves = 8, kManyExperts = 4, kManyRows = 64;
+constexpr int kUnitBytes = 128, kUnitPitch = kUnitBytes + 16; // the pitch spreads the rows over the banks
+constexpr int kManyMaxChunks = 1023 * kManyWaves;
+
+template <bool BF16>
+__global__ void __launch_bounds__(kManyThreads)
+router_logits_many_kernel(const void* __restrict__ x, const float* __restrict__ W, const float* __restrict__ bias,
+                          int rows, int H, int E, float* __restrict__ logits) {
+    constexpr int kChunkBytes = NAIWA_ROUTER_CHUNK * (BF16 ? 2 : 4), kPer = kUnitBytes / kChunkBytes;
+    constexpr float kMagic = 12582912.0f; // 1.5 2^23
+    constexpr uint32_t kMagicBits = 0x4B400000u;
+    __shared__ __align__(16) uint8_t tile[kManyWaves][kManyRows * kUnitPitch];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int e0 = blockIdx.x * kManyExperts, t0 = blockIdx.y * kManyRows;
+    const int nchunks = H / NAIWA_ROUTER_CHUNK, nunits = (nchunks + kPer - 1) / kPer;
+    const int64_t row_bytes = (int64_t)nchunks * kChunkBytes;
+    // read-only for the launch and uniform over the wave: the constant address space makes
+    // them scalar loads also behind the LDS stores
+    typedef const __attribute__((address_space(4))) float cfloat;
+    int64_t we[kManyExperts];
+#pragma unroll
+    for (int j = 0; j < kManyExperts; ++j) we[j] = (int64_t)min(e0 + j, E - 1) * H;
+    // piece i of a lane: row 8 i + lane / 8, its 16 bytes lane % 8 of the unit
+    const uint8_t* src = (const uint8_t*)x + 16 * (lane & 7);
+    uint8_t* mine = tile[wave];
+    uint4 pre[8];
+    auto fetch = [&](int u) {
+        const int64_t at = (int64_t)u * kUnitBytes;
+        const bool in = at + 16 * (lane & 7) < row_bytes; // the last unit may be a part
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int t = min(t0 + 8 * i + (lane >> 3), rows - 1);
+            pre[i] = in ? *reinterpret_cast<const uint4*>(src + t * row_bytes + at) : uint4{0, 0, 0, 0};
+        }
+    };
+    uint32_t sa[kManyExperts] = {}, sb[kManyExperts] = {};
+    float mag[kManyExperts] = {};
+    int count = 0;
+    if (wave < nunits) fetch(wave);
+    for (int u = wave; u < nunits; u += kManyWaves) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            *reinterpret_cast<uint4*>(mine + (8 * i + (lane >> 3)) * kUnitPitch + 16 * (lane & 7)) = pre[i];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        if (u + kManyWaves < nunits) fetch(u + kManyWaves);
+        const int nc = min(kPer, nchunks - u * kPer);
+        count += nc;
+        // a chunk's loads go out before the chunk ahead of it is computed
+        float w[kManyExperts][8], xv[8];
+        auto load = [&](int c) {
+            naiwa_load_x8(mine + lane * kUnitPitch + c * kChunkBytes, BF16, 0, xv);
+#pragma unroll
+            for (int j = 0; j < kManyExperts; ++j) {
+                const cfloat* src = (const cfloat*)(W + we[j] + (u * kPer + c) * NAIWA_ROUTER_CHUNK);
+#pragma unroll
+                for (int q = 0; q < 8; ++q) w[j][q] = src[q];
+            }
+        };
+        load(0);
+        for (int c = 0; c < nc; ++c) {
+            float wc[kManyExperts][8], xc[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                xc[q] = xv[q];
+#pragma unroll
+                for (int j = 0; j < kManyExperts; ++j) wc[j][q] = w[j][q];
+            }
+            load(min(c + 1, nc - 1));
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < kManyExperts; ++j) {
+                float p = 0.0f;
+#pragma unroll
+                for (int q = 0; q < 8; ++q) p = __builtin_fmaf(wc[j][q], xc[q], p);
+                const float ta = __builtin_fmaf(p, 1024.0f, kMagic);
+                const float rest = __builtin_fmaf(ta - kMagic, -0x1p-10f, p);
+                sa[j] += __float_as_uint(ta);
+                sb[j] += __float_as_uint(__builtin_fmaf(rest, 4294967296.0f, kMagic));
+                mag[j] += __builtin_fabsf(p);
+            }
+        }
+    }
+    long long sum[kManyExperts];
+#pragma unroll
+    for (int j = 0; j < kManyExperts; ++j) {
+        const uint32_t off = (uint32_t)count * kMagicBits;
+        sum[j] = (long long)(int32_t)(sa[j] - off) * (1ll << 22) + (int32_t)(sb[j] - off);
+        if (!(mag[j] < 4096.0f)) {
+            const int64_t row = (int64_t)min(t0 + lane, rows - 1) * H;
+            sum[j] = 0;
+            for (int u = wave; u < nunits; u += kManyWaves)
+                for (int c = u * kPer; c < min(nchunks, (u + 1) * kPer); ++c) {
+                    float xv[8];
+                    naiwa_load_x8(x, BF16, row + (int64_t)c * NAIWA_ROUTER_CHUNK, xv);
+                    sum[j] += naiwa_router_chunk(W + we[j] + c * NAIWA_ROUTER_CHUNK, xv);
+                }
+        }
+    }
+    __syncthreads(); // every wave is done with its tile
+    long long* part = reinterpret_cast<long long*>(&tile[0][0]);
+    static_assert(sizeof(tile) >= sizeof(long long) * kManyWaves * kManyExperts * 64, "sums fit");
+#pragma unroll
+    for (int j = 0; j < kManyExperts; ++j) part[(wave * kManyExperts + j) * 64 + lane] = sum[j];
+    __syncthreads();
+    // thread i: expert i % 4 of row i / 4, so that a row's logits are written together
+    const int j = threadIdx.x % kManyExperts, r = threadIdx.x / kManyExperts;
+    if (r < kManyRows && t0 + r < rows && e0 + j < E) {
+        long long acc = 0;
+#pragma unroll
+        for (int w = 0; w < kManyWaves; ++w) acc += part[(w * kManyExperts + j) * 64 + r];
+        logits[(int64_t)(t0 + r) * E + e0 + j] = naiwa_router_fix_to_f32(acc) + (bias ? bias[e0 + j] : 0.0f);
     }
 }
 
@@ -282,15 +412,28 @@ extern "C" int naiwa_router_topk_ld(const void* x, int x_dtype, const float* W, 
         logits = (float*)naiwa_scratch(NAIWA_SCRATCH_ROUTER, (size_t)rows * E * 4, &rc);
         if (!logits) return rc;
     }
-    // one block per (expert, row) for few rows, and whenever the 16-row blocks would not
-    // fill the CUs (Mixtral at 64 rows: 32 of them); the same bits either way
+    // One block per (expert, row) for few rows, and whenever the 16-row blocks would not
+    // fill the CUs (Mixtral at 64 rows: 32 of them).  64-row tiles of 4 experts where enough
+    // of them share the chip, as a wave's walk through its part of K takes 15 us or more
+    // whatever their number.  Logits and top-k, 16-row blocks and 64-row tiles: 512 / 1,024 /
+    // 1,999 / 4,096 rows of 128 experts (H 2048; 256 / 512 / 1,024 / 2,048 tiles) 29 / 61 /
+    // 111 / 219 us and 22 / 30 / 52 / 96; 4,096 rows of 8 experts (H 4096, 128 tiles) 54 and
+    // 38; fewer: 256 rows of 128 experts (128 tiles) 18.5 and 20.5, 512 rows of 64 experts
+    // (128) 16 and 19, 1,024 rows of 8 experts (H 4096, 32) 20 and 31.  The same bits every way.
+    const int xb = x_dtype == NAIWA_BF16;
     const int64_t row_blocks = (int64_t)E * ((rows + kLogitRows - 1) / kLogitRows);
+    const int64_t groups = (E + kManyExperts - 1) / kManyExperts, tiles = (rows + kManyRows - 1) / kManyRows;
     if (rows <= kLogitFewRows || row_blocks < 256) {
         router_logits_kernel<<<dim3((unsigned)E, (unsigned)std::min(rows, 65535)), kLogitThreads, 0, st>>>(
-            x, x_dtype == NAIWA_BF16, W, bias, rows, H, E, logits);
+            x, xb, W, bias, rows, H, E, logits);
+    } else if ((groups * tiles >= 256 || groups * tiles * H >= 1 << 19) && H / NAIWA_ROUTER_CHUNK <= kManyMaxChunks) {
+        const dim3 lg((unsigned)groups, (unsigned)tiles);
+        if (xb)
+            router_logits_many_kernel<true><<<lg, kManyThreads, 0, st>>>(x, W, bias, rows, H, E, logits);
+        else
+            router_logits_many_kernel<false><<<lg, kManyThreads, 0, st>>>(x, W, bias, rows, H, E, logits);
     } else {
         const dim3 lg((unsigned)E, (unsigned)((rows + kLogitRows - 1) / kLogitRows));
-        const int xb = x_dtype == NAIWA_BF16;
         if (H == 512 * 4)
             router_logits_rows_kernel<4><<<lg, kLogitThreads, 0, st>>>(x, xb, W, bias, rows, H, E, logits);
         else if (H == 512 * 8)
