@@ -620,12 +620,13 @@ extern "C" int naiwa_moe_prefill(const naiwa_bank* gate, const naiwa_bank* up, c
     const Bank bg{(const uint8_t*)gate->base, gate->slot_stride, rbg}, bu{(const uint8_t*)up->base, up->slot_stride, rbg};
     const Bank bd{(const uint8_t*)down->base, down->slot_stride, rbd};
     const unsigned tiles8 = (unsigned)((max_tiles + 7) / 8 * 8);
-    // XCD order when the experts average at most two tiles (few weight strips to share
-    // between tiles, activation rows shared by every column block); with many tiles an
-    // expert (a 4096-token Mixtral chunk: 16), the plain order keeps a column's weight
-    // strip in one XCD's L2 across the tiles running at once.  DeepSeek-V2-Lite chunk:
-    // FETCH -27 % (gate/up) and -26 % (down) at the same time; Mixtral 4096 tokens in
-    // XCD order: 27.8K against 32.8K tok/s.
+    // XCD order while the experts average at most 128 pairs, one or two tiles (few weight
+    // strips to share between tiles, activation rows shared by every column block); with
+    // many tiles an expert (a 4096-token Mixtral chunk: 8 of 128 pairs), the plain order
+    // keeps a column's weight strip in one XCD's L2 across the tiles running at once.
+    // XCD and plain order: DeepSeek-V2-Lite chunk 260 and 267 us (FETCH -27 % for gate/up,
+    // -26 % for down), 1,999 tokens of 128 experts 442 and 463; Mixtral 4096 tokens 3,345
+    // and 3,039.
     const int xcd = n <= (int64_t)128 * slots ? 1 : 0;
     const bool g4 = gate->dtype == NAIWA_Q4_K, d4 = down->dtype == NAIWA_Q4_K;
     const Gemms g{bg, bu, bd, xp, hp, ypair, perm, w, H, I, k, act, xcd, tl};
