@@ -82,12 +82,13 @@ router_logits_rows_kernel(const void* x, int x_bf16, const float* W, const float
 // 2^22, the remainder and its product are exact, and a 2^22 is even, so ties go the same
 // way), and 6 operations instead of a float-to-int64 conversion's 12 or more.  A lane adds
 // up |p|; where that sum is not below 2^12 (NaN too), its chunks are summed again by
-// naiwa_router_chunk.  A wave's b sums stay in 32 bits for up to 1023 chunks.
+// naiwa_router_chunk.  |b| is at most 2^21, so a wave's b sums stay in 32 bits for up to 1023
+// chunks; waves take whole units (8 bf16 or 4 f32 chunks), so 1016 chunks are the limit.
 // A wave per row and expert (the kernel above) converts x for every expert and reduces 64-bit sums
 // over its lanes: 1,999 rows of 128 experts, H 2048, 111 us against 42-52 here.
 constexpr int kManyThreads = 512, kManyWaves = 8, kManyExperts = 4, kManyRows = 64;
 constexpr int kUnitBytes = 128, kUnitPitch = kUnitBytes + 16; // the pitch spreads the rows over the banks
-constexpr int kManyMaxChunks = 1023 * kManyWaves;
+constexpr int kManyMaxChunks = 1016 * kManyWaves; // 127 bf16 or 254 f32 units a wave
 
 template <bool BF16>
 __global__ void __launch_bounds__(kManyThreads)

@@ -41,3 +41,15 @@ def test_many_row_logits_of_large_chunks(gpu):
     want = O.router_logits(O.from_bf16(x), W)
     assert np.abs(want[::3]).max() > 2.0 ** 12
     assert np.array_equal(logits.view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("H", [65024, 65088, 65472])   # the largest in 64-row tiles, and past it
+@pytest.mark.parametrize("x_f32", [False, True])
+def test_many_row_logits_of_half_way_chunks(gpu, H, x_f32):
+    """Every chunk is 2^-11, where the low part of the split rounding is largest: the low sums of
+    a wave's chunks still fit 32 bits at the longest rows the tiles take."""
+    rows, E = 512, 128
+    x = np.full((rows, H), 0x3F80, np.uint16)                       # 1.0
+    W = np.full((E, H), np.float32(2.0 ** -14), np.float32)
+    _, _, logits = gpu_router(gpu, x, W, 4, O.ROUTE_TOPK_SOFTMAX, x_f32=x_f32)
+    assert np.all(logits == np.float32(H * 2.0 ** -14))
