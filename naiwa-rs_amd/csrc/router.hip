@@ -395,6 +395,19 @@ int naiwa_route_one_publish(const void* x, int x_dtype, int H, const float* W1, 
     return naiwa_hip_rc(hipGetLastError());
 }
 
+// Whether a call's logits go to 64-row tiles.  A wave's walk through its part of K takes
+// 13 us or more whatever the number of tiles, so tiles pay from a number of logits on, and
+// as both kernels' times grow with H, that number hardly depends on it.  Logits and top-k,
+// wave-per-row blocks and 64-row tiles: 512 rows of 64 experts (32,768 logits) 17.2 and
+// 19.5 us at H 2048, 56 and 60 at H 8192; 640 rows (40,960) 19.6 and 19.6, 83 and 60; 705
+// rows 21.3 and 19.6 at H 2048; 65 rows of 128 experts at H 8192 26 and 56; 1,999 rows of
+// 128 experts at H 2048 111 and 52.  With few experts the line lies lower: 2,048 / 3,072 /
+// 4,096 rows of 8 experts 16.1 / 25.6 / 27.8 and 19.8 / 20.9 / 22.9 at H 2048, 36 / 43 / 53
+// and 42 / 44 / 45 at H 5120.
+extern "C" int naiwa_router_row_tiles(int rows, int H, int E) {
+    return (int64_t)rows * E >= (E < 12 ? 30000 : 44000) && H / NAIWA_ROUTER_CHUNK <= kManyMaxChunks;
+}
+
 extern "C" int naiwa_router_topk_ld(const void* x, int x_dtype, const float* W, const float* bias, int rows, int H,
                                     int E, int k, int mode, uint32_t* ids_out, float* w_out, int ld,
                                     float* logits_out, int64_t stream) {
@@ -414,20 +427,14 @@ extern "C" int naiwa_router_topk_ld(const void* x, int x_dtype, const float* W, 
         if (!logits) return rc;
     }
     // One block per (expert, row) for few rows, and whenever the 16-row blocks would not
-    // fill the CUs (Mixtral at 64 rows: 32 of them).  64-row tiles of 4 experts where enough
-    // of them share the chip, as a wave's walk through its part of K takes 15 us or more
-    // whatever their number.  Logits and top-k, 16-row blocks and 64-row tiles: 512 / 1,024 /
-    // 1,999 / 4,096 rows of 128 experts (H 2048; 256 / 512 / 1,024 / 2,048 tiles) 29 / 61 /
-    // 111 / 219 us and 22 / 30 / 52 / 96; 4,096 rows of 8 experts (H 4096, 128 tiles) 54 and
-    // 38; fewer: 256 rows of 128 experts (128 tiles) 18.5 and 20.5, 512 rows of 64 experts
-    // (128) 16 and 19, 1,024 rows of 8 experts (H 4096, 32) 20 and 31.  The same bits every way.
+    // fill the CUs (Mixtral at 64 rows: 32 of them).  The same bits every way.
     const int xb = x_dtype == NAIWA_BF16;
     const int64_t row_blocks = (int64_t)E * ((rows + kLogitRows - 1) / kLogitRows);
     const int64_t groups = (E + kManyExperts - 1) / kManyExperts, tiles = (rows + kManyRows - 1) / kManyRows;
     if (rows <= kLogitFewRows || row_blocks < 256) {
         router_logits_kernel<<<dim3((unsigned)E, (unsigned)std::min(rows, 65535)), kLogitThreads, 0, st>>>(
             x, xb, W, bias, rows, H, E, logits);
-    } else if ((groups * tiles >= 256 || groups * tiles * H >= 1 << 19) && H / NAIWA_ROUTER_CHUNK <= kManyMaxChunks) {
+    } else if (naiwa_router_row_tiles(rows, H, E)) {
         const dim3 lg((unsigned)groups, (unsigned)tiles);
         if (xb)
             router_logits_many_kernel<true><<<lg, kManyThreads, 0, st>>>(x, W, bias, rows, H, E, logits);

@@ -10,14 +10,13 @@ from test_gpu_routing import gpu_router
 pytestmark = pytest.mark.gpu
 
 
-# each of at least 256 tiles of 64 rows x 4 experts, or of fewer at a larger H
 @pytest.mark.parametrize("rows,H,E,x_f32", [
     (512, 2048, 128, False),   # whole tiles
     (450, 512, 129, False),    # a ragged row tile and expert group
     (1090, 520, 61, False),    # a part of a unit at the end of K
     (8200, 64, 8, False),      # one unit: seven of the eight waves have none
     (1000, 1032, 66, True),    # f32 rows, a part of a unit
-    (65, 8192, 126, False),    # 64 tiles at H 8192
+    (65, 8192, 126, False),    # few logits at a large H: not in tiles
 ])
 def test_many_row_logits_bit_exact(gpu, rows, H, E, x_f32):
     x = S.activations_bf16(4200 + rows, rows, H)
