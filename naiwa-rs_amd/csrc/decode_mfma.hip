@@ -37,15 +37,19 @@
 //
 // Rounded operands (BF).  The layers of a chain route on activations that the layers before
 // them rounded, so any change of rounding flips an expert near the cut of a top-k somewhere
-// and with it all that follows: whole steps (the layered stack, the partial cache) keep x, h
-// and the dequantised weights in bf16, and with them their results bit for bit.
+// and with it all that follows: whole steps (the layered stack, the partial cache) of at most 512
+// pairs a layer keep x, h and the dequantised weights in bf16 and the order of the sums that
+// the first matrix-core decode had, and with them its results bit for bit.  (Larger layers ran
+// on the vector path, with f32 weights, and take the exact operands now.)
 //
-// K order: group G = 4 s + g of 8 f16 is lane group g's A operand at step s.
+// K order: group G = 4 s + g of 8 values is lane group g's A operand at step s.
 //   Q4_K (256 values): lane group g takes 64-value chunk g; step s = 2 p + t its
 //        quant bytes 8 p + 0..7, low nibbles for t = 0 and high ones for t = 1:
 //        values 64 g + 32 t + 8 p + (0 2 1 3 4 6 5 7);
-//   Q8_0 (128 values): step s is block s, so that D has one scale: values
-//        32 s + 8 g + 0..7, the natural order.
+//   Q8_0 (128 values), exact: step s is block s, so that D has one scale: values
+//        32 s + 8 g + 0..7, the natural order;
+//   Q8_0, rounded: lane group g takes block g, values 32 g + 8 s + 0..7 at step s: the order
+//        is part of the bits of the sums.
 #include "decode_mfma.h"
 #include "common.h"
 #include "segments.h"
@@ -79,13 +83,13 @@ template <> struct KB<NAIWA_Q8_0> {
 };
 
 // The group that holds run r (values 8 r .. 8 r + 7) of a K-block.
-template <int DT>
+template <int DT, bool BF>
 __device__ __forceinline__ int group_of_run(int r) {
     if (DT == NAIWA_Q4_K) {
         const int g = r >> 3, t = (r >> 2) & 1, p = r & 3;
         return 4 * (2 * p + t) + g;
     }
-    return r;
+    return BF ? 4 * (r & 3) + (r >> 2) : r;
 }
 
 // The power of two that brings magnitude mx to [2^9, 2^10), as its exponent (at most
@@ -166,7 +170,7 @@ seg_prep_kernel(const uint32_t* slot_ids, const float* w, int n, int width, int 
         for (int run = tid; run < runs; run += kThreads) {
             float f[8];
             run_of(run, f);
-            *reinterpret_cast<half8v*>(xa + (size_t)t * H + run / R * KB<DT>::kVals + 8 * group_of_run<DT>(run % R)) =
+            *reinterpret_cast<half8v*>(xa + (size_t)t * H + run / R * KB<DT>::kVals + 8 * group_of_run<DT, BF>(run % R)) =
                 pack_run_bf16<DT>(f);
         }
         return;
@@ -195,7 +199,7 @@ seg_prep_kernel(const uint32_t* slot_ids, const float* w, int n, int width, int 
         if (in) run_of(run, f);
         const half8v o = pack_run<DT>(f, sc, sum);
         const int kb = run / R, r = run % R;
-        if (in) *reinterpret_cast<half8v*>(xa + (size_t)t * H + kb * KB<DT>::kVals + 8 * group_of_run<DT>(r)) = o;
+        if (in) *reinterpret_cast<half8v*>(xa + (size_t)t * H + kb * KB<DT>::kVals + 8 * group_of_run<DT, BF>(r)) = o;
         if (DT == NAIWA_Q4_K) {
             sum += __shfl_xor(sum, 1, 64);
             sum += __shfl_xor(sum, 2, 64);
@@ -262,8 +266,8 @@ __device__ __forceinline__ half2v bytes_f16(uint32_t w, uint32_t sel) {
 
 // One lane's raw weight words of a K-block (NP rows), out of LDS: the stage is free for the
 // next copies as soon as every lane holds its own.
-template <int DT, int NP> struct WRegs;
-template <int NP> struct WRegs<NAIWA_Q4_K, NP> {
+template <int DT, int NP, bool BF> struct WRegs;
+template <int NP, bool BF> struct WRegs<NAIWA_Q4_K, NP, BF> {
     u32x4 hd[NP], q0[NP], q1[NP]; // header; quant bytes 0-15 and 16-31 of 64-value chunk g
     __device__ __forceinline__ void load(const WTile<NAIWA_Q4_K, NP>& wt, int g, int m) {
 #pragma unroll
@@ -275,7 +279,7 @@ template <int NP> struct WRegs<NAIWA_Q4_K, NP> {
         }
     }
 };
-template <int NP> struct WRegs<NAIWA_Q8_0, NP> {
+template <int NP> struct WRegs<NAIWA_Q8_0, NP, false> {
     // block s: d at byte 34 s, this lane's 8 codes from 34 s + 2 + 8 g; even blocks start on
     // a word (codes in 3 words from 34 s + 8 g), odd ones 2 bytes into one (codes in 2 words)
     uint32_t ev[NP][2][3], od[NP][2][2], dw[NP][4];
@@ -302,11 +306,34 @@ template <int NP> struct WRegs<NAIWA_Q8_0, NP> {
     }
 };
 
+template <int NP> struct WRegs<NAIWA_Q8_0, NP, true> {
+    // block g, at byte 34 g: its d, and its codes from the word that holds the first (even g:
+    // from that word's third byte on, so 9 words; odd g: 8 whole words, the eighth again)
+    uint32_t w[NP][9], sh;
+    uint16_t dh[NP];
+    __device__ __forceinline__ void load(const WTile<NAIWA_Q8_0, NP>& wt, int g, int m) {
+        sh = 2u - 2u * (uint32_t)(g & 1);
+#pragma unroll
+        for (int q = 0; q < NP; ++q) {
+            const uint8_t* blk = wt.v + q * WTile<NAIWA_Q8_0, NP>::kMat + m * KB<NAIWA_Q8_0>::kBytes + g * NAIWA_Q8_0_BYTES;
+            const uint32_t* p = reinterpret_cast<const uint32_t*>(blk + 2 * (g & 1));
+            dh[q] = *reinterpret_cast<const uint16_t*>(blk);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) w[q][i] = p[i];
+            w[q][8] = p[8 - (g & 1)];
+        }
+    }
+    __device__ __forceinline__ float d(int q, int) const { return naiwa_f16_to_f32(dh[q]); }
+    __device__ __forceinline__ uint32_t code(int q, int s, int i) const {
+        return __builtin_amdgcn_alignbyte(w[q][2 * s + i + 1], w[q][2 * s + i], sh);
+    }
+};
+
 // One K-block of a wave: acc[q][mt] += rows q of the weights times the A tile's subtiles.
 // fac (h only): the row's per-chunk f16 factors from this K-block's chunk on.
 // BF: activations and dequantised weights rounded to bf16, accumulated over the K-blocks.
 template <int DT, int NP, int MT, int MR, bool HF, bool BF>
-__device__ __forceinline__ void kblock(const WRegs<DT, NP>& wr, const ATile<DT, MR, BF>& at, const uint16_t* fac,
+__device__ __forceinline__ void kblock(const WRegs<DT, NP, BF>& wr, const ATile<DT, MR, BF>& at, const uint16_t* fac,
                                        int fst, int g, int m, const NibMask& nm, floatx4 (&acc)[NP][MT]) {
     using A = ATile<DT, MR, BF>;
     auto arow = [&](int mt) { return MR < 16 ? (m & (MR - 1)) : 16 * mt + m; };
@@ -554,7 +581,7 @@ template <int DT, int NP, int MT, int MR, bool BF> struct KLoop {
             wait_copies();
             lds_barrier();
             issue_a(kb0 + jn, (j + 1) & 1);
-            WRegs<DT, NP> wr;
+            WRegs<DT, NP, BF> wr;
             wr.load(sm.w[wave], g, m);
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // held in registers: the stage is free
             issue_w(kb0 + jn);
@@ -632,7 +659,7 @@ gateup_mfma_kernel(Bank gate, Bank up, const _Float16* xa, const _Float16* xs, c
             }
             if constexpr (BF) {
                 if (mm < cnt)
-                    *reinterpret_cast<half8v*>(ha + pos * I + kb * KV + 8 * group_of_run<DD>(r)) = pack_run_bf16<DD>(f);
+                    *reinterpret_cast<half8v*>(ha + pos * I + kb * KV + 8 * group_of_run<DD, BF>(r)) = pack_run_bf16<DD>(f);
                 continue;
             }
 #pragma unroll
@@ -644,7 +671,7 @@ gateup_mfma_kernel(Bank gate, Bank up, const _Float16* xa, const _Float16* xs, c
                 sum += __shfl_xor(sum, 2, 64);
             }
             if (mm < cnt) {
-                *reinterpret_cast<half8v*>(ha + pos * I + kb * KV + 8 * group_of_run<DD>(r)) = o;
+                *reinterpret_cast<half8v*>(ha + pos * I + kb * KV + 8 * group_of_run<DD, BF>(r)) = o;
                 if (DD == NAIWA_Q4_K && (run & 3) == 0) put_sum(hs + (pos * (I / 256) + kb) * 16, r >> 2, sum);
                 if (run == 0) he[pos * (I / kChunk) + n0 / kChunk] = (int8_t)ex;
             }
