@@ -34,6 +34,8 @@
 //   x: one scale per token (prep kernel);
 //   h: one scale per (pair, 64 features), the block's own strip, stored beside it;
 //      the down kernel brings a row's strips to one scale as it reads the A operand.
+// An infinity among them cancels to NaN; where h overflowed, the combine forms the sums of
+// products instead (an infinite x gives NaN: some gate is -inf, and its activation NaN).
 //
 // Rounded operands (BF).  The layers of a chain route on activations that the layers before
 // them rounded, so any change of rounding flips an expert near the cut of a top-k somewhere
@@ -739,13 +741,52 @@ down_mfma_kernel(Bank down, const _Float16* ha, const _Float16* hs, const int8_t
     }
 }
 
+// Where h overflowed: the exponent that scale_exp gives a strip with an infinity, and no other.
+constexpr int8_t kInfExp = 136 - 255;
+struct HArg {
+    Bank down;
+    const _Float16* ha;
+    const int8_t* he; // null: h in bf16, whose sums of products keep infinities
+    int I, ks, q4;
+    const uint32_t* slot_ids;
+};
+
+// The dot of down row r of a slot with K part kp of an h that holds infinities, as sums of
+// products give it: the exact operands' split sums lose it (inf - inf in d D - dmin M and in a
+// sum's low half).  Next to infinities and NaNs the finite values do not count.
+__device__ float infinite_dot(const HArg& a, uint32_t slot, uint32_t pos, int kp, int r) {
+    const int k0 = kp * a.ks, kn = min(a.ks, a.I - k0);
+    const uint16_t* h = reinterpret_cast<const uint16_t*>(a.ha) + (size_t)pos * a.I + k0;
+    const uint8_t* row = a.down.base + (int64_t)slot * a.down.stride + (int64_t)r * a.down.row_bytes;
+    float sum = 0.0f;
+#pragma unroll 1
+    for (int k = 0; k < kn; ++k) {
+        const uint32_t bits = h[k]; // position k of the K order
+        if ((bits & 0x7c00u) != 0x7c00u) continue;
+        float w;
+        if (a.q4) {
+            const uint8_t* blk = row + (k0 + k) / 256 * NAIWA_Q4_K_BYTES;
+            const int G = k % 256 / 8, t = (G / 4) & 1, g = G & 3;
+            const uint32_t byte = blk[16 + 32 * g + 8 * (G / 8) + q4_elem(k % 8)];
+            float sc, mn;
+            q4k_scale_min(*reinterpret_cast<const u32x4*>(blk), 2 * g + t, sc, mn);
+            w = __builtin_fmaf((float)(t ? byte >> 4 : byte & 15u), sc, mn);
+        } else {
+            const uint8_t* blk = row + (k0 + k) / 32 * NAIWA_Q8_0_BYTES;
+            w = naiwa_f16_to_f32(*reinterpret_cast<const uint16_t*>(blk)) * (float)(int8_t)blk[2 + k % 32];
+        }
+        sum += w * naiwa_f16_to_f32(bits);
+    }
+    return sum;
+}
+
 // out (token, row) from the K parts' unweighted dots: the token's pairs in ascending sorted
 // position (= ascending slot), each w * (its parts in part order), from 0 or from out.  inv
 // gives a pair's position (all ones: dropped), so a token's list takes one round of loads.
 // With res (bf16 [rows, H]): x = bf16(x + y) in place.  4 rows a lane.
 __global__ void __launch_bounds__(64)
 combine_mfma_kernel(const float* dpart, int kparts, int npairs, int H, int width, const uint32_t* inv, const float* w,
-                    int accumulate, float* out, uint16_t* res) {
+                    int accumulate, float* out, uint16_t* res, HArg h) {
     const int lane = threadIdx.x, t = blockIdx.y, r = blockIdx.x * 256 + 4 * lane;
     const bool in = r < H;
     const uint32_t pos = lane < width ? inv[(size_t)t * width + lane] : 0xffffffffu;
@@ -809,6 +850,36 @@ combine_mfma_kernel(const float* dpart, int kparts, int npairs, int H, int width
             }
             add(wk, sum);
         }
+    }
+    // a NaN may be an infinity that the dots lost: the row's pairs again, those of infinite h by
+    // infinite_dot
+    const bool nan = in && h.he && (acc[0] != acc[0] || acc[1] != acc[1] || acc[2] != acc[2] || acc[3] != acc[3]);
+    if (__builtin_expect(__ballot(nan) != 0, 0)) {
+        float sum[4];
+#pragma unroll 1
+        for (int i = 0; i < 4; ++i) {
+            sum[i] = in && accumulate ? out[o + i] : 0.0f;
+#pragma unroll 1
+            for (int k = 0; k < cnt; ++k) {
+                uint32_t pk;
+                float wk, v = 0.0f;
+                pair(k, pk, wk);
+                const int src = __ffsll((long long)__ballot(valid && rank == k)) - 1;
+                const uint32_t slot = h.slot_ids[(size_t)t * width + src];
+#pragma unroll 1
+                for (int p = 0; p < kparts; ++p) {
+                    bool inf = false;
+                    for (int c = p * h.ks / kChunk; c < min((p + 1) * h.ks, h.I) / kChunk; ++c)
+                        inf |= h.he[(size_t)pk * (h.I / kChunk) + c] == kInfExp;
+                    v += !in ? 0.0f : inf ? infinite_dot(h, slot, pk, p, r + i)
+                                          : dpart[((size_t)p * npairs + pk) * H + r + i];
+                }
+                sum[i] = __builtin_fmaf(wk, v, sum[i]);
+            }
+        }
+        if (nan)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[i] = sum[i];
     }
     if (!in) return;
     if (res)
@@ -936,7 +1007,8 @@ int naiwa_decode_mfma(const naiwa_bank* gate, const naiwa_bank* up, const naiwa_
         experts_rounding<NAIWA_Q8_0, NAIWA_Q4_K>(c, bf16);
     else
         experts_rounding<NAIWA_Q8_0, NAIWA_Q8_0>(c, bf16);
+    const HArg h{c.d, c.ha, bf16 ? nullptr : c.he, I, ks, d4, slot_ids};
     combine_mfma_kernel<<<dim3((H + 255) / 256, rows), 64, 0, st>>>(c.dpart, kparts, n, H, width, inv, w, accumulate, out,
-                                                                    res);
+                                                                    res, h);
     return naiwa_hip_rc(hipGetLastError());
 }

@@ -127,3 +127,67 @@ def test_chain_rounding_at_tile_edges(gpu, dt, H, I, E, k, rows):
             print(f"  max_rel_err={err:.3e}", flush=True)
             assert err < 1e-2
     assert np.array_equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("dt,H,I,rows", [
+    ((Q4, Q4, Q4), 256, 256, 4),
+    ((Q4, Q4, Q8), 512, 384, 9),
+    ((Q8, Q8, Q4), 384, 2304, 33),     # two K parts: the overflow in the first one
+    ((Q8, Q8, Q8), 256, 256, 5),
+])
+def test_an_intermediate_value_past_f32_gives_infinities(gpu, dt, H, I, rows):
+    """One feature of h overflows: the outputs are infinite with the sign of its down weight
+    (NaN where that is zero), as a sum of products gives, and other rows are not touched."""
+    nm = gpu
+    rng = np.random.default_rng(rows)
+    f = 5
+    g, u, d = (rng.normal(0, 0.02, s).astype(np.float32) for s in ((I, H), (I, H), (H, I)))
+    g[f] *= 4096
+    u[f] *= 4096
+    q = [O.quantize(t, a) for t, a in zip(dt, (g, u, d))]
+    gw, uw, dw = (O.dequantize_f64(t, a, a0.shape[1]) for t, a, a0 in zip(dt, q, (g, u, d)))
+    banks = nm.LayerBanks(1, H, I, dt)
+    banks.load(0, *q)
+    x = rng.normal(0, 1, (rows, H)).astype(np.float32)
+    x *= np.where(x @ gw.reshape(I, H)[f].astype(np.float32) > 0, 1, -1)[:, None].astype(np.float32)  # gates of f > 0
+    x[1:] *= np.float32(1e18)                         # row 0 stays ordinary
+    xd = nm.DeviceBuffer.from_array(x)
+    ids, w = nm.DeviceBuffer.from_array(np.zeros(rows, np.uint32)), nm.DeviceBuffer.from_array(np.ones(rows, np.float32))
+    out = nm.DeviceBuffer(rows * H * 4)
+    nm.indexed_moe_fused_decode(banks, xd, nm.F32, ids, w, rows, 1, out)
+    got = out.download(np.float32).reshape(rows, H)
+    hf = (x.astype(np.float64) @ gw.reshape(I, H)[f]) * (x.astype(np.float64) @ uw.reshape(I, H)[f])
+    assert np.isfinite(got[0]).all()
+    assert (np.abs(hf[1:]) > 1e39).sum() >= rows - 3
+    for t in np.nonzero(np.abs(hf) > 1e39)[0]:
+        want = np.sign(hf[t]) * np.sign(dw.reshape(H, I)[:, f])
+        assert np.array_equal(np.isposinf(got[t]), want > 0)
+        assert np.array_equal(np.isneginf(got[t]), want < 0)
+        assert np.array_equal(np.isnan(got[t]), want == 0)
+
+
+@pytest.mark.parametrize("dt", [(Q4, Q4, Q4), (Q8, Q8, Q8)])
+@pytest.mark.parametrize("rows", [4, 12, 40])
+def test_infinite_and_nan_activations_stay_in_their_rows(gpu, dt, rows):
+    nm = gpu
+    H = I = 512
+    banks, _, keep = _layer(nm, 8600 + rows, 2, H, I, dt)
+    rng = np.random.default_rng(rows)
+    x = rng.normal(0, 1, (rows, H)).astype(np.float32)
+    ids = nm.DeviceBuffer.from_array(rng.integers(0, 2, (rows, 2)).astype(np.uint32))
+    w = nm.DeviceBuffer.from_array(np.full((rows, 2), 0.5, np.float32))
+
+    def call(x):
+        xd, out = nm.DeviceBuffer.from_array(x), nm.DeviceBuffer(rows * H * 4)
+        nm.indexed_moe_fused_decode(banks, xd, nm.F32, ids, w, rows, 2, out)
+        return out.download(np.float32).reshape(rows, H)
+
+    plain = call(x)
+    bad = x.copy()
+    bad[1, 300] = np.inf
+    bad[2, 100] = np.nan
+    bad[rows - 1, 7] = -np.inf
+    got = call(bad)
+    assert np.isnan(got[[1, 2, rows - 1]]).all()
+    others = [t for t in range(rows) if t not in (1, 2, rows - 1)]
+    assert np.array_equal(got[others], plain[others])
