@@ -400,7 +400,7 @@ __device__ __forceinline__ void kblock(const WRegs<DT, NP, BF>& wr, const ATile<
             if constexpr (HF) {
                 const uint16_t* f = fac + arow(mt) * fst;
                 fg[mt] = splat(__builtin_bit_cast(_Float16, f[g]));
-                const half2v fj = h2(*reinterpret_cast<const uint32_t*>(f + 2 * (g & 1)));
+                const half2v fj = *reinterpret_cast<const half2v*>(f + 2 * (g & 1));
                 xs[mt] *= half4v{fj[0], fj[0], fj[1], fj[1]};
             }
         }
@@ -454,7 +454,7 @@ __device__ __forceinline__ void kblock(const WRegs<DT, NP, BF>& wr, const ATile<
         half2v fc[MT];
         if constexpr (HF) {
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt) fc[mt] = h2(*reinterpret_cast<const uint32_t*>(fac + arow(mt) * fst));
+            for (int mt = 0; mt < MT; ++mt) fc[mt] = *reinterpret_cast<const half2v*>(fac + arow(mt) * fst);
         }
 #pragma unroll
         for (int s = 0; s < KB<DT>::kSteps; ++s) {
@@ -691,7 +691,7 @@ down_mfma_kernel(Bank down, const _Float16* ha, const _Float16* hs, const int8_t
     constexpr int NP = 2;    // two strips of 64 rows: H is a multiple of 128 in every served format
     constexpr int kFac = 34; // K parts of at most 2048: 32 chunks, rows an odd number of words apart
     __shared__ Smem<DD, NP, MR, BF> sm;
-    __shared__ uint16_t fac[BF ? 1 : MR][kFac];
+    __shared__ __align__(4) uint16_t fac[BF ? 1 : MR][kFac]; // read two at a time
     __shared__ float rs[BF ? 1 : MR];
     const int sg = blockIdx.z;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
