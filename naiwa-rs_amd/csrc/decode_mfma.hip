@@ -2,7 +2,7 @@
 // calls of several rows, exact in the weights.
 //
 // A block of 4 waves takes one slot segment (the sorted pairs of one slot) and a
-// strip of weight rows (64 gate and the same 64 up rows, or 128 down rows);
+// strip of weight rows (64 gate and the same 64 up rows, or 64 or 128 down rows);
 // chunks of up to MR of the segment's tokens are the A operand of
 // v_mfma_f32_16x16x32_f16.  Lane l = 16 g + m holds A[m][8 g + 0..7] (token m),
 // B[8 g + 0..7][m] (weight row m of the wave's 16) and D[4 g + i][m].
@@ -682,13 +682,12 @@ gateup_mfma_kernel(Bank gate, Bank up, const _Float16* xa, const _Float16* xs, c
     }
 }
 
-// down: block (128 rows, K part, slot segment); the unweighted partial dot of (K part,
-// sorted position, row) into dpart.
-template <int DD, int MT, int MR, bool BF>
+// down: block (NP strips of 64 rows, K part, slot segment); the unweighted partial dot of (K
+// part, sorted position, row) into dpart.
+template <int DD, int NP, int MT, int MR, bool BF>
 __global__ void __launch_bounds__(kThreads, 2)
 down_mfma_kernel(Bank down, const _Float16* ha, const _Float16* hs, const int8_t* he, int H, int I, int ks, int npairs,
                  const int* seg_count, const uint32_t* seg_key, const uint32_t* seg_begin, float* dpart) {
-    constexpr int NP = 2;    // two strips of 64 rows: H is a multiple of 128 in every served format
     constexpr int kFac = 34; // K parts of at most 2048: 32 chunks, rows an odd number of words apart
     __shared__ Smem<DD, NP, MR, BF> sm;
     __shared__ __align__(4) uint16_t fac[BF ? 1 : MR][kFac]; // read two at a time
@@ -905,8 +904,20 @@ template <int DG, int DD, int MT, int MR, bool BF>
 void experts(const Call& c) {
     gateup_mfma_kernel<DG, DD, MT, MR, BF><<<dim3(c.I / kF, c.segs), kThreads, 0, c.st>>>(
         c.g, c.u, c.xa, c.xs, c.xr, c.H, c.I, c.seg_count, c.seg_key, c.seg_begin, c.tok, c.act, c.ha, c.hs, c.he);
-    down_mfma_kernel<DD, MT, MR, BF><<<dim3(c.H / (2 * kF), c.kparts, c.segs), kThreads, 0, c.st>>>(
-        c.d, c.ha, c.hs, c.he, c.H, c.I, c.ks, c.n, c.seg_count, c.seg_key, c.seg_begin, c.dpart);
+    auto down = [&](auto* kernel, int np) {
+        kernel<<<dim3(c.H / (np * kF), c.kparts, c.segs), kThreads, 0, c.st>>>(
+            c.d, c.ha, c.hs, c.he, c.H, c.I, c.ks, c.n, c.seg_count, c.seg_key, c.seg_begin, c.dpart);
+    };
+    // One strip of 64 down rows a block where two leave few blocks a CU: a block walks its K part
+    // one K-block's latency after the other, and a second strip makes each of them longer.  Two and
+    // one strips (blocks of two): 4 experts, H 512, I 1024, Q8_0, 64 rows (16) 46.0 and 38.8 us; 8
+    // experts, H 1024, I 2048, Q8_0, 128 rows (64) 72.3 and 59.2; 32 experts, H 2560, I 1536, Q4_K,
+    // 100 rows (640) 73.2 and 70.2; 60 experts, H 3072, I 1024, Q4_K, 64 rows (1,440) 84.5 and 87.0;
+    // 8 experts, H 4096, I 14336, Q4_K, 64 rows (1,792) 231 and 243.
+    if ((int64_t)(c.H / (2 * kF)) * c.kparts * c.segs < 1024)
+        down(down_mfma_kernel<DD, 1, MT, MR, BF>, 1);
+    else
+        down(down_mfma_kernel<DD, 2, MT, MR, BF>, 2);
 }
 
 // Token rows of the A tile.  8: a segment of a call of at most 8 rows holds no more (unless

@@ -38,6 +38,9 @@ CASES = [
     ((Q8, Q8, Q8), 384, 128, 8, 4, 64),
     ((Q8, Q8, Q8), 512, 2176, 4, 2, 128),   # the last K part 128
     ((Q8, Q8, Q8), 1024, 640, 8, 8, 9),
+    ((Q4, Q4, Q4), 2048, 256, 64, 8, 8),    # two strips of down rows a block
+    ((Q4, Q4, Q8), 4096, 128, 32, 4, 11),
+    ((Q8, Q8, Q8), 2048, 128, 64, 8, 64),
 ]
 CRCS = [
     (0xD82292C2, 0x40582F51),
@@ -47,6 +50,9 @@ CRCS = [
     (0x1B1B5870, 0x5C0EC3A5),
     (0x6CF94595, 0x905DD976),
     (0x7D1449DF, 0xE654BB32),
+    (0xC0AEE869, 0xC469268E),
+    (0xA416CE1D, 0xC3613152),
+    (0x31548153, 0x41809160),
 ]
 
 
