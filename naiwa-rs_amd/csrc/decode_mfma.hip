@@ -229,7 +229,9 @@ __device__ __forceinline__ void dma4(const void* base, uint32_t off, uint32_t ld
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
                  :: "v"(off), "s"(base), "s"(lds) : "memory", "m0");
 }
-__device__ __forceinline__ void wait_copies() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+// until at most N of the wave's copies (and loads), the last ones, are in flight
+template <int N>
+__device__ __forceinline__ void wait_copies() { asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory"); }
 __device__ __forceinline__ void lds_barrier() {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
@@ -493,11 +495,19 @@ __device__ __forceinline__ void kblock(const WRegs<DT, NP, BF>& wr, const ATile<
     }
 }
 
-// LDS of one block: a weight stage per wave and two A tiles.  More weight stages cost
-// blocks: with 2 the 8- and 96-row calls at H 2048, I 768 took 63 and 131 us against 61
-// and 120, and 16 and 64 rows at H 4096, I 14336 the same 188 and 227.
-template <int DT, int NP, int MR, bool BF> struct Smem {
-    WTile<DT, NP> w[kThreads / 64];
+// LDS of one block: the weight stages of each wave and two A tiles.  More weight stages cost
+// blocks: with 2 of Q4_K the 8- and 96-row calls at H 2048, I 768 took 63 and 131 us against
+// 61 and 120, and 16 and 64 rows at H 4096, I 14336 the same 188 and 227.
+//
+// A Q8_0 K-block is half as long as a Q4_K one, and where few blocks share a CU its copies'
+// latency shows: two stages for rounded operands and for gate/up with exact ones beside the
+// smaller tiles.  One and two stages, Q8_0: a layered layer of 17 / 64 rows at H 2048, I 768, 128
+// experts 68.0 / 117.9 and 63.6 / 110.1 us; gate/up, 4 rows, 60 experts, H 3072, I 1024 43.9 and
+// 41.9, 16 rows, 128 experts, H 2048, I 768 106 and 103; where they cost a block a CU: down, 64
+// rows there 111 and 114, gate/up of 32-row tiles, 64 rows, 8 experts, H 4096, I 14336 349 and 361.
+template <int DT, int NP, int MR, bool BF, bool UP> struct Smem { // UP: of gate/up
+    static constexpr int kStages = DT == NAIWA_Q8_0 && (BF || (UP && MR < 32)) ? 2 : 1;
+    WTile<DT, NP> w[kStages][kThreads / 64];
     ATile<DT, MR, BF> a[2];
 };
 
@@ -511,27 +521,28 @@ __device__ __forceinline__ uint32_t scalar_ld(const uint32_t* p) {
 // out the first copies (weights first: they need nothing but the segment), run() goes
 // through the K-blocks with one barrier each: the wave's copies for it have landed (its own
 // vmcnt), the barrier makes every wave's part of the A tile visible and frees the other A
-// buffer, the next A copies go out, the lanes take their weight words, the next K-block's
-// copies go out into the freed stage, and the K-block is computed.
-template <int DT, int NP, int MT, int MR, bool BF> struct KLoop {
+// buffer, the next A copies go out, the lanes take their weight words, the copies of the
+// K-block kStages further on go out into the freed stage, and the K-block is computed.
+template <int DT, int NP, int MT, int MR, bool BF, bool UP> struct KLoop {
     using A = ATile<DT, MR, BF>;
     using W = WTile<DT, NP>;
     static constexpr int PB = W::k16 ? 16 : 4, kPer = KB<DT>::kBytes / PB; // pieces per row
     static constexpr int kAd = (A::kDma + 3) / 4; // A copies of a wave: instructions wave, wave + 4, ...
-    Smem<DT, NP, MR, BF>& sm;
+    Smem<DT, NP, MR, BF, UP>& sm;
     const uint8_t *abase, *sums;
     const uint8_t* wrow[NP];
     int kb0, nkb, lane, wave;
     uint32_t woff[W::kDma], aoff[kAd], soff[kAd];
 
-    __device__ __forceinline__ void issue_w(int kb) {
+    static constexpr int kStages = Smem<DT, NP, MR, BF, UP>::kStages;
+    __device__ __forceinline__ void issue_w(int kb, int stage) {
 #pragma unroll
         for (int q = 0; q < NP; ++q) {
             const uint8_t* wb = wrow[q] + (size_t)kb * KB<DT>::kBytes;
 #pragma unroll
             for (int i = 0; i < W::kDma; ++i)
                 if (64 * (i + 1) <= W::kPieces || lane < W::kPieces - 64 * i) {
-                    const uint32_t l = lds_addr(sm.w[wave].v + q * W::kMat + 64 * PB * i);
+                    const uint32_t l = lds_addr(sm.w[stage][wave].v + q * W::kMat + 64 * PB * i);
                     if (W::k16)
                         dma16(wb, woff[i], l);
                     else
@@ -558,7 +569,7 @@ template <int DT, int NP, int MT, int MR, bool BF> struct KLoop {
             const int p = min(lane + 64 * i, W::kPieces - 1);
             woff[i] = (uint32_t)((p / kPer) * row_bytes) + (uint32_t)(p % kPer) * PB;
         }
-        issue_w(kb0);
+        issue_w(kb0, 0);
 #pragma unroll
         for (int i = 0; i < kAd; ++i) {
             const int d = min(wave + 4 * i, A::kDma - 1);
@@ -573,26 +584,29 @@ template <int DT, int NP, int MT, int MR, bool BF> struct KLoop {
             soff[i] = rs * srow + 16u * (uint32_t)(lane & 1);
         }
         issue_a(kb0, 0);
+        if (kStages == 2) issue_w(kb0 + min(1, nkb - 1), 1);
     }
     template <bool HF, int NFAC>
     __device__ __forceinline__ void run(const uint16_t (*fac)[NFAC], floatx4 (&acc)[NP][MT]) {
         const int g = lane >> 4, m = lane & 15;
         const NibMask nm = nib_mask();
         for (int j = 0; j < nkb; ++j) {
-            const int jn = min(j + 1, nkb - 1);
-            wait_copies();
+            const int jn = min(j + 1, nkb - 1), stage = kStages == 2 ? j & 1 : 0;
+            // all but the next stage's weights, the last copies issued (every wave issues all kDma
+            // of each matrix)
+            wait_copies<kStages == 2 ? NP * W::kDma : 0>();
             lds_barrier();
             issue_a(kb0 + jn, (j + 1) & 1);
             WRegs<DT, NP, BF> wr;
-            wr.load(sm.w[wave], g, m);
+            wr.load(sm.w[stage][wave], g, m);
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // held in registers: the stage is free
-            issue_w(kb0 + jn);
+            issue_w(kb0 + min(j + kStages, nkb - 1), stage);
             kblock<DT, NP, MT, MR, HF, BF>(wr, sm.a[j & 1], HF ? &fac[0][j * (KB<DT>::kVals / kChunk)] : nullptr, NFAC, g, m,
                                        nm, acc);
         }
         // the last K-block's copies went out once more: they land before the LDS is used for
         // anything else
-        wait_copies();
+        wait_copies<0>();
         lds_barrier();
     }
 };
@@ -605,7 +619,7 @@ gateup_mfma_kernel(Bank gate, Bank up, const _Float16* xa, const _Float16* xs, c
                    const int* seg_count, const uint32_t* seg_key, const uint32_t* seg_begin, const uint32_t* tok,
                    int act, _Float16* ha, _Float16* hs, int8_t* he) {
     constexpr int kHt = kF + 4; // floats per row of the h exchange
-    __shared__ Smem<DG, 2, MR, BF> sm;
+    __shared__ Smem<DG, 2, MR, BF, true> sm;
     static_assert(sizeof(float) * MR * kHt <= sizeof(sm), "the h exchange reuses the tiles");
     const int sg = blockIdx.y;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -618,7 +632,7 @@ gateup_mfma_kernel(Bank gate, Bank up, const _Float16* xa, const _Float16* xs, c
     if (sg >= segs) return;
     const int n0 = blockIdx.x * kF;
     const int64_t r0 = n0 + 16 * wave;
-    KLoop<DG, 2, MT, MR, BF> kl{sm, (const uint8_t*)xa, (const uint8_t*)xs,
+    KLoop<DG, 2, MT, MR, BF, true> kl{sm, (const uint8_t*)xa, (const uint8_t*)xs,
                                  {gate.base + (int64_t)slot * gate.stride + r0 * gate.row_bytes,
                                   up.base + (int64_t)slot * up.stride + r0 * up.row_bytes},
                                  0, H / KB<DG>::kVals, lane, wave};
@@ -689,7 +703,7 @@ __global__ void __launch_bounds__(kThreads, 2)
 down_mfma_kernel(Bank down, const _Float16* ha, const _Float16* hs, const int8_t* he, int H, int I, int ks, int npairs,
                  const int* seg_count, const uint32_t* seg_key, const uint32_t* seg_begin, float* dpart) {
     constexpr int kFac = 34; // K parts of at most 2048: 32 chunks, rows an odd number of words apart
-    __shared__ Smem<DD, NP, MR, BF> sm;
+    __shared__ Smem<DD, NP, MR, BF, false> sm;
     __shared__ __align__(4) uint16_t fac[BF ? 1 : MR][kFac]; // read two at a time
     __shared__ float rs[BF ? 1 : MR];
     const int sg = blockIdx.z;
@@ -702,7 +716,7 @@ down_mfma_kernel(Bank down, const _Float16* ha, const _Float16* hs, const int8_t
     if (sg >= segs) return;
     const int kp = blockIdx.y, k0 = kp * ks, kn = min(ks, I - k0);
     const int64_t r0 = (int64_t)blockIdx.x * (NP * kF) + 16 * wave; // matrix q: rows r0 + 64 q
-    KLoop<DD, NP, MT, MR, BF> kl{sm, (const uint8_t*)ha, (const uint8_t*)hs, {}, k0 / KB<DD>::kVals,
+    KLoop<DD, NP, MT, MR, BF, false> kl{sm, (const uint8_t*)ha, (const uint8_t*)hs, {}, k0 / KB<DD>::kVals,
                                   kn / KB<DD>::kVals, lane, wave};
 #pragma unroll
     for (int q = 0; q < NP; ++q)
