@@ -611,8 +611,8 @@ template <int DT, int NP, int MT, int MR, bool BF, bool UP> struct KLoop {
     }
 };
 
-// gate/up: block (64 features, slot segment); h = act(gate) * up of the pair at its sorted
-// position, f16 in the K order of DD with a scale per (pair, 64 features).
+// gate/up: block (64 features, slot segment, chunks z, z + gridDim.z, ...); h = act(gate) * up
+// of the pair at its sorted position, f16 in the K order of DD with a scale per (pair, 64 features).
 template <int DG, int DD, int MT, int MR, bool BF>
 __global__ void __launch_bounds__(kThreads, 2)
 gateup_mfma_kernel(Bank gate, Bank up, const _Float16* xa, const _Float16* xs, const float* xr, int H, int I,
@@ -636,7 +636,7 @@ gateup_mfma_kernel(Bank gate, Bank up, const _Float16* xa, const _Float16* xs, c
                                  {gate.base + (int64_t)slot * gate.stride + r0 * gate.row_bytes,
                                   up.base + (int64_t)slot * up.stride + r0 * up.row_bytes},
                                  0, H / KB<DG>::kVals, lane, wave};
-    for (int c0 = b; c0 < e; c0 += MR) {
+    for (int c0 = b + (int)blockIdx.z * MR; c0 < e; c0 += (int)gridDim.z * MR) {
         const int cnt = min(MR, e - c0);
         // rows past the segment repeat its last token; their results are dropped
         kl.start(gate.row_bytes, (uint32_t)H * 2, (uint32_t)(H / 256) * 32,
@@ -696,12 +696,12 @@ gateup_mfma_kernel(Bank gate, Bank up, const _Float16* xa, const _Float16* xs, c
     }
 }
 
-// down: block (NP strips of 64 rows, K part, slot segment); the unweighted partial dot of (K
-// part, sorted position, row) into dpart.
+// down: block (NP strips of 64 rows, K part and chunks as gate/up's, slot segment); the
+// unweighted partial dot of (K part, sorted position, row) into dpart.
 template <int DD, int NP, int MT, int MR, bool BF>
 __global__ void __launch_bounds__(kThreads, 2)
-down_mfma_kernel(Bank down, const _Float16* ha, const _Float16* hs, const int8_t* he, int H, int I, int ks, int npairs,
-                 const int* seg_count, const uint32_t* seg_key, const uint32_t* seg_begin, float* dpart) {
+down_mfma_kernel(Bank down, const _Float16* ha, const _Float16* hs, const int8_t* he, int H, int I, int ks, int kparts,
+                 int npairs, const int* seg_count, const uint32_t* seg_key, const uint32_t* seg_begin, float* dpart) {
     constexpr int kFac = 34; // K parts of at most 2048: 32 chunks, rows an odd number of words apart
     __shared__ Smem<DD, NP, MR, BF, false> sm;
     __shared__ __align__(4) uint16_t fac[BF ? 1 : MR][kFac]; // read two at a time
@@ -714,14 +714,14 @@ down_mfma_kernel(Bank down, const _Float16* ha, const _Float16* hs, const int8_t
     const int segs = (int)scalar_ld((const uint32_t*)seg_count);
     asm volatile("" ::"s"(slot), "s"(b), "s"(e), "s"(segs)); // one round trip
     if (sg >= segs) return;
-    const int kp = blockIdx.y, k0 = kp * ks, kn = min(ks, I - k0);
+    const int kp = blockIdx.y % kparts, k0 = kp * ks, kn = min(ks, I - k0);
     const int64_t r0 = (int64_t)blockIdx.x * (NP * kF) + 16 * wave; // matrix q: rows r0 + 64 q
     KLoop<DD, NP, MT, MR, BF, false> kl{sm, (const uint8_t*)ha, (const uint8_t*)hs, {}, k0 / KB<DD>::kVals,
                                   kn / KB<DD>::kVals, lane, wave};
 #pragma unroll
     for (int q = 0; q < NP; ++q)
         kl.wrow[q] = down.base + (int64_t)slot * down.stride + (r0 + kF * q) * down.row_bytes;
-    for (int c0 = b; c0 < e; c0 += MR) {
+    for (int c0 = b + blockIdx.y / kparts * MR; c0 < e; c0 += gridDim.y / kparts * MR) {
         const int cnt = min(MR, e - c0);
         kl.start(down.row_bytes, (uint32_t)I * 2, (uint32_t)(I / 256) * 32,
                  [&](int r) { return (uint32_t)(c0 + min(r, cnt - 1)); });
@@ -916,11 +916,22 @@ struct Call {
 
 template <int DG, int DD, int MT, int MR, bool BF>
 void experts(const Call& c) {
-    gateup_mfma_kernel<DG, DD, MT, MR, BF><<<dim3(c.I / kF, c.segs), kThreads, 0, c.st>>>(
+    // Blocks along a segment: a block takes every nz-th chunk of its tokens.  One, except where
+    // the segments average so many tokens that most have several chunks and no CU has a second
+    // gate/up block to turn to; then as many as chunks (of 32 tokens in about an average and a
+    // deviation), up to 8 blocks a CU.  One and nz, whole calls: 4 experts, H 512, I 1024, 64 / 200
+    // rows (32 / 100 tokens a segment) Q8_0 38.7 / 69.7 and 26.1 / 27.4 us, Q4_K 32.6 / 57.8 and
+    // 23.0 / 25.2; 8 experts, H 4096, I 2048, 128 rows Q8_0 118 and 86.  Below: 24 tokens 66.9 and
+    // 74.0 there (one chunk each).  More blocks: 8 experts, H 4096, I 8192, Q4_K, 45 tokens 246 and 258.
+    const int gub = c.I / kF * c.segs;
+    int nz = 1;
+    if (MR == 32 && gub <= 256 && c.n >= 25 * c.segs)
+        nz = (int)std::min<int64_t>(((int64_t)c.n + 42 * c.segs - 1) / (32 * c.segs), 2048 / gub);
+    gateup_mfma_kernel<DG, DD, MT, MR, BF><<<dim3(c.I / kF, c.segs, nz), kThreads, 0, c.st>>>(
         c.g, c.u, c.xa, c.xs, c.xr, c.H, c.I, c.seg_count, c.seg_key, c.seg_begin, c.tok, c.act, c.ha, c.hs, c.he);
     auto down = [&](auto* kernel, int np) {
-        kernel<<<dim3(c.H / (np * kF), c.kparts, c.segs), kThreads, 0, c.st>>>(
-            c.d, c.ha, c.hs, c.he, c.H, c.I, c.ks, c.n, c.seg_count, c.seg_key, c.seg_begin, c.dpart);
+        kernel<<<dim3(c.H / (np * kF), c.kparts * nz, c.segs), kThreads, 0, c.st>>>(
+            c.d, c.ha, c.hs, c.he, c.H, c.I, c.ks, c.kparts, c.n, c.seg_count, c.seg_key, c.seg_begin, c.dpart);
     };
     // One strip of 64 down rows a block where two leave few blocks a CU: a block walks its K part
     // one K-block's latency after the other, and a second strip makes each of them longer.  Two and

@@ -36,6 +36,10 @@ def _layer(nm, seed, E, H, I, dt):
     ((Q4, Q4, Q8), 256, 2176, 2, 1, 65, True),      # the last K part 128; segments past 32 rows
     ((Q4, Q4, Q4), 512, 256, 16, 8, 150, False),    # 1,200 pairs
     ((Q8, Q8, Q8), 256, 256, 8, 16, 40, False),     # 640 pairs, the widest row of pairs
+    # several blocks along a segment: chunks past a block's first, blocks without one
+    ((Q4, Q4, Q4), 256, 256, 2, 1, 50, False),      # 25 tokens a segment
+    ((Q8, Q8, Q8), 256, 2304, 3, 2, 200, True),     # five blocks, two K parts
+    ((Q4, Q4, Q8), 512, 128, 1, 1, 1000, False),    # 32 chunks
     # two strips of down rows a block (1,024 blocks of them), in each tile height
     ((Q4, Q4, Q4), 2048, 256, 64, 8, 8, False),
     ((Q4, Q4, Q8), 4096, 128, 32, 3, 11, False),
