@@ -499,15 +499,9 @@ __device__ __forceinline__ void kblock(const WRegs<DT, NP, BF>& wr, const ATile<
 // blocks: with 2 of Q4_K the 8- and 96-row calls at H 2048, I 768 took 63 and 131 us against
 // 61 and 120, and 16 and 64 rows at H 4096, I 14336 the same 188 and 227.
 //
-// A Q8_0 K-block is half as long as a Q4_K one, and where few blocks share a CU its copies'
-// latency shows: two stages for rounded operands and for gate/up with exact ones beside the
-// smaller tiles.  One and two stages, Q8_0: a layered layer of 17 / 64 rows at H 2048, I 768, 128
-// experts 68.0 / 117.9 and 63.6 / 110.1 us; gate/up, 4 rows, 60 experts, H 3072, I 1024 43.9 and
-// 41.9, 16 rows, 128 experts, H 2048, I 768 106 and 103; where they cost a block a CU: down, 64
-// rows there 111 and 114, gate/up of 32-row tiles, 64 rows, 8 experts, H 4096, I 14336 349 and 361.
-template <int DT, int NP, int MR, bool BF, bool UP> struct Smem { // UP: of gate/up
-    static constexpr int kStages = DT == NAIWA_Q8_0 && (BF || (UP && MR < 32)) ? 2 : 1;
-    WTile<DT, NP> w[kStages][kThreads / 64];
+// ST weight stages of each wave.
+template <int DT, int NP, int MR, bool BF, int ST> struct Smem {
+    WTile<DT, NP> w[ST][kThreads / 64];
     ATile<DT, MR, BF> a[2];
 };
 
@@ -522,19 +516,18 @@ __device__ __forceinline__ uint32_t scalar_ld(const uint32_t* p) {
 // through the K-blocks with one barrier each: the wave's copies for it have landed (its own
 // vmcnt), the barrier makes every wave's part of the A tile visible and frees the other A
 // buffer, the next A copies go out, the lanes take their weight words, the copies of the
-// K-block kStages further on go out into the freed stage, and the K-block is computed.
-template <int DT, int NP, int MT, int MR, bool BF, bool UP> struct KLoop {
+// K-block ST further on go out into the freed stage, and the K-block is computed.
+template <int DT, int NP, int MT, int MR, bool BF, int ST> struct KLoop {
     using A = ATile<DT, MR, BF>;
     using W = WTile<DT, NP>;
     static constexpr int PB = W::k16 ? 16 : 4, kPer = KB<DT>::kBytes / PB; // pieces per row
     static constexpr int kAd = (A::kDma + 3) / 4; // A copies of a wave: instructions wave, wave + 4, ...
-    Smem<DT, NP, MR, BF, UP>& sm;
+    Smem<DT, NP, MR, BF, ST>& sm;
     const uint8_t *abase, *sums;
     const uint8_t* wrow[NP];
     int kb0, nkb, lane, wave;
     uint32_t woff[W::kDma], aoff[kAd], soff[kAd];
 
-    static constexpr int kStages = Smem<DT, NP, MR, BF, UP>::kStages;
     __device__ __forceinline__ void issue_w(int kb, int stage) {
 #pragma unroll
         for (int q = 0; q < NP; ++q) {
@@ -584,23 +577,23 @@ template <int DT, int NP, int MT, int MR, bool BF, bool UP> struct KLoop {
             soff[i] = rs * srow + 16u * (uint32_t)(lane & 1);
         }
         issue_a(kb0, 0);
-        if (kStages == 2) issue_w(kb0 + min(1, nkb - 1), 1);
+        if (ST == 2) issue_w(kb0 + min(1, nkb - 1), 1);
     }
     template <bool HF, int NFAC>
     __device__ __forceinline__ void run(const uint16_t (*fac)[NFAC], floatx4 (&acc)[NP][MT]) {
         const int g = lane >> 4, m = lane & 15;
         const NibMask nm = nib_mask();
         for (int j = 0; j < nkb; ++j) {
-            const int jn = min(j + 1, nkb - 1), stage = kStages == 2 ? j & 1 : 0;
+            const int jn = min(j + 1, nkb - 1), stage = ST == 2 ? j & 1 : 0;
             // all but the next stage's weights, the last copies issued (every wave issues all kDma
             // of each matrix)
-            wait_copies<kStages == 2 ? NP * W::kDma : 0>();
+            wait_copies<ST == 2 ? NP * W::kDma : 0>();
             lds_barrier();
             issue_a(kb0 + jn, (j + 1) & 1);
             WRegs<DT, NP, BF> wr;
             wr.load(sm.w[stage][wave], g, m);
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // held in registers: the stage is free
-            issue_w(kb0 + min(j + kStages, nkb - 1), stage);
+            issue_w(kb0 + min(j + ST, nkb - 1), stage);
             kblock<DT, NP, MT, MR, HF, BF>(wr, sm.a[j & 1], HF ? &fac[0][j * (KB<DT>::kVals / kChunk)] : nullptr, NFAC, g, m,
                                        nm, acc);
         }
@@ -613,13 +606,13 @@ template <int DT, int NP, int MT, int MR, bool BF, bool UP> struct KLoop {
 
 // gate/up: block (64 features, slot segment, chunks z, z + gridDim.z, ...); h = act(gate) * up
 // of the pair at its sorted position, f16 in the K order of DD with a scale per (pair, 64 features).
-template <int DG, int DD, int MT, int MR, bool BF>
+template <int DG, int DD, int MT, int MR, bool BF, int ST>
 __global__ void __launch_bounds__(kThreads, 2)
 gateup_mfma_kernel(Bank gate, Bank up, const _Float16* xa, const _Float16* xs, const float* xr, int H, int I,
                    const int* seg_count, const uint32_t* seg_key, const uint32_t* seg_begin, const uint32_t* tok,
                    int act, _Float16* ha, _Float16* hs, int8_t* he) {
     constexpr int kHt = kF + 4; // floats per row of the h exchange
-    __shared__ Smem<DG, 2, MR, BF, true> sm;
+    __shared__ Smem<DG, 2, MR, BF, ST> sm;
     static_assert(sizeof(float) * MR * kHt <= sizeof(sm), "the h exchange reuses the tiles");
     const int sg = blockIdx.y;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -632,7 +625,7 @@ gateup_mfma_kernel(Bank gate, Bank up, const _Float16* xa, const _Float16* xs, c
     if (sg >= segs) return;
     const int n0 = blockIdx.x * kF;
     const int64_t r0 = n0 + 16 * wave;
-    KLoop<DG, 2, MT, MR, BF, true> kl{sm, (const uint8_t*)xa, (const uint8_t*)xs,
+    KLoop<DG, 2, MT, MR, BF, ST> kl{sm, (const uint8_t*)xa, (const uint8_t*)xs,
                                  {gate.base + (int64_t)slot * gate.stride + r0 * gate.row_bytes,
                                   up.base + (int64_t)slot * up.stride + r0 * up.row_bytes},
                                  0, H / KB<DG>::kVals, lane, wave};
@@ -702,8 +695,9 @@ template <int DD, int NP, int MT, int MR, bool BF>
 __global__ void __launch_bounds__(kThreads, 2)
 down_mfma_kernel(Bank down, const _Float16* ha, const _Float16* hs, const int8_t* he, int H, int I, int ks, int kparts,
                  int npairs, const int* seg_count, const uint32_t* seg_key, const uint32_t* seg_begin, float* dpart) {
+    constexpr int ST = BF && DD == NAIWA_Q8_0 ? 2 : 1; // weight stages (see Smem)
     constexpr int kFac = 34; // K parts of at most 2048: 32 chunks, rows an odd number of words apart
-    __shared__ Smem<DD, NP, MR, BF, false> sm;
+    __shared__ Smem<DD, NP, MR, BF, ST> sm;
     __shared__ __align__(4) uint16_t fac[BF ? 1 : MR][kFac]; // read two at a time
     __shared__ float rs[BF ? 1 : MR];
     const int sg = blockIdx.z;
@@ -716,7 +710,7 @@ down_mfma_kernel(Bank down, const _Float16* ha, const _Float16* hs, const int8_t
     if (sg >= segs) return;
     const int kp = blockIdx.y % kparts, k0 = kp * ks, kn = min(ks, I - k0);
     const int64_t r0 = (int64_t)blockIdx.x * (NP * kF) + 16 * wave; // matrix q: rows r0 + 64 q
-    KLoop<DD, NP, MT, MR, BF, false> kl{sm, (const uint8_t*)ha, (const uint8_t*)hs, {}, k0 / KB<DD>::kVals,
+    KLoop<DD, NP, MT, MR, BF, ST> kl{sm, (const uint8_t*)ha, (const uint8_t*)hs, {}, k0 / KB<DD>::kVals,
                                   kn / KB<DD>::kVals, lane, wave};
 #pragma unroll
     for (int q = 0; q < NP; ++q)
@@ -927,19 +921,39 @@ void experts(const Call& c) {
     int nz = 1;
     if (MR == 32 && gub <= 256 && c.n >= 25 * c.segs)
         nz = (int)std::min<int64_t>(((int64_t)c.n + 42 * c.segs - 1) / (32 * c.segs), 2048 / gub);
-    gateup_mfma_kernel<DG, DD, MT, MR, BF><<<dim3(c.I / kF, c.segs, nz), kThreads, 0, c.st>>>(
-        c.g, c.u, c.xa, c.xs, c.xr, c.H, c.I, c.seg_count, c.seg_key, c.seg_begin, c.tok, c.act, c.ha, c.hs, c.he);
+    auto gateup = [&](auto* kernel) {
+        kernel<<<dim3(c.I / kF, c.segs, nz), kThreads, 0, c.st>>>(
+            c.g, c.u, c.xa, c.xs, c.xr, c.H, c.I, c.seg_count, c.seg_key, c.seg_begin, c.tok, c.act, c.ha, c.hs, c.he);
+    };
+    // A Q8_0 K-block is half as long as a Q4_K one, so its copies' latency shows twice as often:
+    // two weight stages where the LDS for them costs no block a CU: rounded operands, and gate/up
+    // of the smaller tiles while a CU has one block at most.  One and two stages, Q8_0: a layered
+    // layer of 17 / 64 rows at H 2048, I 768, 128 experts 68.0 / 117.9 and 63.6 / 110.1 us; exact,
+    // 4 rows, 60 experts, H 3072, I 1024 43.9 and 41.9; 16 rows, 256 experts, H 1024, I 512 (1,024
+    // gate/up blocks) 53.9 and 57.1, and down at 64 rows, 128 experts, H 2048, I 768 111 and 114.
+    constexpr bool q8 = DG == NAIWA_Q8_0;
+    if constexpr (q8 && !BF && MR < 32) {
+        if (gub <= 256)
+            gateup(gateup_mfma_kernel<DG, DD, MT, MR, BF, 2>);
+        else
+            gateup(gateup_mfma_kernel<DG, DD, MT, MR, BF, 1>);
+    } else {
+        gateup(gateup_mfma_kernel<DG, DD, MT, MR, BF, q8 && BF ? 2 : 1>);
+    }
     auto down = [&](auto* kernel, int np) {
         kernel<<<dim3(c.H / (np * kF), c.kparts * nz, c.segs), kThreads, 0, c.st>>>(
             c.d, c.ha, c.hs, c.he, c.H, c.I, c.ks, c.kparts, c.n, c.seg_count, c.seg_key, c.seg_begin, c.dpart);
     };
     // One strip of 64 down rows a block where two leave few blocks a CU: a block walks its K part
-    // one K-block's latency after the other, and a second strip makes each of them longer.  Two and
-    // one strips (blocks of two): 4 experts, H 512, I 1024, Q8_0, 64 rows (16) 46.0 and 38.8 us; 8
-    // experts, H 1024, I 2048, Q8_0, 128 rows (64) 72.3 and 59.2; 32 experts, H 2560, I 1536, Q4_K,
-    // 100 rows (640) 73.2 and 70.2; 60 experts, H 3072, I 1024, Q4_K, 64 rows (1,440) 84.5 and 87.0;
-    // 8 experts, H 4096, I 14336, Q4_K, 64 rows (1,792) 231 and 243.
-    if ((int64_t)(c.H / (2 * kF)) * c.kparts * c.segs < 1024)
+    // one K-block's latency after the other, and a second strip makes each of them longer (with
+    // exact Q4_K operands least, which unpack the least and share each A operand between strips).
+    // Two and one strips (blocks of two): Q8_0, 4 experts, H 512, I 1024, 64 rows (16) 46.0 and 38.8
+    // us; 8 experts, H 1024, I 2048, 128 rows (64) 72.3 and 59.2; 60 experts, H 2048, I 1024, 32
+    // rows (960) 65.9 and 62.1.  Q4_K, 8 experts, H 4096, I 2048, 16 rows (256) 39.4 and 37.7; 60
+    // experts, H 1024, I 512, 128 rows (480) 33.4 and 36.7; H 3072, I 1024, 64 rows (1,440) 84.5 and
+    // 87.0; 8 experts, H 4096, I 14336, 64 rows (1,792) 231 and 243.
+    const int64_t blocks2 = (int64_t)(c.H / (2 * kF)) * c.kparts * c.segs;
+    if (blocks2 <= (DD == NAIWA_Q4_K && !BF ? 256 : 1023))
         down(down_mfma_kernel<DD, 1, MT, MR, BF>, 1);
     else
         down(down_mfma_kernel<DD, 2, MT, MR, BF>, 2);

@@ -36,6 +36,9 @@ def _layer(nm, seed, E, H, I, dt):
     ((Q4, Q4, Q8), 256, 2176, 2, 1, 65, True),      # the last K part 128; segments past 32 rows
     ((Q4, Q4, Q4), 512, 256, 16, 8, 150, False),    # 1,200 pairs
     ((Q8, Q8, Q8), 256, 256, 8, 16, 40, False),     # 640 pairs, the widest row of pairs
+    # one weight stage (more than a gate/up block a CU) in the 8- and 16-row tiles
+    ((Q8, Q8, Q8), 256, 1152, 16, 2, 8, False),
+    ((Q8, Q8, Q8), 384, 1152, 16, 2, 16, True),
     # several blocks along a segment: chunks past a block's first, blocks without one
     ((Q4, Q4, Q4), 256, 256, 2, 1, 50, False),      # 25 tokens a segment
     ((Q8, Q8, Q8), 256, 2304, 3, 2, 200, True),     # five blocks, two K parts
