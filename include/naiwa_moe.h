@@ -202,12 +202,12 @@ int naiwa_moe_decode_ex(const naiwa_bank* gate, const naiwa_bank* up, const naiw
 /* No counterpart in the reference.  naiwa_moe_decode_ex for callers that cannot
  * allocate (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc): the same kernels and the same results bit for bit, with
- * the scratch (segments, permutation, h) in a fixed device array of
- * NAIWA_DECODE_NOALLOC_SCRATCH_BYTES per GPU, held until the process ends,
- * instead of the library's grow-only buffer.  No hipMalloc, hipFree or
- * allocating routine is called; nothing is cleared with a memset.  A call of
- * n = rows * width pairs (H the hidden size, I the intermediate size, a(v) = v
- * rounded up to a multiple of 256) needs
+ * the scratch (segments, permutation, x and h in 16 bits, dots) in a fixed
+ * device array of NAIWA_DECODE_NOALLOC_SCRATCH_BYTES per GPU, held until the
+ * process ends, instead of the library's grow-only buffer.  No hipMalloc,
+ * hipFree or allocating routine is called; nothing is cleared with a memset.
+ * A call of n = rows * width pairs (H the hidden size, I the intermediate size,
+ * a(v) = v rounded up to a multiple of 256) is accepted when
  *   S = 256 + 2 a(4 n) + a(4 (n + 1)) + T  bytes, where
  *   T = a(max(n D, a(2 rows H) + 2 n I)) + ceil(I / 2048) 4 n H
  *       when n <= 512 and width <= 16 (h staged once in the down format, D =
@@ -215,12 +215,17 @@ int naiwa_moe_decode_ex(const naiwa_bank* gate, const naiwa_bank* up, const naiw
  *       rounded up to a multiple of 16; plus the f32 dots of each 2048-wide
  *       K part of down),
  *   T = 4 n I otherwise (h as f32),
- * which naiwa_moe_decode_scratch_bytes returns; the entry point returns
- * NAIWA_E_TOO_LARGE, before any device call, when S exceeds the array.  The
- * 8 MiB array holds 56 pairs (rows <= 28 at top-2) at H 4096, I 14336, Q4_K;
- * 2712 pairs (rows <= 339 at top-8) at H 2048, I 768.  S is not monotone in n:
- * the staged path's K-part dots cost more per pair than f32 h, so at H 5120,
- * I 1536, top-6, rows 1-55 and 86-227 fit and rows 56-85 do not.
+ * is at most the array's size; naiwa_moe_decode_scratch_bytes returns S, and
+ * the entry point returns NAIWA_E_TOO_LARGE, before any device call, for a
+ * larger one.  The 8 MiB array admits 56 pairs (rows <= 28 at top-2) at H 4096,
+ * I 14336, Q4_K; 2712 pairs (rows <= 339 at top-8) at H 2048, I 768.  S is not
+ * monotone in n: the staged path's K-part dots cost more per pair than f32 h, so
+ * at H 5120, I 1536, top-6, rows 1-55 and 86-227 fit and rows 56-85 do not.
+ * Calls of 4 rows or more on the matrix cores keep dots for every pair: of those
+ * accepted, calls of n <= 512 run in one pass, larger ones in the fewest passes
+ * over groups of rows whose scratch fits, each pass reading the experts' weights
+ * again (the 2712 pairs above take 4, in 2.5 times the time of the allocating
+ * entry point).
  * Every call on one GPU uses that GPU's one array: calls that overlap
  * on the device (other streams, other host threads) race and must be ordered
  * by the caller. */
@@ -228,10 +233,11 @@ int naiwa_moe_decode_ex(const naiwa_bank* gate, const naiwa_bank* up, const naiw
 int naiwa_moe_decode_noalloc(const naiwa_bank* gate, const naiwa_bank* up, const naiwa_bank* down,
                              const void* x, int x_dtype, const uint32_t* slot_ids, const float* w,
                              int rows, int width, int act, float* out, int flags, int64_t stream);
-/* No counterpart in the reference.  The scratch bytes S (above) that a decode
- * call of rows x width pairs needs at hidden size H, intermediate size I and
- * down format down_dtype; the no-alloc entry point accepts the call when S <=
- * NAIWA_DECODE_NOALLOC_SCRATCH_BYTES.  0 for an empty call, -1 for invalid
+/* No counterpart in the reference.  S (above) of a call of rows x width pairs at
+ * hidden size H, intermediate size I and down format down_dtype: the no-alloc
+ * entry point accepts the call when S <= NAIWA_DECODE_NOALLOC_SCRATCH_BYTES.
+ * (The other entry points take what they need from the library's buffer, at
+ * most 256 MiB on the matrix cores.)  0 for an empty call, -1 for invalid
  * sizes.  No device call. */
 int64_t naiwa_moe_decode_scratch_bytes(int rows, int width, int H, int I, int down_dtype);
 

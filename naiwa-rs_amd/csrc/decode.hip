@@ -723,12 +723,14 @@ int tok_cap(int dtype, int k) {
     return cap < 1 ? 0 : (cap > kTokMax ? kTokMax : cap);
 }
 
-// Scratch of one decode call (n = rows * width pairs), and the size the no-alloc entry
-// point's capacity is stated in:
+// Scratch of one decode call on the vector path (n = rows * width pairs), and the size that
+// the no-alloc entry point admits calls by, on the matrix cores too:
 //   seg_count, bad | seg_key[n] | seg_begin[n+1] | perm[n] | h | dpart.
-// Staged-h path: h = n vectors in the down format's dot layout, dpart = K parts x n x H
-// f32.  Otherwise h = n x I f32 and no dpart.  Calls on the matrix cores lay out their
-// own (NaiwaMfmaLayout) and take as many passes over the rows as it needs to fit.
+// Staged-h path: h = n vectors in the down format's dot layout (or the size of x and h in 16
+// bits, if larger: the admitted calls are those of an earlier layout), dpart = K parts x n x H
+// f32.  Otherwise h = n x I f32 and no dpart.  Calls on the matrix cores lay out their own
+// (NaiwaMfmaLayout): no larger than this for calls of the staged-h path; larger ones take as
+// many passes over the rows as it needs to fit.
 struct DecodeScratch {
     size_t off_key, off_begin, off_perm, off_h, off_dpart, total;
     DecodeScratch(int rows, int width, int H, int I, int down_dtype) {
@@ -738,7 +740,6 @@ struct DecodeScratch {
         off_perm = off_begin + (((size_t)(n + 1) * 4 + 255) & ~size_t(255));
         off_h = off_perm + (((size_t)n * 4 + 255) & ~size_t(255));
         if (split_path(n, width)) {
-            // h in the down format's dot layout, or x and h in 16 bits
             const size_t x16 = ((size_t)rows * H * 2 + 255) & ~size_t(255);
             const size_t hb = std::max((size_t)n * naiwa_stage_bytes(down_dtype, I), x16 + (size_t)n * I * 2);
             off_dpart = off_h + ((hb + 255) & ~size_t(255));
@@ -774,8 +775,8 @@ MfmaPlan mfma_plan(const naiwa_bank* gate, const naiwa_bank* up, const naiwa_ban
                chain && split_path(rows * width, width), 0, 0};
     if (!p.on) return p;
     const int H = gate->k, I = gate->n;
-    p.rows = naiwa_decode_mfma_rows_per_pass(rows, width, H, I, split_parts(I), cap);
-    p.bytes = NaiwaMfmaLayout(p.rows, width, H, I, split_parts(I)).total;
+    p.rows = naiwa_decode_mfma_rows_per_pass(rows, width, H, I, split_parts(I), down->dtype, cap);
+    p.bytes = NaiwaMfmaLayout(p.rows, width, H, I, split_parts(I), down->dtype).total;
     return p;
 }
 
@@ -1074,7 +1075,7 @@ extern "C" int naiwa_moe_decode_noalloc(const naiwa_bank* gate, const naiwa_bank
     if (width > 0 && DecodeScratch(rows, width, gate->k, gate->n, down->dtype).total > kNoAllocScratchBytes)
         return NAIWA_E_TOO_LARGE;
     // on the matrix cores in passes that fit: an accepted call has at least 4 rows there, so
-    // one row takes little more than a quarter of the array
+    // one row takes no more than about a quarter of the array
     const MfmaPlan mfma = mfma_plan(gate, up, down, x, rows, width, kNoAllocScratchBytes, false);
     if (mfma.on && mfma.bytes > kNoAllocScratchBytes) return NAIWA_E_TOO_LARGE;
     uint8_t* ws = nullptr;

@@ -14,14 +14,15 @@ bool naiwa_decode_mfma_ok(const naiwa_bank* gate, const naiwa_bank* up, const na
 
 // Scratch of one pass over `rows` rows.
 struct NaiwaMfmaLayout {
-    size_t off_key, off_begin, off_perm, off_inv, off_xa, off_xs, off_xr, off_ha, off_hs, off_he, off_dpart, total;
-    NaiwaMfmaLayout(int rows, int width, int H, int I, int kparts);
+    size_t off_key, off_begin, off_perm, off_inv, off_ha, off_hs, off_he, off_xa, off_xs, off_xr, off_dpart, total;
+    NaiwaMfmaLayout(int rows, int width, int H, int I, int kparts, int down_dtype);
 };
 
-// The most rows (of `rows`, halved until they fit) one pass may take with `bytes` of scratch.
-// A row's result does not depend on the rows beside it, so a call in several passes gives
-// the bits of one pass.
-int naiwa_decode_mfma_rows_per_pass(int rows, int width, int H, int I, int kparts, size_t bytes);
+// Rows per pass of a call in the fewest passes that fit `bytes` of scratch each (1 when none
+// do).  A row's result does not depend on the rows beside it, so a call in several passes
+// gives the bits of one pass.
+extern "C" int naiwa_decode_mfma_rows_per_pass(int rows, int width, int H, int I, int kparts, int down_dtype,
+                                               size_t bytes);
 
 // One pass over scratch ws (NaiwaMfmaLayout(rows, ...).total bytes): out = (accumulate ? out
 // : 0) + the weighted experts, and with res (bf16 [rows, H]) x = bf16(x + out) in place

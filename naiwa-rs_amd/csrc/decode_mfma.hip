@@ -997,30 +997,29 @@ bool naiwa_decode_mfma_ok(const naiwa_bank* gate, const naiwa_bank* up, const na
     return ((uintptr_t)x & 15) == 0; // 16-byte loads of x
 }
 
-NaiwaMfmaLayout::NaiwaMfmaLayout(int rows, int width, int H, int I, int kparts) {
+NaiwaMfmaLayout::NaiwaMfmaLayout(int rows, int width, int H, int I, int kparts, int down_dtype) {
     const size_t n = (size_t)rows * width;
     off_key = 256;
     off_begin = off_key + a256(n * 4);
     off_perm = off_begin + a256((n + 1) * 4);
     off_inv = off_perm + a256(n * 4);
-    off_xa = off_inv + a256(n * 4);
-    off_xs = off_xa + a256((size_t)rows * H * 2);
-    off_xr = off_xs + a256((size_t)rows * ((H + 255) / 256) * 32);
-    off_ha = off_xr + a256((size_t)rows * 4);
+    off_ha = off_inv + a256(n * 4);
     off_hs = off_ha + a256(n * I * 2);
-    off_he = off_hs + a256(n * ((I + 255) / 256) * 32);
-    off_dpart = off_he + a256(n * (I / kChunk));
-    total = off_dpart + (size_t)kparts * n * H * 4;
+    off_he = off_hs + (down_dtype == NAIWA_Q4_K ? a256(n * (I / 256) * 32) : 0);
+    // the laid-out x, which gate/up reads, and over it the dots that down writes after it
+    off_xa = off_dpart = off_he + a256(n * (I / kChunk));
+    off_xs = off_xa + a256((size_t)rows * H * 2);
+    off_xr = off_xs + a256((size_t)rows * (H / 256) * 32);
+    total = std::max(off_xr + a256((size_t)rows * 4), off_dpart + (size_t)kparts * n * H * 4);
 }
 
-int naiwa_decode_mfma_rows_per_pass(int rows, int width, int H, int I, int kparts, size_t bytes) {
-    // 32-bit offsets into x and h
-    int r = rows;
+int naiwa_decode_mfma_rows_per_pass(int rows, int width, int H, int I, int kparts, int down_dtype, size_t bytes) {
     auto fits = [&](int q) {
-        return NaiwaMfmaLayout(q, width, H, I, kparts).total <= bytes && (uint64_t)q * H * 2 <= UINT32_MAX &&
-               (uint64_t)q * width * I * 2 <= UINT32_MAX;
+        return NaiwaMfmaLayout(q, width, H, I, kparts, down_dtype).total <= bytes &&
+               (uint64_t)q * H * 2 <= UINT32_MAX && (uint64_t)q * width * I * 2 <= UINT32_MAX; // 32-bit offsets
     };
-    while (r > 1 && !fits(r)) r = (r + 1) / 2;
+    int passes = 1, r = rows;
+    while (r > 1 && !fits(r)) r = (rows + passes) / (passes + 1), ++passes; // rows in passes + 1 passes, rounded up
     return r;
 }
 
@@ -1028,7 +1027,7 @@ int naiwa_decode_mfma(const naiwa_bank* gate, const naiwa_bank* up, const naiwa_
                       const uint32_t* slot_ids, const float* w, int rows, int width, int act, float* out,
                       int accumulate, uint16_t* res, int ks, int kparts, bool bf16, uint8_t* ws, hipStream_t st) {
     const int H = gate->k, I = gate->n, n = rows * width;
-    const NaiwaMfmaLayout L(rows, width, H, I, kparts);
+    const NaiwaMfmaLayout L(rows, width, H, I, kparts, down->dtype);
     Call c;
     c.g = Bank{(const uint8_t*)gate->base, gate->slot_stride, naiwa_row_bytes(gate->dtype, H)};
     c.u = Bank{(const uint8_t*)up->base, up->slot_stride, naiwa_row_bytes(up->dtype, H)};

@@ -92,3 +92,27 @@ def test_noalloc_capacity_is_checked_before_any_device_call():
     assert L.naiwa_moe_decode_scratch_bytes(0, 8, 2048, 768, Q4K) == 0
     assert L.naiwa_moe_decode_scratch_bytes(1, 8, 2048, 770, Q4K) == -1
     assert L.naiwa_moe_decode_scratch_bytes(1, 8, 2048, 768, 99) == -1
+
+
+def test_noalloc_calls_of_at_most_512_pairs_run_in_one_pass():
+    """On the matrix cores the fixed array holds every admitted call of at most 512 pairs in one
+    pass over the weights; larger admitted calls take the fewest passes that fit."""
+    L = naiwa_moe.lib()
+    raw = ctypes.CDLL(_lib.LIB_PATH)
+    rows_per_pass = raw.naiwa_decode_mfma_rows_per_pass
+    rows_per_pass.argtypes = [ctypes.c_int] * 6 + [ctypes.c_size_t]
+    cap = 8 << 20
+    checked = 0
+    for dt, step in ((naiwa_moe.Q4_K, 256), (naiwa_moe.Q8_0, 128)):
+        for H in (256, 512, 1024, 2048, 2560, 4096, 5120, 7168, 14336, 20480):
+            for I in (step, 768, 1024, 1408 // step * step, 1536, 2048, 2304, 4096, 14336):
+                kparts = (I + min(I, 2048) - 1) // min(I, 2048)
+                for width in range(1, 17):
+                    for rows in range(4, 512 // width + 1):
+                        if L.naiwa_moe_decode_scratch_bytes(rows, width, H, I, dt) > cap:
+                            continue
+                        assert rows_per_pass(rows, width, H, I, kparts, dt, cap) == rows, (dt, H, I, width, rows)
+                        checked += 1
+    assert checked > 10000
+    assert rows_per_pass(339, 8, 2048, 768, 1, naiwa_moe.Q4_K, cap) == 85
+    assert rows_per_pass(10, 1, 1 << 21, 256, 1, naiwa_moe.Q4_K, cap) == 1
