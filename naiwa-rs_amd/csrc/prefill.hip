@@ -548,6 +548,20 @@ void launch_gemms(bool wide, unsigned tiles, hipStream_t st, const Gemms& g) {
 
 } // namespace
 
+// 128-pair tiles where the experts average more pairs than a 64-pair tile holds and
+// one launch gives every CU a block; below either line the 64-pair tiles' 8-wave blocks
+// keep more loads in flight.  Whole calls, 64- and 128-pair tiles: H 2048, I 768, 128
+// experts, 64 / 81 / 125 / 162 pairs an expert 311 / 390 / 515 / 652 us and 266 / 308 /
+// 438 / 557; H 2048, I 1408, 66 experts (Q8_0 down) 62 / 85 / 133 pairs 253 / 328 / 447
+// and 275 / 300 / 348; H 4096, I 14336, 8 experts, 64 / 256 / 1024 pairs 510 / 1,137 /
+// 3,924 and 431 / 931 / 3,061.  Few blocks: H 2048, I 1024, 16 experts, 82 pairs (128
+// blocks) 92 and 108; H 2560, I 1792, 18 experts of Q8_0, 100 pairs (252) 163 and 168;
+// H 1024, I 512, 8 experts, 128 pairs (32) 54 and 62.
+extern "C" int naiwa_prefill_wide_tiles(int64_t n, int slots, int I) {
+    const int64_t tiles = std::max<int64_t>((n + kWideM - 1) / kWideM, slots);
+    return n > (int64_t)64 * slots && tiles * (I / kTNG) >= 256;
+}
+
 extern "C" int naiwa_moe_prefill(const naiwa_bank* gate, const naiwa_bank* up, const naiwa_bank* down, const void* x,
                                  const uint32_t* slot_ids, const float* w, int T, int k, int act, float* out,
                                  int flags, int64_t stream) {
@@ -575,17 +589,7 @@ extern "C" int naiwa_moe_prefill(const naiwa_bank* gate, const naiwa_bank* up, c
 
     // scratch: perm [n] | offsets [slots + 1] | bad | tiles 3 x max + n | xp bf16 [T, H] | h bf16 [n, I] |
     //          ypair f32 [n, H]
-    // 128-pair tiles where the experts average more pairs than a 64-pair tile holds and
-    // one launch gives every CU a block; below either line the 64-pair tiles' 8-wave blocks
-    // keep more loads in flight.  Whole calls, 64- and 128-pair tiles: H 2048, I 768, 128
-    // experts, 64 / 81 / 125 / 162 pairs an expert 311 / 390 / 515 / 652 us and 266 / 308 /
-    // 438 / 557; H 2048, I 1408, 66 experts (Q8_0 down) 62 / 85 / 133 pairs 253 / 328 / 447
-    // and 275 / 300 / 348; H 4096, I 14336, 8 experts, 64 / 256 / 1024 pairs 510 / 1,137 /
-    // 3,924 and 431 / 931 / 3,061.  Few blocks: H 2048, I 1024, 16 experts, 82 pairs (128
-    // blocks) 92 and 108; H 2560, I 1792, 18 experts of Q8_0, 100 pairs (252) 163 and 168;
-    // H 1024, I 512, 8 experts, 128 pairs (32) 54 and 62.
-    const int64_t wide_tiles = std::max<int64_t>((n + kWideM - 1) / kWideM, slots);
-    const bool wide = n > (int64_t)64 * slots && wide_tiles * (I / kTNG) >= 256 &&
+    const bool wide = naiwa_prefill_wide_tiles(n, slots, I) &&
                       32 * std::max(rbg, rbd) <= (int64_t)UINT32_MAX; // a strip's row offsets have 32 bits
     const int tm = wide ? kWideM : kTM;
     const int64_t max_tiles = (n + tm - 1) / tm + slots;

@@ -18,6 +18,9 @@
 
 #include <type_traits>
 
+// Whether a call of n pairs over `slots` experts takes the 128-pair tiles (prefill.hip).
+extern "C" int naiwa_prefill_wide_tiles(int64_t n, int slots, int I);
+
 namespace {
 
 constexpr int kWide = 256;   // 4 waves, two 32-feature weight strips each

@@ -1,5 +1,4 @@
-"""Which router calls take 64-row tiles (no device needed): by their number of logits, where
-both kernels were measured, and not by the hidden size."""
+"""Which calls take which kernels, where a rule on their sizes decides (no device needed)."""
 import ctypes
 
 import pytest
@@ -14,5 +13,16 @@ from naiwa_moe import _lib
     (1999, 2048, 128, True), (512, 2048, 128, True), (512, 65024, 128, True), (512, 65032, 128, False),
 ])
 def test_router_tiles_by_logits(rows, H, E, tiles):
+    """64-row tiles by the number of logits, where both kernels were timed, not by the hidden size."""
     lib = ctypes.CDLL(_lib.LIB_PATH)
     assert bool(lib.naiwa_router_row_tiles(rows, H, E)) == tiles
+
+
+@pytest.mark.parametrize("n,slots,I,wide", [
+    (64 * 128, 128, 768, False), (64 * 128 + 1, 128, 768, True),   # pairs an expert
+    (1312, 16, 1024, False), (1312, 16, 2048, True),               # 128 and 256 blocks
+    (4096 * 2, 8, 14336, True), (512 * 8, 66, 1408, False),
+])
+def test_prefill_tiles_by_pairs_and_blocks(n, slots, I, wide):
+    lib = ctypes.CDLL(_lib.LIB_PATH)
+    assert bool(lib.naiwa_prefill_wide_tiles(ctypes.c_int64(n), slots, I)) == wide
