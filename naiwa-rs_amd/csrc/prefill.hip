@@ -550,13 +550,15 @@ void launch_gemms(bool wide, unsigned tiles, hipStream_t st, const Gemms& g) {
 
 // 128-pair tiles where the experts average more pairs than a 64-pair tile holds and
 // one launch gives every CU a block; below either line the 64-pair tiles' 8-wave blocks
-// keep more loads in flight.  Whole calls, 64- and 128-pair tiles: H 2048, I 768, 128
-// experts, 64 / 81 / 125 / 162 pairs an expert 311 / 390 / 515 / 652 us and 266 / 308 /
-// 438 / 557; H 2048, I 1408, 66 experts (Q8_0 down) 62 / 85 / 133 pairs 253 / 328 / 447
-// and 275 / 300 / 348; H 4096, I 14336, 8 experts, 64 / 256 / 1024 pairs 510 / 1,137 /
-// 3,924 and 431 / 931 / 3,061.  Few blocks: H 2048, I 1024, 16 experts, 82 pairs (128
-// blocks) 92 and 108; H 2560, I 1792, 18 experts of Q8_0, 100 pairs (252) 163 and 168;
-// H 1024, I 512, 8 experts, 128 pairs (32) 54 and 62.
+// keep more loads in flight.  64- and 128-pair tiles, moe_prefill alone, at 48 / 62 / 66 / 100
+// pairs an expert: H 2048, I 1408, 66 experts, Q8_0 down 212 / 218 / 253 / 307 us and 226 /
+// 238 / 246 / 277; H 2048, I 768, 128 experts, Q4_K 201 / 230 / 246 / 296 and 168 / 183 /
+// 189 / 225, Q8_0 293 / 343 / 361 / 421 and 277 / 291 / 295 / 327; H 4096, I 14336, 8 experts,
+// Q4_K 374 / 514 / 522 / 556 and 389 / 432 / 432 / 505, Q8_0 689 / 916 / 919 / 929 and 817 /
+// 846 / 847 / 894.  Above 64 pairs every such shape gains; under it some lose, by up to 19 %,
+// and others gain up to 20 %: 64 is the first line that costs none.  Few blocks: H 2048,
+// I 1024, 16 experts, Q8_0 gate, 100 pairs (128 blocks) 81 and 95, 160 pairs (160) 116 and 94;
+// H 1024, I 512, 8 experts, 300 pairs (76) 47.5 and 54.8, 500 pairs (128) 62 and 59.
 extern "C" int naiwa_prefill_wide_tiles(int64_t n, int slots, int I) {
     const int64_t tiles = std::max<int64_t>((n + kWideM - 1) / kWideM, slots);
     return n > (int64_t)64 * slots && tiles * (I / kTNG) >= 256;
