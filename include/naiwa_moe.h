@@ -186,7 +186,14 @@ int64_t naiwa_projection_bytes(int dtype, int64_t n, int64_t k);
  * x [rows, H] bf16 or f32 (x_dtype), slot_ids/w [rows, width] device arrays,
  * out [rows, H] f32.  Weight-0 entries (the reference's padding) are skipped.
  * The combine is atomics-free: per output row, slots are added in ascending
- * slot order, the same on every run. */
+ * slot order, the same on every run.
+ * Rounding.  Calls of 1-3 rows (and shapes the matrix cores do not take) round x
+ * and h to 16 bits (bf16 for Q4_K weights, f16 for Q8_0) and dequantise in f32.
+ * Calls of 4 rows or more (H, I multiples of 256 for Q4_K, 128 for Q8_0; width <= 16;
+ * x 16-byte aligned) take the weights as exact integers with f32 scales, and x
+ * and h as f16 times a power of two per row (x) or per 64 features (h): any
+ * finite magnitude, within 4e-4 of a 64-bit result.  A NaN or an infinity stays in
+ * its row; an infinite activation gives NaN there. */
 int naiwa_moe_decode(const naiwa_bank* gate, const naiwa_bank* up, const naiwa_bank* down,
                      const void* x, int x_dtype, const uint32_t* slot_ids, const float* w,
                      int rows, int width, int act, float* out, int64_t stream);
@@ -297,8 +304,17 @@ int naiwa_moe_prefill(const naiwa_bank* gate, const naiwa_bank* up, const naiwa_
 /* A decode stack: per layer, x <- bf16(x + MoE_l(x)) with the router,      */
 /* top-k, expert decode and combine all on the device.  The reference runs  */
 /* one CachedExperts::forward per MoE layer (src/moe/cached_layer.rs:524)   */
-/* after the model's router; this entry chains those calls for a whole      */
-/* decode step so no routing decision leaves the GPU.                       */
+/* after the model's router; this entry runs them all for a whole decode    */
+/* step so no routing decision leaves the GPU.                              */
+/* NAIWA_STACK_LAYERED chains naiwa_router_topk, the decode of one layer and */
+/* the residual add.  Up to 3 rows, and past 512 pairs a layer, the results  */
+/* are bit for bit those of a host that chains the public calls.  In between */
+/* (4 rows or more on the matrix cores) a step's layers -- the partial       */
+/* cache's too -- round x, h and the dequantised weights to bf16, where      */
+/* naiwa_moe_decode rounds less: the layers route on what the layers before  */
+/* them rounded, so a host that chains naiwa_moe_decode itself gets other    */
+/* bits (3e-3 of a layer's output), and from then on other experts where two */
+/* logits are that close.                                                    */
 /* ======================================================================== */
 typedef struct naiwa_layer {
     const float* router;            /* [E, H] f32                                */

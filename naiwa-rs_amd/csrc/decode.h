@@ -4,7 +4,8 @@
 #include "../../include/naiwa_moe.h"
 
 // naiwa_moe_decode_ex of bf16 x as a layer of a whole step.  The calls of this file give the
-// same bits for the same layer; past 3 rows naiwa_moe_decode rounds less (decode_mfma.hip).
+// same bits for the same layer; from 4 rows to 512 pairs naiwa_moe_decode rounds less
+// (decode_mfma.hip).
 int naiwa_moe_decode_chain(const naiwa_bank* gate, const naiwa_bank* up, const naiwa_bank* down, const void* x,
                            const uint32_t* slot_ids, const float* w, int rows, int width, int act, float* out,
                            int flags, int64_t stream);

@@ -15,11 +15,11 @@
 // to LDS by DMA with consecutive lanes on consecutive pieces of a row (5.5 TB/s
 // for the copies alone) and the lanes unpack from LDS.  Measured, router included,
 // against register loads with weights rounded to bf16 (time; bytes of weights / time):
-// 8 rows of 128 experts top-8 at H 2048, I 768, Q4_K 69.7 -> 58.3 us (2.4 TB/s; five
-// launches' starts are 20 us of it), 96 rows 1,310 (the vector path then) -> 115 us
-// (3.0 TB/s); 8 experts top-2 at H 4096, I 14336 16 rows 213 -> 187-193 us (4.1-4.2),
-// 64 rows 258 -> 227-245 us (3.2-3.5).  The distance to a 64-bit reference fell from
-// 3.3e-3 (1.7e-3 on the vector path) to 2.1e-4.
+// 8 rows of 128 experts top-8 at H 2048, I 768, Q4_K 71.2 -> 58.4-59.8 us (2.4 TB/s; the
+// GEMMs are 40 us of it at 3.3), 96 rows 1,303 (the vector path then) -> 115 us (3.0 TB/s);
+// 8 experts top-2 at H 4096, I 14336 16 rows 217 -> 189 us (4.2), 64 rows 258 -> 241 us
+// (3.3).  The distance to a 64-bit reference fell from 3.4e-3 (1.7e-3 on the vector path)
+// to 2.1e-4.
 //
 // Exact operands.  A quantised weight is an integer times a scale, so the B
 // operand is that integer in f16 and the scales are applied in f32 afterwards:

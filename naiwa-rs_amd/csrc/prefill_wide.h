@@ -11,8 +11,9 @@
 // Measured, whole calls with the router: 4,096 tokens of 8 experts top-2, H 4096, I 14336,
 // Q4_K 3,924 -> 3,061 us (0.74 -> 0.94 PFLOP/s; a library bf16 product of 8192^3 reaches
 // 1.24 on this card); 1,999 tokens of 128 experts top-8, H 2048, I 768 516 -> 438 us.  In
-// the first, with A loaded behind the weights (3,184 us), MFMA was busy 54 % and VALU 47 %
-// of the cycles; without the unpacking it took 2,558 us, without the staging of A 2,449.
+// the first, MFMA is busy 57 % and VALU 55 % of gate/up's cycles, 50 % and 44 % of down's.
+// With A loaded behind the weights it took 3,184 us; that build without the unpacking 2,558,
+// without the staging of A 2,449.
 // An interleaving of VALU and MFMA forced by sched_group_barrier was 2 % slower.
 #pragma once
 

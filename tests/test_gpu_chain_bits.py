@@ -59,3 +59,33 @@ CRCS = [
 @pytest.mark.parametrize("case,crc", list(zip(CASES, CRCS)))
 def test_chain_bits(gpu, case, crc):
     assert step_crc(gpu, *case) == crc
+
+
+@pytest.mark.parametrize("dt,E,k,rows", [
+    ((Q4, Q4, Q4), 16, 4, 3),      # the GEMV kernels
+    ((Q4, Q4, Q4), 16, 8, 65),     # 520 pairs: exact operands on both sides
+    ((Q8, Q8, Q8), 16, 8, 70),
+])
+def test_layered_step_is_the_chain_of_the_public_calls(gpu, dt, E, k, rows):
+    """Outside the rounded range a layered step gives the bits of naiwa_router_topk,
+    naiwa_moe_decode and x = bf16(x + y)."""
+    nm = gpu
+    H, I = 256, 256
+    layers = []
+    for l in range(2):
+        g, u, d, r = S.layer(9200 + l, E, H, I, dt)
+        banks, rd = nm.LayerBanks(E, H, I, dt), nm.DeviceBuffer.from_array(r)
+        for e in range(E):
+            banks.load(e, g[e], u[e], d[e])
+        layers.append((banks, rd))
+    x = S.activations_bf16(9202, rows, H)
+    xd = nm.DeviceBuffer.from_array(x)
+    nm.stack_decode([nm.layer_desc(rd, b) for b, rd in layers], xd, rows, H, E, k,
+                    mode=O.ROUTE_SOFTMAX_TOPK_RENORM, fused=False)
+    ids, w, y = nm.DeviceBuffer(rows * k * 4), nm.DeviceBuffer(rows * k * 4), nm.DeviceBuffer(rows * H * 4)
+    for banks, rd in layers:
+        hd = nm.DeviceBuffer.from_array(x)
+        nm.router_topk(hd, nm.BF16, rd, rows, H, E, k, ids, w, mode=O.ROUTE_SOFTMAX_TOPK_RENORM)
+        nm.indexed_moe_fused_decode(banks, hd, nm.BF16, ids, w, rows, k, y)
+        x = O.to_bf16(O.from_bf16(x) + y.download(np.float32).reshape(rows, H))
+    assert np.array_equal(xd.download(np.uint16).reshape(rows, H), x)

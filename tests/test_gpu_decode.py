@@ -303,9 +303,9 @@ def test_matrix_core_decode(gpu, dt, H, I, E, k, rows, x_f32, act):
 @pytest.mark.parametrize("x_f32", [False, True])
 def test_matrix_core_decode_takes_activations_of_1e5(gpu, x_f32):
     """The matrix-core decode (8 rows) with every other token's activations scaled
-    to ~1e5 (h then reaches ~1e9, far past the f16 range): bf16 operands keep the
-    exponent range, so both groups of rows land within the 1e-2 bar of the oracle,
-    each against its own scale."""
+    to ~1e5 (h then reaches ~1e9, far past the f16 range): x and h carry a power of
+    two per row and per 64 features, so both groups of rows land within the 1e-2 bar
+    of the oracle, each against its own scale."""
     nm = gpu
     dt, H, I, E, k, rows = (O.Q4_K, O.Q4_K, O.Q8_0), 512, 384, 6, 3, 8
     g, u, d, r = S.layer(2600, E, H, I, dt)
