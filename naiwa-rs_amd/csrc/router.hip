@@ -399,13 +399,13 @@ int naiwa_route_one_publish(const void* x, int x_dtype, int H, const float* W1, 
 // 13 us or more whatever the number of tiles, so tiles pay from a number of logits on, and
 // as both kernels' times grow with H, that number hardly depends on it.  Logits and top-k,
 // wave-per-row blocks and 64-row tiles: 512 rows of 64 experts (32,768 logits) 17.2 and
-// 19.5 us at H 2048, 56 and 60 at H 8192; 640 rows (40,960) 19.6 and 19.6, 83 and 60; 705
-// rows 21.3 and 19.6 at H 2048; 65 rows of 128 experts at H 8192 26 and 56; 1,999 rows of
-// 128 experts at H 2048 111 and 52.  With few experts the line lies lower: 2,048 / 3,072 /
-// 4,096 rows of 8 experts 16.1 / 25.6 / 27.8 and 19.8 / 20.9 / 22.9 at H 2048, 36 / 43 / 53
-// and 42 / 44 / 45 at H 5120.
+// 19.5 us at H 2048, 56 and 60 at H 8192; at H 2048 705 rows (45,120) 21.3 and 19.6, 688
+// (44,032) of f32 22.7 and 23.6, 782 (50,048) 25.3 and 24.0; 65 rows of 128 experts at H 8192
+// 26 and 56; 1,999 rows of 128 experts at H 2048 111 and 52.  With few experts the line lies
+// lower: 2,048 / 3,072 / 4,096 rows of 8 experts 16.1 / 25.6 / 27.8 and 19.8 / 20.9 / 22.9 at
+// H 2048, 36 / 43 / 53 and 42 / 44 / 45 at H 5120.
 extern "C" int naiwa_router_row_tiles(int rows, int H, int E) {
-    return (int64_t)rows * E >= (E < 12 ? 30000 : 44000) && H / NAIWA_ROUTER_CHUNK <= kManyMaxChunks;
+    return (int64_t)rows * E >= (E < 12 ? 30000 : 50000) && H / NAIWA_ROUTER_CHUNK <= kManyMaxChunks;
 }
 
 extern "C" int naiwa_router_topk_ld(const void* x, int x_dtype, const float* W, const float* bias, int rows, int H,
