@@ -10,7 +10,7 @@
 #define NAIWA_ROUTER_MAX_K 32
 
 // Whether naiwa_router_topk computes the logits of a call in 64-row tiles (router.hip).
-extern "C" int naiwa_router_row_tiles(int rows, int H, int E);
+extern "C" int naiwa_router_row_tiles(int rows, int H, int E, int x_bf16);
 
 // 8 activations starting at element `off` (bf16 or f32 source).
 __device__ __forceinline__ void naiwa_load_x8(const void* x, int x_bf16, int64_t off, float* xv) {

@@ -396,16 +396,27 @@ int naiwa_route_one_publish(const void* x, int x_dtype, int H, const float* W1, 
 }
 
 // Whether a call's logits go to 64-row tiles.  A wave's walk through its part of K takes
-// 13 us or more whatever the number of tiles, so tiles pay from a number of logits on, and
-// as both kernels' times grow with H, that number hardly depends on it.  Logits and top-k,
-// wave-per-row blocks and 64-row tiles: 512 rows of 64 experts (32,768 logits) 17.2 and
-// 19.5 us at H 2048, 56 and 60 at H 8192; at H 2048 705 rows (45,120) 21.3 and 19.6, 688
-// (44,032) of f32 22.7 and 23.6, 782 (50,048) 25.3 and 24.0; 65 rows of 128 experts at H 8192
-// 26 and 56; 1,999 rows of 128 experts at H 2048 111 and 52.  With few experts the line lies
-// lower: 2,048 / 3,072 / 4,096 rows of 8 experts 16.1 / 25.6 / 27.8 and 19.8 / 20.9 / 22.9 at
-// H 2048, 36 / 43 / 53 and 42 / 44 / 45 at H 5120.
-extern "C" int naiwa_router_row_tiles(int rows, int H, int E) {
-    return (int64_t)rows * E >= (E < 12 ? 30000 : 50000) && H / NAIWA_ROUTER_CHUNK <= kManyMaxChunks;
+// 13 us or more whatever the number of tiles, so tiles pay from a number of logits on.  As
+// both kernels' times grow with H that number hardly depends on it, but on three things:
+// the wave-per-row kernel holds its router row at H 2048 and 4096 only and is slower per
+// logit elsewhere; it reads a row once per expert from the caches, where the many rows of
+// few experts don't fit; and f32 rows cost tiles twice the LDS traffic.  Each line is
+// where the two kernels' times cross, over 9 hidden sizes, 20 numbers of experts and 20 of
+// logits.  Logits and top-k, wave-per-row blocks and 64-row tiles, in us, below and above it:
+//   64 experts, H 2048: 704 rows 20.8 and 19.5, 571 rows 17.6 and 19.4; f32 704 rows 22.6 and
+//   23.8, 797 rows 25.2 and 24.2.  H 4096: 438 rows 28.5 and 31.2, 516 rows 44.6 and 33.7; f32
+//   625 rows 37.6 and 38.3, 797 rows 46.2 and 38.8.  60 experts, H 3840: 517 rows 30.0 and
+//   33.2, 609 rows 45.5 and 33.5.  16 experts, H 5120: 1,938 rows 38.4 and 42.2, 2,063 rows
+//   57.2 and 42.8; H 4096: 1,500 rows 34.6 and 33.9, 1,563 rows 47.8 and 34.2.  8 experts, H
+//   8192: 2,750 rows 61.6 and 61.0, 4,125 rows 107.6 and 65.7; f32 1,750 rows 71.7 and 69.0.
+extern "C" int naiwa_router_row_tiles(int rows, int H, int E, int x_bf16) {
+    static const int lines[3][3][2] = { // [other H, 2048, 4096][E < 12, E < 32, more][f32, bf16]
+        {{16000, 23000}, {24000, 31000}, {33000, 34000}},
+        {{16000, 23000}, {34000, 28000}, {50000, 45000}},
+        {{16000, 23000}, {28000, 24000}, {45000, 31000}},
+    };
+    const int line = lines[H == 2048 ? 1 : H == 4096 ? 2 : 0][E < 12 ? 0 : E < 32 ? 1 : 2][x_bf16 != 0];
+    return (int64_t)rows * E >= line && H / NAIWA_ROUTER_CHUNK <= kManyMaxChunks;
 }
 
 extern "C" int naiwa_router_topk_ld(const void* x, int x_dtype, const float* W, const float* bias, int rows, int H,
@@ -434,7 +445,7 @@ extern "C" int naiwa_router_topk_ld(const void* x, int x_dtype, const float* W, 
     if (rows <= kLogitFewRows || row_blocks < 256) {
         router_logits_kernel<<<dim3((unsigned)E, (unsigned)std::min(rows, 65535)), kLogitThreads, 0, st>>>(
             x, xb, W, bias, rows, H, E, logits);
-    } else if (naiwa_router_row_tiles(rows, H, E)) {
+    } else if (naiwa_router_row_tiles(rows, H, E, xb)) {
         const dim3 lg((unsigned)groups, (unsigned)tiles);
         if (xb)
             router_logits_many_kernel<true><<<lg, kManyThreads, 0, st>>>(x, W, bias, rows, H, E, logits);

@@ -11,11 +11,23 @@ from naiwa_moe import _lib
     (65, 7168, 256, False), (688, 2048, 64, False), (512, 5120, 60, False), (2048, 8192, 8, False), (65, 2048, 512, False),
     (4032, 4096, 8, True), (4096, 4096, 8, True), (1024, 5120, 60, True), (2048, 4096, 32, True),
     (1999, 2048, 128, True), (512, 2048, 128, True), (512, 65024, 128, True), (512, 65032, 128, False),
+    (629, 3840, 60, True), (512, 4096, 64, True), (1024, 4096, 32, True), (2048, 4096, 16, True),   # and in wave-per-row blocks
+    (512, 2048, 64, False), (750, 2048, 64, True), (4125, 8192, 8, True), (4095, 8192, 3, False),
 ])
 def test_router_tiles_by_logits(rows, H, E, tiles):
     """64-row tiles by the number of logits, where both kernels were timed, not by the hidden size."""
     lib = ctypes.CDLL(_lib.LIB_PATH)
-    assert bool(lib.naiwa_router_row_tiles(rows, H, E)) == tiles
+    assert bool(lib.naiwa_router_row_tiles(rows, H, E, 1)) == tiles
+
+
+@pytest.mark.parametrize("rows,H,E,tiles", [
+    (512, 4096, 64, False), (2048, 4096, 16, True), (750, 2048, 64, False), (782, 2048, 64, True),
+    (629, 3840, 60, True), (65, 7168, 256, False), (2050, 8192, 8, True), (512, 65032, 128, False),
+])
+def test_router_tiles_by_logits_of_f32_rows(rows, H, E, tiles):
+    """f32 rows cost the tiles more: another line."""
+    lib = ctypes.CDLL(_lib.LIB_PATH)
+    assert bool(lib.naiwa_router_row_tiles(rows, H, E, 0)) == tiles
 
 
 @pytest.mark.parametrize("n,slots,I,wide", [
