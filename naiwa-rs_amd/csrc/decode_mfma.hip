@@ -58,6 +58,7 @@
 #include "unpack_bf16.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace {
 
@@ -689,9 +690,11 @@ gateup_mfma_kernel(Bank gate, Bank up, const _Float16* xa, const _Float16* xs, c
     }
 }
 
-// down: block (NP strips of 64 rows, K part and chunks as gate/up's, slot segment); the
-// unweighted partial dot of (K part, sorted position, row) into dpart.
-template <int DD, int NP, int MT, int MR, bool BF>
+// down: block (NP strips of 64 rows, K part and with SPLIT chunks as gate/up's, slot segment);
+// the unweighted partial dot of (K part, sorted position, row) into dpart.  Without SPLIT a block
+// takes all chunks of its segment: the split's scalars, spilled around the K loop, cost 8 experts
+// of H 4096, I 14336, Q4_K, at 64 rows 84.0 us against 82.1 where there is nothing to split.
+template <int DD, int NP, int MT, int MR, bool BF, bool SPLIT>
 __global__ void __launch_bounds__(kThreads, 2)
 down_mfma_kernel(Bank down, const _Float16* ha, const _Float16* hs, const int8_t* he, int H, int I, int ks, int kparts,
                  int npairs, const int* seg_count, const uint32_t* seg_key, const uint32_t* seg_begin, float* dpart) {
@@ -708,14 +711,14 @@ down_mfma_kernel(Bank down, const _Float16* ha, const _Float16* hs, const int8_t
     const int segs = (int)scalar_ld((const uint32_t*)seg_count);
     asm volatile("" ::"s"(slot), "s"(b), "s"(e), "s"(segs)); // one round trip
     if (sg >= segs) return;
-    const int kp = blockIdx.y % kparts, k0 = kp * ks, kn = min(ks, I - k0);
+    const int kp = SPLIT ? blockIdx.y % kparts : blockIdx.y, k0 = kp * ks, kn = min(ks, I - k0);
     const int64_t r0 = (int64_t)blockIdx.x * (NP * kF) + 16 * wave; // matrix q: rows r0 + 64 q
     KLoop<DD, NP, MT, MR, BF, ST> kl{sm, (const uint8_t*)ha, (const uint8_t*)hs, {}, k0 / KB<DD>::kVals,
                                   kn / KB<DD>::kVals, lane, wave};
 #pragma unroll
     for (int q = 0; q < NP; ++q)
         kl.wrow[q] = down.base + (int64_t)slot * down.stride + (r0 + kF * q) * down.row_bytes;
-    for (int c0 = b + blockIdx.y / kparts * MR; c0 < e; c0 += gridDim.y / kparts * MR) {
+    for (int c0 = b + (SPLIT ? blockIdx.y / kparts * MR : 0); c0 < e; c0 += SPLIT ? gridDim.y / kparts * MR : MR) {
         const int cnt = min(MR, e - c0);
         kl.start(down.row_bytes, (uint32_t)I * 2, (uint32_t)(I / 256) * 32,
                  [&](int r) { return (uint32_t)(c0 + min(r, cnt - 1)); });
@@ -953,10 +956,15 @@ void experts(const Call& c) {
     // experts, H 1024, I 512, 128 rows (480) 33.4 and 36.7; H 3072, I 1024, 64 rows (1,440) 84.5 and
     // 87.0; 8 experts, H 4096, I 14336, 64 rows (1,792) 231 and 243.
     const int64_t blocks2 = (int64_t)(c.H / (2 * kF)) * c.kparts * c.segs;
-    if (blocks2 <= (DD == NAIWA_Q4_K && !BF ? 256 : 1023))
-        down(down_mfma_kernel<DD, 1, MT, MR, BF>, 1);
-    else
-        down(down_mfma_kernel<DD, 2, MT, MR, BF>, 2);
+    auto strips = [&](auto split) {
+        if (blocks2 <= (DD == NAIWA_Q4_K && !BF ? 256 : 1023))
+            down(down_mfma_kernel<DD, 1, MT, MR, BF, split>, 1);
+        else
+            down(down_mfma_kernel<DD, 2, MT, MR, BF, split>, 2);
+    };
+    if constexpr (MR == 32)
+        if (nz > 1) return strips(std::true_type{});
+    strips(std::false_type{});
 }
 
 // Token rows of the A tile.  8: a segment of a call of at most 8 rows holds no more (unless
