@@ -24,6 +24,10 @@ struct NaiwaMfmaLayout {
 extern "C" int naiwa_decode_mfma_rows_per_pass(int rows, int width, int H, int I, int kparts, int down_dtype,
                                                size_t bytes);
 
+// Strips of 64 down rows a block of a call of `rows` rows of `width` pairs (decode_mfma.hip);
+// exact_q4: Q4_K down weights, not rounded to bf16.
+extern "C" int naiwa_decode_mfma_down_strips(int rows, int width, int slots, int H, int kparts, int exact_q4);
+
 // One pass over scratch ws (NaiwaMfmaLayout(rows, ...).total bytes): out = (accumulate ? out
 // : 0) + the weighted experts, and with res (bf16 [rows, H]) x = bf16(x + out) in place
 // (out may then be null).  K parts of ks values of I, kparts of them.

@@ -58,6 +58,7 @@
 #include "unpack_bf16.h"
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 namespace {
@@ -902,7 +903,7 @@ combine_mfma_kernel(const float* dpart, int kparts, int npairs, int H, int width
 
 struct Call {
     Bank g, u, d;
-    int H, I, rows, n, segs, ks, kparts, act;
+    int H, I, rows, n, slots, segs, ks, kparts, act;
     int* seg_count;
     uint32_t *seg_key, *seg_begin, *tok;
     _Float16 *xa, *xs, *ha, *hs;
@@ -947,17 +948,10 @@ void experts(const Call& c) {
         kernel<<<dim3(c.H / (np * kF), c.kparts * nz, c.segs), kThreads, 0, c.st>>>(
             c.d, c.ha, c.hs, c.he, c.H, c.I, c.ks, c.kparts, c.n, c.seg_count, c.seg_key, c.seg_begin, c.dpart);
     };
-    // One strip of 64 down rows a block where two leave few blocks a CU: a block walks its K part
-    // one K-block's latency after the other, and a second strip makes each of them longer (with
-    // exact Q4_K operands least, which unpack the least and share each A operand between strips).
-    // Two and one strips (blocks of two): Q8_0, 4 experts, H 512, I 1024, 64 rows (16) 46.0 and 38.8
-    // us; 8 experts, H 1024, I 2048, 128 rows (64) 72.3 and 59.2; 60 experts, H 2048, I 1024, 32
-    // rows (960) 65.9 and 62.1.  Q4_K, 8 experts, H 4096, I 2048, 16 rows (256) 39.4 and 37.7; 60
-    // experts, H 1024, I 512, 128 rows (480) 33.4 and 36.7; H 3072, I 1024, 64 rows (1,440) 84.5 and
-    // 87.0; 8 experts, H 4096, I 14336, 64 rows (1,792) 231 and 243.
-    const int64_t blocks2 = (int64_t)(c.H / (2 * kF)) * c.kparts * c.segs;
+    const bool one = naiwa_decode_mfma_down_strips(c.rows, c.n / c.rows, c.slots, c.H, c.kparts,
+                                                   DD == NAIWA_Q4_K && !BF) == 1;
     auto strips = [&](auto split) {
-        if (blocks2 <= (DD == NAIWA_Q4_K && !BF ? 256 : 1023))
+        if (one)
             down(down_mfma_kernel<DD, 1, MT, MR, BF, split>, 1);
         else
             down(down_mfma_kernel<DD, 2, MT, MR, BF, split>, 2);
@@ -1021,6 +1015,26 @@ NaiwaMfmaLayout::NaiwaMfmaLayout(int rows, int width, int H, int I, int kparts, 
     total = std::max(off_xr + a256((size_t)rows * 4), off_dpart + (size_t)kparts * n * H * 4);
 }
 
+// Strips of 64 down rows a block: one where two leave few blocks a CU.  A block walks its K part
+// one K-block's latency after the other, and a second strip makes each of them longer (with
+// exact Q4_K operands least, which unpack the least and share each A operand between strips);
+// past 1.4 blocks a CU one strip pays where the halves spread evener, so that the fullest CU has
+// fewer strips, up to 4 blocks a CU.  The blocks counted are those that have a segment when the rows' slots
+// are drawn evenly.  Two and one strips (blocks of two, as counted), weights cold: Q8_0, 8 experts, H
+// 4096, I 2048, 4 rows (175) 65.6 and 60.2 us; 60 experts, H 3072, I 1024, 4 rows (347) 51.1 and
+// 48.8; H 2048, I 1408, 8 / 32 rows (407 / 854) 72.3 and 72.7 / 131.1 and 125.7; 16 experts, H 4096, I 1024, 64 rows
+// (512) 63.3 and 64.5; 32 experts, H 2560, I 1536, 64 rows (640) 107.5 and 103.8; 8 experts, H
+// 6144, I 4096, 16 rows (760) 136.9 and 139.6; H 4096, I 14336, 64 rows (1,792) 347 and 354.  Exact
+// Q4_K, 8 experts, H 4096, I 2048, 16 rows (253) 47.3 and 45.3; 60 experts, H 3072, I 1024, 4 / 16
+// rows (347 / 963) 37.8 and 36.3 / 65.9 and 68.2; 8 experts, H 4096, I 14336, 64 rows 230 and 243.
+extern "C" int naiwa_decode_mfma_down_strips(int rows, int width, int slots, int H, int kparts, int exact_q4) {
+    const double miss = 1.0 - std::min(1.0, (double)width / slots); // a slot's chance to be in no pair of a row
+    const double fill = (double)(H / (2 * kF)) * kparts * slots * (1.0 - std::pow(miss, rows)) / 256; // blocks a CU
+    if (fill <= 1.4) return 1;
+    if (exact_q4 || fill >= 4.0) return 2;
+    return std::ceil(2.0 * fill) < 2.0 * std::ceil(fill - 0.04) ? 1 : 2;
+}
+
 int naiwa_decode_mfma_rows_per_pass(int rows, int width, int H, int I, int kparts, int down_dtype, size_t bytes) {
     auto fits = [&](int q) {
         return NaiwaMfmaLayout(q, width, H, I, kparts, down_dtype).total <= bytes &&
@@ -1040,7 +1054,8 @@ int naiwa_decode_mfma(const naiwa_bank* gate, const naiwa_bank* up, const naiwa_
     c.g = Bank{(const uint8_t*)gate->base, gate->slot_stride, naiwa_row_bytes(gate->dtype, H)};
     c.u = Bank{(const uint8_t*)up->base, up->slot_stride, naiwa_row_bytes(up->dtype, H)};
     c.d = Bank{(const uint8_t*)down->base, down->slot_stride, naiwa_row_bytes(down->dtype, I)};
-    c.H = H, c.I = I, c.rows = rows, c.n = n, c.segs = std::max(1, std::min(n, gate->slots));
+    c.H = H, c.I = I, c.rows = rows, c.n = n;
+    c.slots = gate->slots, c.segs = std::max(1, std::min(n, gate->slots));
     c.ks = ks, c.kparts = kparts, c.act = act, c.st = st;
     c.seg_count = (int*)ws;
     c.seg_key = (uint32_t*)(ws + L.off_key);

@@ -38,3 +38,15 @@ def test_router_tiles_by_logits_of_f32_rows(rows, H, E, tiles):
 def test_prefill_tiles_by_pairs_and_blocks(n, slots, I, wide):
     lib = ctypes.CDLL(_lib.LIB_PATH)
     assert bool(lib.naiwa_prefill_wide_tiles(ctypes.c_int64(n), slots, I)) == wide
+
+
+@pytest.mark.parametrize("rows,width,slots,H,kparts,exact_q4,strips", [
+    (4, 2, 8, 4096, 1, True, 1), (64, 2, 8, 4096, 1, True, 1), (4, 4, 60, 3072, 1, True, 1),      # up to 1.4 blocks a CU
+    (16, 4, 60, 3072, 1, True, 2), (64, 2, 8, 4096, 7, True, 2), (64, 2, 16, 4096, 1, True, 2),
+    (4, 4, 60, 3072, 1, False, 1), (64, 4, 32, 2560, 1, False, 1), (32, 4, 60, 2048, 1, False, 1),  # 2.5 and 3.3
+    (64, 2, 16, 4096, 1, False, 2), (64, 2, 8, 6144, 2, False, 2), (5, 8, 66, 2048, 1, False, 2),   # 2, 3 and under 2
+    (64, 2, 8, 4096, 7, False, 2), (8, 1, 1, 512, 1, False, 1), (1, 16, 4, 512, 1, False, 1),
+])
+def test_down_strips_by_blocks_a_cu(rows, width, slots, H, kparts, exact_q4, strips):
+    lib = ctypes.CDLL(_lib.LIB_PATH)
+    assert lib.naiwa_decode_mfma_down_strips(rows, width, slots, H, kparts, exact_q4) == strips

@@ -39,8 +39,9 @@ CASES = [
     ((Q8, Q8, Q8), 512, 2176, 4, 2, 128),   # the last K part 128
     ((Q8, Q8, Q8), 1024, 640, 8, 8, 9),
     ((Q4, Q4, Q4), 2048, 256, 64, 8, 8),    # two strips of down rows a block
-    ((Q4, Q4, Q8), 4096, 128, 32, 4, 11),
+    ((Q4, Q4, Q8), 4096, 128, 32, 4, 11),   # one
     ((Q8, Q8, Q8), 2048, 128, 64, 8, 64),
+    ((Q4, Q4, Q8), 4096, 128, 32, 4, 40),   # and in 16-row tiles
 ]
 CRCS = [
     (0xD82292C2, 0x40582F51),
@@ -53,6 +54,7 @@ CRCS = [
     (0xC0AEE869, 0xC469268E),
     (0xA416CE1D, 0xC3613152),
     (0x31548153, 0x41809160),
+    (0x4F544149, 0xFB8383EA),
 ]
 
 
